@@ -381,10 +381,10 @@ __global__ void __launch_bounds__(256) gen_kernel(WorldView w, const FrameConst*
     const CamView& cam = fc->cam;
     const uint32_t tiles_x = (uint32_t)(cam.W + 15) / 16u;
     const uint32_t tiles_y = (uint32_t)(cam.H + 15) / 16u;
-    const uint32_t tile = vpt::xcd_remap(blockIdx.x, tiles_x * tiles_y);
+    const vpt::TileXY tile = vpt::screen_tile(tiles_x, tiles_y);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int px = (int)(tile % tiles_x) * 16 + (wave & 1) * 8 + (lane & 7);
-    const int py = (int)(tile / tiles_x) * 16 + (wave >> 1) * 8 + (lane >> 3);
+    const int px = (int)tile.x * 16 + (wave & 1) * 8 + (lane & 7);
+    const int py = (int)tile.y * 16 + (wave >> 1) * 8 + (lane >> 3);
     bool emit_s = false, emit_g = false;
     vpt_qray rs, rg;
     if (px < cam.W && py < cam.H) {
@@ -450,10 +450,10 @@ __global__ void __launch_bounds__(256) shade_kernel(const FrameConst* __restrict
     const CamView& cam = fc->cam;
     const uint32_t tiles_x = (uint32_t)(cam.W + 15) / 16u;
     const uint32_t tiles_y = (uint32_t)(cam.H + 15) / 16u;
-    const uint32_t tile = vpt::xcd_remap(blockIdx.x, tiles_x * tiles_y);
+    const vpt::TileXY tile = vpt::screen_tile(tiles_x, tiles_y);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int px = (int)(tile % tiles_x) * 16 + (wave & 1) * 8 + (lane & 7);
-    const int py = (int)(tile / tiles_x) * 16 + (wave >> 1) * 8 + (lane >> 3);
+    const int px = (int)tile.x * 16 + (wave & 1) * 8 + (lane & 7);
+    const int py = (int)tile.y * 16 + (wave >> 1) * 8 + (lane >> 3);
     if (px >= cam.W || py >= cam.H) return;
     const uint32_t i = (uint32_t)py * (uint32_t)cam.W + (uint32_t)px;
     const float dist = gb_t[i];
@@ -527,10 +527,10 @@ __global__ void __launch_bounds__(256) frame_primary_kernel(WorldView w, const F
     const CamView& cam = fc->cam;
     const uint32_t tiles_x = (uint32_t)(cam.W + 15) / 16u;
     const uint32_t tiles_y = (uint32_t)(cam.H + 15) / 16u;
-    const uint32_t tile = vpt::xcd_remap(blockIdx.x, tiles_x * tiles_y);
+    const vpt::TileXY tile = vpt::screen_tile(tiles_x, tiles_y);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int px = (int)(tile % tiles_x) * 16 + (wave & 1) * 8 + (lane & 7);
-    const int py = (int)(tile / tiles_x) * 16 + (wave >> 1) * 8 + (lane >> 3);
+    const int px = (int)tile.x * 16 + (wave & 1) * 8 + (lane & 7);
+    const int py = (int)tile.y * 16 + (wave >> 1) * 8 + (lane >> 3);
     unsigned long long samples = 0, rays = 0;
     if (px < cam.W && py < cam.H) {
         Vec3 dir = vpt::primary_dir(cam, px, py);

@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "vpt/vpt_numerics.h"
+#include "vpt_tiles.h"
 
 namespace vpt {
 
@@ -371,12 +372,19 @@ __device__ inline uint32_t hw_f2h(float x) { return (uint32_t)__builtin_bit_cast
 
 // Blocks are dealt to the 8 XCDs round-robin by hardware; remap the block
 // index so that XCD k receives a contiguous 1/8 of the tiles, keeping
-// neighbouring tiles (which touch the same bricks) in one L2.
+// neighbouring tiles in one L2.
 __device__ inline uint32_t xcd_remap(uint32_t bid, uint32_t nblocks)
 {
     uint32_t per = nblocks / 8u;
     if (per == 0u || bid >= per * 8u) return bid;
     return (bid & 7u) * per + (bid >> 3);
+}
+
+// The tile of a block in a launch of one block per tile: XCD k takes the
+// k-th eighth of the tiles in strip order.
+__device__ inline TileXY screen_tile(uint32_t tx, uint32_t ty)
+{
+    return strip_tile(xcd_remap(blockIdx.x, tx * ty), tx, ty);
 }
 
 }  // namespace vpt

@@ -3,8 +3,9 @@
 //
 // One lane per ray.  A 256-lane workgroup covers a 16x16 pixel tile made of
 // four 8x8 wavefront squares (square footprints keep a wavefront's rays on
-// neighbouring bricks), and tiles are dealt to XCDs in contiguous screen
-// bands (xcd_remap) so each XCD's L2 holds one region of the world.
+// neighbouring bricks), and tiles are dealt to XCDs in vertical screen
+// strips (screen_tile) so each XCD's L2 holds one region of the world and
+// all of them have about the same work.
 #include <hip/hip_runtime.h>
 #include <string.h>
 
@@ -192,10 +193,10 @@ __device__ inline void tile_pixel(int W, int H, int& px, int& py)
 {
     const uint32_t tiles_x = (uint32_t)(W + 15) / 16u;
     const uint32_t tiles_y = (uint32_t)(H + 15) / 16u;
-    const uint32_t tile = vpt::xcd_remap(blockIdx.x, tiles_x * tiles_y);
+    const vpt::TileXY tile = vpt::screen_tile(tiles_x, tiles_y);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    px = (int)(tile % tiles_x) * 16 + (wave & 1) * 8 + (lane & 7);
-    py = (int)(tile / tiles_x) * 16 + (wave >> 1) * 8 + (lane >> 3);
+    px = (int)tile.x * 16 + (wave & 1) * 8 + (lane & 7);
+    py = (int)tile.y * 16 + (wave >> 1) * 8 + (lane >> 3);
 }
 
 // Adds this lane's DF samples to counter[0] and traced rays to counter[1]
@@ -415,34 +416,18 @@ __device__ inline bool queue_slot(uint32_t k, const uint32_t* __restrict__ count
     return found;
 }
 
-// Pixels of the 16x16 tiles [a, b) of a W x H image (tiles row-major).
-size_t tile_range_pixels(uint32_t a, uint32_t b, int W, int H)
-{
-    const uint32_t tx = (uint32_t)(W + 15) / 16u;
-    auto width_upto = [&](uint32_t x1) -> size_t {   // columns of tiles 0 .. x1 - 1 of a row
-        return x1 == 0 ? 0 : (size_t)16 * (x1 - 1) + (size_t)std::min(16, W - 16 * (int)(x1 - 1));
-    };
-    size_t n = 0;
-    for (uint32_t t = a; t < b;) {
-        const uint32_t y = t / tx, x0 = t % tx, x1 = std::min(tx, x0 + (b - t));
-        n += (width_upto(x1) - width_upto(x0)) * (size_t)std::min(16, H - 16 * (int)y);
-        t += x1 - x0;
-    }
-    return n;
-}
-
 // The queues for gi_bounce_kernel's grid (tile_grid, tiles dealt by
-// xcd_remap: XCD k takes tiles [k * per, (k + 1) * per), per = tiles / 8,
-// and the tiles from 8 * per on go one each to XCDs 0, 1, ...).  Returns
-// the total capacity, W * H.
+// screen_tile: XCD k takes tiles [k * per, (k + 1) * per) in strip order,
+// per = tiles / 8, and the tiles from 8 * per on go one each to XCDs 0, 1,
+// ...).  Returns the total capacity, W * H.
 uint32_t gi_queues(int W, int H, GiQueues& q)
 {
     const uint32_t tiles = ((uint32_t)(W + 15) / 16u) * ((uint32_t)(H + 15) / 16u);
     const uint32_t per = tiles / 8u;
     uint32_t base = 0;
     for (uint32_t k = 0; k < 8; k++) {
-        size_t cap = tile_range_pixels(k * per, (k + 1) * per, W, H);
-        if (8u * per + k < tiles) cap += tile_range_pixels(8u * per + k, 8u * per + k + 1, W, H);
+        size_t cap = vpt::strip_pixels((k + 1) * per, W, H) - vpt::strip_pixels(k * per, W, H);
+        if (8u * per + k < tiles) cap += vpt::strip_pixels(8u * per + k + 1, W, H) - vpt::strip_pixels(8u * per + k, W, H);
         q.base[k] = base;
         q.cap[k] = (uint32_t)cap;
         base += (uint32_t)cap;
@@ -1181,11 +1166,11 @@ __global__ void __launch_bounds__(256) reflect_rough2_kernel(WorldView w, CamVie
 {
     // 16x8 pixels per block: each wavefront 8x4 pixels, two lanes per pixel
     const uint32_t tiles_x = (uint32_t)(cam.W + 15) / 16u, tiles_y = (uint32_t)(cam.H + 7) / 8u;
-    const uint32_t tile = vpt::xcd_remap(blockIdx.x, tiles_x * tiles_y);
+    const vpt::TileXY tile = vpt::screen_tile(tiles_x, tiles_y);
     const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
     const int sample = lane & 1, pl = lane >> 1;
-    const int px = (int)(tile % tiles_x) * 16 + (wave & 1) * 8 + (pl & 7);
-    const int py = (int)(tile / tiles_x) * 8 + (wave >> 1) * 4 + (pl >> 3);
+    const int px = (int)tile.x * 16 + (wave & 1) * 8 + (pl & 7);
+    const int py = (int)tile.y * 8 + (wave >> 1) * 4 + (pl >> 3);
     const bool valid = px < cam.W && py < cam.H;   // the same for both lanes of a pair
     const size_t npx = (size_t)cam.W * cam.H;
     const size_t i = valid ? (size_t)py * cam.W + px : 0;
