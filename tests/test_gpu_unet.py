@@ -140,6 +140,51 @@ def test_denoise_entry_point(ctx, net):
     pm.close()
 
 
+@pytest.mark.parametrize("h,w", [(4, 4), (8, 16), (20, 12), (16, 36), (64, 60), (132, 100), (360, 640), (1080, 1920)])
+def test_denoise_activations(ctx, h, w):
+    """vpt_unet_denoise (16-channel input, head in the last convolution) and
+    vpt_unet_forward on the assembled input give the same activations and
+    output bit for bit, with odd tile remainders and with both tile sizes;
+    the last activation is the one of the weights that the pass ran with."""
+    torch = _torch()
+    from voxelpathtracer_amd import World, generate_terrain, gi_params, make_camera
+    from voxelpathtracer_amd.world import DeviceGBuffer
+    world = World(ctx, 64, 64, 64)
+    world.m_WorldData[...] = generate_terrain(64, 64, 64, h_min=10, h_max=45)
+    world.Buffer()
+    world.GenerateDistanceField()
+    cam, _, _ = make_camera((32.5, 52.5, 32.5), 40.0, -20.0, w, h)
+    gb = DeviceGBuffer(w, h)
+    tex = torch.empty((h, w, 8), dtype=torch.int16, device="cuda")
+    rgb = torch.empty((h, w, 3), dtype=torch.float32, device="cuda")
+    world.trace_primary(cam, gb, 350)
+    world.trace_gi(cam, gb, gi_params(50.0, 3), rgb, tex)
+    u = UNet(ctx, 1, h, w)
+    u.init(5)
+    x = torch.empty((h, w, 32), dtype=torch.int16, device="cuda")
+    a = torch.empty((h, w, 3), dtype=torch.float32, device="cuda")
+    b = torch.empty((h, w, 3), dtype=torch.float32, device="cuda")
+    u.assemble(gb, tex, x)
+    u.forward(x, 1, h, w, a, mode=1)
+    fwd = [u.activation(i, 1, h, w) for i in range(13)]
+    params = u.get_params()
+    u.denoise(gb, tex, b)
+    u.set_params(params * 1.5)   # the activations read below are the denoise pass's
+    den = [u.activation(i, 1, h, w) for i in range(13)]
+    np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+    for i in range(13):
+        np.testing.assert_array_equal(fwd[i], den[i], err_msg=str(i))
+    xf = bf16_to_f32(fwd[0])
+    with torch.no_grad():
+        ref_out, acts = unet_ref.forward(unet_ref.unpack(params), torch.from_numpy(xf))
+    # bf16 values of fp32 sums in another order, as in test_forward_matches_cpu
+    for i, name in ((9, "d1a"), (12, "d0b")):
+        assert _rel(bf16_to_f32(fwd[i]), acts[name].numpy()) < 1e-2, name
+    assert _rel(a.cpu().numpy(), np.maximum(np.expm1(ref_out.numpy()[0]), 0.0)) < 2e-2
+    u.close()
+    world.close()
+
+
 def test_training_beats_input(ctx, net):
     """Tracer-rendered pairs (1 spp -> 64 spp at 64x64), 150 Adam steps: the
     loss falls and the network beats its own 1-spp input on held-out pairs."""

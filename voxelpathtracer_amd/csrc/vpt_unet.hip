@@ -16,11 +16,12 @@
 // Activations are bf16 NHWC (channels a multiple of 32); weights are bf16
 // [tap][cout][cin] copies of fp32 master weights; every product accumulates
 // in fp32 on the MFMA units (v_mfma_f32_16x16x32_bf16).  A 3x3 convolution
-// is an implicit GEMM: M = 16 pixels of an output row, N = 16 output
-// channels, K = 32 input channels of one tap.  A 16x32 pixel tile and its
-// one-pixel halo are staged in LDS per 32-channel slice together with the
-// slice's weights for all nine taps; upsampling and concatenation are folded
-// into that staging, bias / ReLU / 2x2 average pooling into the epilogue.
+// is an implicit GEMM: M = 16 output channels, N = 16 pixels of an output
+// row, K = 32 input channels of one tap.  A pixel tile and its one-pixel
+// halo are loaded into LDS per 32-channel slice together with the slice's
+// weights for all nine taps; upsampling and concatenation are folded into
+// that load, bias / ReLU / 2x2 average pooling / the output head into the
+// epilogue.  vpt_unet_denoise's input has 16 stored channels (10 are used).
 // The backward pass reuses the forward kernel with flipped, transposed
 // weights (data gradient, ReLU mask in the epilogue) and an MFMA kernel for
 // the weight gradient (K = pixels, LDS-transposed tiles, per-slice partials
@@ -93,8 +94,16 @@ struct ConvArgs {
     const uint16_t* mask;// [n][h][w][cout]: y = acc where mask > 0, else 0 (no bias / ReLU)
     uint16_t* y;         // [n][h][w][cout]
     uint16_t* pool;      // [n][h/2][w/2][cout] 2x2 average of y, or null
+    const uint16_t* zero;// 1 KiB of zeros (read for pixels outside the image)
+    const float* head_w;  // [3][32], [3]: the 1x1 output head over y (32 channels), or null
+    const float* head_b;
+    float* head_out;     // [n][h][w][3]
+    int head_exp;        // head_out = max(exp(.) - 1, 0)
     int ca, cb, a_up, relu;
+    int a16;             // input A holds only its first 16 channels (the others are zero)
+    int* a16_out;        // a16 is noted here, or null
     int n, h, w_, cout;
+    int near;            // 32-bit byte offsets reach over a tile's halo
 };
 
 // Loads 8 channels (16 bytes) of the conv input at (img, gy, gx), channel
@@ -115,188 +124,416 @@ __device__ inline uint4 load_in8(const ConvArgs& p, int img, int gy, int gx, int
     return *reinterpret_cast<const uint4*>(p.b + off);
 }
 
-// 3x3 convolution, stride 1, zero padding, 512 threads on 16 x 32 pixel
-// tiles (wave v owns rows 4(v%4)..+3, columns 16(v/4)..+15), persistent: a workgroup
-// walks (tile, 32-channel slice) steps, tile = blockIdx.x + k * gridDim.x,
-// with the next step's global loads in flight (in registers) while the
-// current step is multiplied and the finished tile is written out.  The
-// epilogue goes through LDS so each lane stores 16 contiguous bytes.
-// Per wave and tap: NT weight fragments and 4 pixel-row fragments from LDS
-// (conflict-free 16-byte reads at an 80-byte pixel pitch) feed 4 x NT MFMAs.
-template <int COUT_T>
-__global__ void __launch_bounds__(512) conv3x3_wide_kernel(ConvArgs p)
+typedef __attribute__((address_space(1))) const void GlobalPtr;
+typedef __attribute__((address_space(3))) void LdsPtr;
+
+// Two floats rounded to bf16 (nearest even, as f2bf), a in the low half.
+__device__ inline uint32_t pack_bf(float a, float b)
 {
-    constexpr int NT = COUT_T / 16;
-    constexpr int TW = 32, TH = 16, HW = TW + 2, HH = TH + 2;
-    constexpr int A_ELEMS = HH * HW * 4;          // 16-byte pieces of the halo slice
-    constexpr int B_ELEMS = 9 * COUT_T * 4;       // 16-byte pieces of the weight slice
-    constexpr int A_PER = (A_ELEMS + 511) / 512;
-    constexpr int B_PER = (B_ELEMS + 511) / 512;
-    constexpr int OROW = COUT_T + 8;              // epilogue pitch (halves) per pixel
-    constexpr int A_BYTES = HH * HW * kRow * 2, B_BYTES = 9 * COUT_T * kRow * 2;
-    static_assert(8 * 64 * OROW * 2 <= A_BYTES + B_BYTES, "epilogue staging does not fit");
-    __shared__ __attribute__((aligned(16))) uint8_t smem[A_BYTES + B_BYTES];
-    uint16_t* sA = reinterpret_cast<uint16_t*>(smem);
-    uint16_t* sB = reinterpret_cast<uint16_t*>(smem + A_BYTES);
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// v of the other lane of each even-odd pair.
+__device__ inline float next_lane(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
+}
+
+// The sum of v over the lanes with the same lane % 16: v_permlane16_swap of
+// v with itself leaves the even and the odd row of each pair of 16-lane rows
+// in both rows, v_permlane32_swap likewise the halves.
+__device__ inline float sum_rows(float v)
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// This wave's LDS reads and asynchronous loads have ended, and every wave's
+// of the workgroup.  (The empty asm keeps the compiler from moving memory
+// operations across.)
+__device__ inline void wait_and_sync()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// The 16-byte piece q (0..3) of the 64-byte row `row` (32 bf16 values of a
+// pixel or of a weight row) lies at place (q + row / 2) % 4 of it: a 16-byte
+// read of the same piece of any 16 consecutive rows is then free of bank
+// conflicts (measured; q ^ (row / 2) % 4 is not for every first row).
+__device__ inline int piece_place(int q, int row) { return (q + (row >> 1)) & 3; }
+__device__ inline int place_piece(int place, int row) { return (place - (row >> 1)) & 3; }
+
+// 3x3 convolution, stride 1, zero padding, as an implicit GEMM: M = 16
+// output channels, N = 16 pixels of an output row, K = 32 input channels of
+// one tap.  A workgroup of WR x WC waves owns a tile of WR * R rows and
+// WC * 16 columns (wave (i, j): R rows, 16 columns) and is persistent: it
+// walks (tile, 32-channel slice) steps, tile = blockIdx.x + k * gridDim.x.
+// A step's halo slice (and, where the layer has more than one slice, its
+// weight slice) is loaded straight into LDS (global_load_lds, no registers)
+// while the step before is multiplied, two buffers, one barrier per step;
+// pixels outside the image read p.zero.  A pixel fragment is read once per
+// (halo row, dx) and multiplied into the up to three output rows that use
+// it, so a step reads 3 * (R + 2) pixel fragments for 9 * R * NT products.
+// The weight rows are ordered so that a lane ends with 8 consecutive
+// channels of its pixel for each 32 channels: bias, ReLU, mask, 2x2 pooling
+// and the 1x1 head run in registers, and 16 lanes store 1 KiB of
+// consecutive pixels (COUT = 32) with one 16-byte store each.
+// kOneSlice (32 input channels): the weights are loaded once per launch.
+// kHead: the network's last convolution, with the 1x1 output head over its
+// stored values in registers (p.y null: the values themselves are not
+// stored).
+// What bounds it at 1920x1080: the 32-channel layers at full resolution move
+// 266 to 300 MB (55 to 75 us, 4 to 5 TB/s), the 64-channel ones are held by
+// the products' issue and what a step does between them (d1a 105 us, 1.1
+// PFLOP/s of the 2.0 that random data sustains; its two waves per SIMD leave
+// the barrier together).  Measured, whole denoise call: 1920x1080 894 -> 632
+// us, 640x360 204 -> 134 us, against a kernel that staged through registers
+// behind two barriers a step, read each pixel fragment for each of the three
+// rows and stored through LDS, with the head and a 32-channel input apart.
+// A second workgroup per CU on 16x16 tiles was slower for these layers.
+template <int NT, int R, int WR, int WC, bool kOneSlice, bool kHead>
+__global__ void __launch_bounds__(64 * WR * WC) conv3x3_kernel(ConvArgs p)
+{
+    constexpr int NW = WR * WC, COUT = NT * 16;
+    // a halo row in LDS: TW + 2 pixels and 2 unused, so that a fragment's
+    // address is one of two per dx plus a constant (see below)
+    constexpr int TH = WR * R, TW = WC * 16, HW = TW + 4, HH = TH + 2;
+    constexpr int A_LOADS = (HH * HW * 4 + 63) / 64;      // 1 KiB wave loads of the halo slice
+    constexpr int B_LOADS = (9 * COUT * 4 + 63) / 64;     // of the weight slice
+    constexpr int A_PER = (A_LOADS + NW - 1) / NW, B_PER = (B_LOADS + NW - 1) / NW;
+    static_assert(9 * COUT * 4 % 64 == 0, "whole weight loads");
+    __shared__ __attribute__((aligned(16))) uint8_t sA0[A_LOADS * 1024], sA1[A_LOADS * 1024];
+    __shared__ __attribute__((aligned(16))) uint8_t sB0[B_LOADS * 1024], sB1[kOneSlice ? 16 : B_LOADS * 1024];
 
     const int tiles_x = (p.w_ + TW - 1) / TW, tiles_y = (p.h + TH - 1) / TH;
     const int per_img = tiles_x * tiles_y;
     const int ntiles = p.n * per_img;
-    const int co0 = blockIdx.y * COUT_T;
+    const int co0 = (int)blockIdx.y * COUT;
     const int cin = p.ca + p.cb;
-    const int nch = cin / kCi;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lm = lane & 15, lk = (lane >> 4) * 8;
-    const int wr = (wave & 3) * 4, wc = (wave >> 2) * 16;
+    const int nch = kOneSlice ? 1 : cin / kCi;
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lm = lane & 15, g = lane >> 4;
+    const int wr = (wave / WC) * R, wc = (wave % WC) * 16;
     if ((int)blockIdx.x >= ntiles) return;
     const int my_tiles = (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
     const int nsteps = my_tiles * nch;
 
-    uint4 ra[A_PER], rb[B_PER];
-    // loads of step `st` (tile blockIdx.x + (st / nch) * gridDim.x, slice st % nch)
-#define VPT_FETCH(ST)                                                                                               \
-    do {                                                                                                            \
-        const int t_ = (int)blockIdx.x + ((ST) / nch) * (int)gridDim.x;                                             \
-        const int c_ = ((ST) % nch) * kCi;                                                                          \
-        const int im_ = t_ / per_img;                                                                               \
-        const int y_ = ((t_ % per_img) / tiles_x) * TH, x_ = ((t_ % per_img) % tiles_x) * TW;                       \
-        _Pragma("unroll") for (int k = 0; k < A_PER; k++)                                                           \
-        {                                                                                                           \
-            const int e = tid + k * 512;                                                                            \
-            const int pix = e >> 2, q = e & 3;                                                                      \
-            ra[k] = e < A_ELEMS ? load_in8(p, im_, y_ + pix / HW - 1, x_ + pix % HW - 1, c_ + q * 8)                \
-                                : make_uint4(0u, 0u, 0u, 0u);                                                       \
-        }                                                                                                           \
-        _Pragma("unroll") for (int k = 0; k < B_PER; k++)                                                           \
-        {                                                                                                           \
-            const int e = tid + k * 512;                                                                            \
-            const int row = e >> 2, q = e & 3;                                                                      \
-            const int tap = row / COUT_T, co = row % COUT_T;                                                        \
-            rb[k] = e < B_ELEMS ? *reinterpret_cast<const uint4*>(p.w + ((size_t)tap * p.cout + co0 + co) * cin +   \
-                                                                  c_ + q * 8)                                       \
-                                : make_uint4(0u, 0u, 0u, 0u);                                                       \
-        }                                                                                                           \
-    } while (0)
-#define VPT_STASH()                                                                                                 \
-    do {                                                                                                            \
-        _Pragma("unroll") for (int k = 0; k < A_PER; k++)                                                           \
-        {                                                                                                           \
-            const int e = tid + k * 512;                                                                            \
-            if (e < A_ELEMS) *reinterpret_cast<uint4*>(&sA[(e >> 2) * kRow + (e & 3) * 8]) = ra[k];                \
-        }                                                                                                           \
-        _Pragma("unroll") for (int k = 0; k < B_PER; k++)                                                           \
-        {                                                                                                           \
-            const int e = tid + k * 512;                                                                            \
-            if (e < B_ELEMS) *reinterpret_cast<uint4*>(&sB[(e >> 2) * kRow + (e & 3) * 8]) = rb[k];                \
-        }                                                                                                           \
-    } while (0)
-
-    f32x4 acc[4][NT];
-    VPT_FETCH(0);
-    VPT_STASH();
-    __syncthreads();
-    for (int st = 0; st < nsteps; st++) {
-        const int chunk = st % nch;
-        if (chunk == 0) {
+    // This lane's byte offsets of its halo pieces from the halo's first
+    // pixel, in input A and in input B, and of its weight pieces from the
+    // slice's first channel: tiles inside the image then load with a scalar
+    // base and no address arithmetic.  LDS weight row tap * COUT + j * 16 +
+    // m holds output channel (j / 2) * 32 + (m / 4) * 8 + (j % 2) * 4 + m % 4.
+    uint32_t off_a[A_PER], off_b[kOneSlice ? 1 : A_PER], off_w[B_PER];
+    uint32_t upper = 0;   // bit k: piece k lies in channels 16..31
+    const int stride_a = kOneSlice && p.a16 ? 16 : p.ca;
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+    for (int k = 0; k < A_PER; k++) {
+        const int piece = (wave + k * NW) * 64 + lane, pix = min(piece >> 2, HH * HW - 1);
+        const int q = place_piece(piece & 3, piece >> 2);
+        const int hy = pix / HW, hx = min(pix % HW, TW + 1);
+        const int ya = p.a_up ? (hy + 1) >> 1 : hy, xa = p.a_up ? (hx + 1) >> 1 : hx;
+        off_a[k] = (uint32_t)(((ya * (p.w_ >> p.a_up) + xa) * stride_a + q * 8) * 2);
+        upper |= (uint32_t)(q >> 1) << k;
+        if (!kOneSlice) off_b[k] = (uint32_t)(((hy * p.w_ + hx) * p.cb + q * 8) * 2);
+    }
 #pragma unroll
-                for (int j = 0; j < NT; j++) acc[r][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < B_PER; k++) {
+        const int piece = (wave + k * NW) * 64 + lane, row = piece >> 2;
+        const int q = place_piece(piece & 3, row);
+        const int tap = row / COUT, j = row % COUT / 16, m = row % 16;
+        const int co = co0 + (j >> 1) * 32 + (m >> 2) * 8 + (j & 1) * 4 + (m & 3);
+        off_w[k] = (uint32_t)(((tap * p.cout + co) * cin + q * 8) * 2);
+    }
+    // The loads of a step, issued one by one between the products of the
+    // step before (issued together they stall a wave for some 2,000
+    // cycles): the addresses of this lane's halo pieces and weights.  A step
+    // on the same input and tile as the one before moves on by 64 bytes
+    // (p.zero has room for that); integer divisions and bounds are left to
+    // the steps that begin a tile or the other input.
+    const uint8_t* src_a[A_PER];
+    const uint16_t* src_w = p.w;
+    auto aim = [&](int t, int c) __attribute__((always_inline)) {
+        src_w = p.w + c * kCi;
+        if (c > 0 && c * kCi != p.ca) {
+#pragma unroll
+            for (int k = 0; k < A_PER; k++) src_a[k] += kCi * sizeof(uint16_t);
+            return;
         }
-        const bool more = st + 1 < nsteps;
-        if (more) VPT_FETCH(st + 1);
+        const int img = t / per_img, rem = t % per_img;
+        const int y0 = (rem / tiles_x) * TH, x0 = (rem % tiles_x) * TW;
+        const bool in_a = kOneSlice || c == 0;
+        const uint16_t* src = in_a ? p.a : p.b;
+        const int up = in_a ? p.a_up : 0;
+        const int ch = in_a ? stride_a : p.cb, hh = p.h >> up, ww = p.w_ >> up;
+        src += (size_t)img * hh * ww * ch;
+        if (p.near && y0 > 0 && x0 > 0 && y0 + TH < p.h && x0 + TW < p.w_) {
+            const uint8_t* base =
+                reinterpret_cast<const uint8_t*>(src + ((ptrdiff_t)((y0 >> up) - 1) * ww + (x0 >> up) - 1) * ch);
 #pragma unroll
-        for (int tap = 0; tap < 9; tap++) {
-            const int dy = tap / 3, dx = tap % 3;
-            bf16x8 bfr[NT];
+            for (int k = 0; k < A_PER; k++) src_a[k] = base + (kOneSlice || in_a ? off_a[k] : off_b[kOneSlice ? 0 : k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < A_PER; k++) {
+                const int piece = (wave + k * NW) * 64 + lane, pix = piece >> 2;
+                const int gy = y0 + pix / HW - 1, gx = x0 + pix % HW - 1;
+                const int q = place_piece(piece & 3, pix);
+                const bool in = (uint32_t)gy < (uint32_t)p.h && (uint32_t)gx < (uint32_t)p.w_ && pix < HH * HW &&
+                                pix % HW < TW + 2;
+                const uint16_t* at = src + ((ptrdiff_t)(gy >> up) * ww + (gx >> up)) * ch + q * 8;
+                src_a[k] = reinterpret_cast<const uint8_t*>(in ? at : p.zero);
+            }
+        }
+        if (kOneSlice && p.a16) {
+            // channels 16..31 of the input are not stored: zeros
+#pragma unroll
+            for (int k = 0; k < A_PER; k++)
+                if (upper >> k & 1) src_a[k] = reinterpret_cast<const uint8_t*>(p.zero);
+        }
+    };
+    auto load = [&](int k, bool weights, uint8_t* la, uint8_t* lb) __attribute__((always_inline)) {
+        if (k < A_PER) {
+            const int i = wave + k * NW;
+            if (i < A_LOADS)
+                __builtin_amdgcn_global_load_lds((GlobalPtr*)src_a[k], (LdsPtr*)(la + i * 1024), 16, 0, 0);
+        } else if (weights && k < A_PER + B_PER) {
+            const int i = wave + (k - A_PER) * NW;
+            if (i < B_LOADS)
+                __builtin_amdgcn_global_load_lds(
+                    (GlobalPtr*)(reinterpret_cast<const uint8_t*>(src_w) + off_w[k - A_PER]), (LdsPtr*)(lb + i * 1024),
+                    16, 0, 0);
+        }
+    };
+    auto frag = [&](const uint8_t* s, int row) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16x8*>(s + row * 64 + piece_place(g, row) * 16);
+    };
+
+    f32x4 acc[R][NT];
+    constexpr bool kRegs = kOneSlice && NT == 2;   // 72 registers; 64 channels' weights stay in LDS
+    bf16x8 wreg[kRegs ? 9 : 1][NT];
+    // One step's products; hook(i) runs before item i's (an item: one halo
+    // row and dx).  Fragments are read ahead of their use: pixel fragments
+    // two items ahead, the weights of (dx, dy), which items dy .. dy + R - 1
+    // of dx use, into the registers that the dx before has just left.  The
+    // scheduling barriers keep the compiler from sinking the reads to the
+    // products that wait for them.
+    constexpr int kItems = 3 * (R + 2);
+    // this lane's pixel of the wave's first halo row, for each dx and for
+    // even and odd halo rows: HW / 2 = 2 (mod 4), so a piece's place moves by
+    // two from row to row
+    static_assert(HW % 8 == 4 && R * HW % 8 == 0, "places repeat every two halo rows");
+    uint32_t pix_at[3][2];
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            const int row = wr * HW + wc + lm + dx;
+            pix_at[dx][v] = (uint32_t)(row * 64 + piece_place(g, row + v * HW) * 16);
+        }
+    auto multiply = [&](const uint8_t* sA, const uint8_t* sB, auto&& hook) __attribute__((always_inline)) {
+        bf16x8 px[3], wf[kRegs ? 1 : 3][NT];
+        auto pixels = [&](int i) __attribute__((always_inline)) {
+            const int hy = i % (R + 2);
+            return *reinterpret_cast<const bf16x8*>(sA + pix_at[i / (R + 2)][hy & 1] + hy * (HW * 64));
+        };
+        auto weights = [&](int dx, int dy) __attribute__((always_inline)) {
+            if (kRegs || dx > 2) return;
 #pragma unroll
             for (int j = 0; j < NT; j++)
-                bfr[j] = *reinterpret_cast<const bf16x8*>(&sB[(tap * COUT_T + j * 16 + lm) * kRow + lk]);
+                wf[kRegs ? 0 : dy][j] = frag(kOneSlice ? sB0 : sB, (dy * 3 + dx) * COUT + j * 16 + lm);
+        };
+        weights(0, 0);
+        px[0] = pixels(0);
+        px[1] = pixels(1);
+        weights(0, 1);
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int hy = wr + r + dy, hx = wc + lm + dx;
-                const bf16x8 afr = *reinterpret_cast<const bf16x8*>(&sA[(hy * HW + hx) * kRow + lk]);
+        for (int i = 0; i < kItems; i++) {
+            const int dx = i / (R + 2), hy = i % (R + 2);
+            if (i + 2 < kItems) px[(i + 2) % 3] = pixels(i + 2);
+            if (hy == 0) weights(dx, 2);
+            if (hy == R) weights(dx + 1, 0);
+            if (hy == R + 1) weights(dx + 1, 1);
+            hook(i);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                const int r = hy - dy;
+                if (r < 0 || r >= R) continue;
 #pragma unroll
                 for (int j = 0; j < NT; j++)
-                    acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr, bfr[j], acc[r][j], 0, 0, 0);
+                    acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        kRegs ? wreg[kRegs ? dy * 3 + dx : 0][j] : wf[kRegs ? 0 : dy][j], px[i % 3], acc[r][j], 0, 0,
+                        0);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
-        if (chunk == nch - 1) {
-            // the tile is complete: epilogue, part 1: bias / ReLU in
-            // registers, bf16 values into this wave's LDS block [64 px][COUT_T],
-            // pooled values stored directly
-            const int t = (int)blockIdx.x + (st / nch) * (int)gridDim.x;
-            const int img = t / per_img;
-            const int ty0 = ((t % per_img) / tiles_x) * TH, tx0 = ((t % per_img) % tiles_x) * TW;
-            uint16_t* so = reinterpret_cast<uint16_t*>(smem) + wave * 64 * OROW;
-            const int xl = 4 * (lane >> 4);
+    };
+
+    // this lane's biases and head weights, read once (in each tile's finish
+    // their latency was exposed)
+    float bias[NT * 4], head[kHead ? 24 : 1], head_b = 0.0f;
 #pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const int col = j * 16 + lm;
-                const float bias = p.bias ? p.bias[co0 + col] : 0.0f;
+    for (int i = 0; i < NT * 4; i++) bias[i] = p.bias ? p.bias[co0 + (i >> 3) * 32 + g * 8 + (i & 7)] : 0.0f;
+    if (kHead) {
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
+        for (int i = 0; i < (kHead ? 24 : 1); i++) head[i] = p.head_w[(i >> 3) * 32 + g * 8 + (i & 7)];
+        head_b = p.head_b[min(g, 2)];
+    }
+    // The finished tile: its values in bf16; with 32 channels stored one by
+    // one between the products of the next tile (64 channels' values would
+    // not fit in the registers).
+    constexpr bool kLater = NT == 2;
+    constexpr int kStores = R * (NT / 2);
+    uint4 out[kLater ? kStores : R];
+    uint16_t* out_at = nullptr;   // this lane's first pixel and channel
+    int out_rows = 0;             // its rows inside the image (0: its column is outside)
+    auto store = [&](int k) __attribute__((always_inline)) {
+        const int jp = k / R, r = k % R;
+        if (r < out_rows && (!kHead || p.y))
+            *reinterpret_cast<uint4*>(out_at + (size_t)r * p.w_ * p.cout + jp * 32) = out[kLater ? k : r];
+    };
+    auto finish = [&](int t) __attribute__((always_inline)) {
+        const int img = t / per_img;
+        const int ty0 = ((t % per_img) / tiles_x) * TH + wr, gx = ((t % per_img) % tiles_x) * TW + wc + lm;
+        const size_t first = (((size_t)img * p.h + ty0) * p.w_ + gx) * p.cout + co0 + g * 8;
+        out_at = p.y + first;
+        out_rows = gx < p.w_ ? min(R, p.h - ty0) : 0;
+#pragma unroll
+        for (int jp = 0; jp < NT / 2; jp++) {
+            uint4* o = out + (kLater ? jp * R : 0);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    v[i] = acc[r][2 * jp + (i >> 2)][i & 3];
+                    if (p.relu) v[i] = fmaxf(v[i] + bias[jp * 8 + i], 0.0f);
+                }
+                o[r] = make_uint4(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]), pack_bf(v[4], v[5]), pack_bf(v[6], v[7]));
+            }
+            if (p.mask) {
+                uint4 mk[R];
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    mk[r] = r < out_rows ? *reinterpret_cast<const uint4*>(p.mask + first + (size_t)r * p.w_ * p.cout +
+                                                                           jp * 32)
+                                         : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    o[r] = make_uint4(mask_pair(o[r].x, mk[r].x), mask_pair(o[r].y, mk[r].y),
+                                      mask_pair(o[r].z, mk[r].z), mask_pair(o[r].w, mk[r].w));
+            }
+            if (kHead) {
+                // the head over the stored values: 8 channels here, the
+                // other 24 of the pixel in lanes +-16, +-32
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const uint32_t u[4] = {o[r].x, o[r].y, o[r].z, o[r].w};
+                    float s[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const float v = __uint_as_float(i & 1 ? u[i >> 1] & 0xffff0000u : u[i >> 1] << 16);
+#pragma unroll
+                        for (int j = 0; j < 3; j++) s[j] += head[j * 8 + i] * v;
+                    }
+#pragma unroll
+                    for (int j = 0; j < 3; j++) {
+                        s[j] = sum_rows(s[j]);
+                    }
+                    // lane group g writes component g
+                    float m = (g == 0 ? s[0] : (g == 1 ? s[1] : s[2])) + head_b;
+                    if (p.head_exp) m = fmaxf(expm1f(m), 0.0f);
+                    if (g < 3 && r < out_rows)
+                        p.head_out[(((size_t)img * p.h + ty0 + r) * p.w_ + gx) * 3 + g] = m;
+                }
+            }
+            if (!kLater) {
+#pragma unroll
+                for (int r = 0; r < R; r++) store(jp * R + r);
+            }
+            if (p.pool) {
+                // 2x2 averages of the stored values: the right neighbour's
+                // pixel is the next lane's
+                const int ph = p.h >> 1, pw = p.w_ >> 1;
+#pragma unroll
+                for (int r = 0; r < R; r += 2) {
+                    const uint32_t u[4] = {o[r].x, o[r].y, o[r].z, o[r].w};
+                    const uint32_t d[4] = {o[r + 1].x, o[r + 1].y, o[r + 1].z, o[r + 1].w};
+                    uint32_t q[4];
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        float v = acc[r][j][i];
-                        if (!p.mask) {
-                            v += bias;
-                            if (p.relu) v = fmaxf(v, 0.0f);
-                        }
-                        const uint16_t hv = f2bf(v);
-                        acc[r][j][i] = bf2f(hv);   // the stored value, for the pooled output
-                        so[(r * 16 + xl + i) * OROW + col] = hv;
-                    }
-                }
-                if (p.pool) {
-                    const int ph = p.h >> 1, pw = p.w_ >> 1;
+                        float s[2];
 #pragma unroll
-                    for (int r2 = 0; r2 < 2; r2++) {
-                        const int gy = ty0 + wr + 2 * r2;
-#pragma unroll
-                        for (int i2 = 0; i2 < 2; i2++) {
-                            const int gx = tx0 + wc + xl + 2 * i2;
-                            if (gy < p.h && gx < p.w_) {
-                                const f32x4 a = acc[2 * r2][j], b = acc[2 * r2 + 1][j];
-                                const float sm = ((a[2 * i2] + a[2 * i2 + 1]) + (b[2 * i2] + b[2 * i2 + 1])) * 0.25f;
-                                p.pool[(((size_t)img * ph + (gy >> 1)) * pw + (gx >> 1)) * p.cout + co0 + col] =
-                                    f2bf(sm);
-                            }
+                        for (int h = 0; h < 2; h++) {
+                            const float a = __uint_as_float(h ? u[i] & 0xffff0000u : u[i] << 16);
+                            const float b = __uint_as_float(h ? d[i] & 0xffff0000u : d[i] << 16);
+                            const float a1 = next_lane(a), b1 = next_lane(b);
+                            s[h] = ((a + a1) + (b + b1)) * 0.25f;
                         }
+                        q[i] = pack_bf(s[0], s[1]);
                     }
+                    if ((lm & 1) == 0 && r < out_rows)
+                        *reinterpret_cast<uint4*>(p.pool +
+                                                  (((size_t)img * ph + ((ty0 + r) >> 1)) * pw + (gx >> 1)) * p.cout +
+                                                  co0 + jp * 32 + g * 8) = make_uint4(q[0], q[1], q[2], q[3]);
                 }
             }
-            __builtin_amdgcn_s_waitcnt(0);
-            __builtin_amdgcn_wave_barrier();
-            // part 2: 16-byte stores of 8 channels of one pixel (mask applied here)
-            constexpr int CH8 = COUT_T / 8;
+        }
+    };
+    if (p.a16_out && blockIdx.x == 0 && threadIdx.x == 0) *p.a16_out = p.a16;
+    {
+        aim((int)blockIdx.x, 0);
 #pragma unroll
-            for (int k = 0; k < CH8; k++) {
-                const int e = lane + k * 64;
-                const int px = e / CH8, c8 = e % CH8;
-                const int gy = ty0 + wr + (px >> 4), gx = tx0 + wc + (px & 15);
-                if (gy >= p.h || gx >= p.w_) continue;
-                uint4 v = *reinterpret_cast<const uint4*>(&so[px * OROW + c8 * 8]);
-                const size_t off = (((size_t)img * p.h + gy) * p.w_ + gx) * p.cout + co0 + c8 * 8;
-                if (p.mask) {
-                    const uint4 mk = *reinterpret_cast<const uint4*>(p.mask + off);
-                    v.x = mask_pair(v.x, mk.x);
-                    v.y = mask_pair(v.y, mk.y);
-                    v.z = mask_pair(v.z, mk.z);
-                    v.w = mask_pair(v.w, mk.w);
-                }
-                *reinterpret_cast<uint4*>(p.y + off) = v;
-            }
-            __syncthreads();
-        }
-        if (more) {
-            VPT_STASH();
-            __syncthreads();
-        }
+        for (int k = 0; k < A_PER + B_PER; k++) load(k, true, sA0, sB0);
     }
-#undef VPT_FETCH
-#undef VPT_STASH
+    if (kRegs) {
+        wait_and_sync();
+#pragma unroll
+        for (int tap = 0; tap < (kRegs ? 9 : 1); tap++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) wreg[tap][j] = frag(sB0, tap * COUT + j * 16 + lm);
+    }
+    // step st: its loads have ended; between its products go the next
+    // step's loads, into the other buffers, and the stores of the tile that
+    // the step before finished
+    int t = (int)blockIdx.x, c = 0;
+    auto step = [&](int st, const uint8_t* a, const uint8_t* b, uint8_t* na, uint8_t* nb)
+        __attribute__((always_inline)) {
+            wait_and_sync();
+            const bool more = st + 1 < nsteps, done = c == 0 && st > 0;
+            const bool last = c + 1 == nch;
+            if (more) aim(last ? t + (int)gridDim.x : t, last ? 0 : c + 1);
+            if (done) finish(t - (int)gridDim.x);
+            if (c == 0) {
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[r][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            multiply(a, b, [&](int i) __attribute__((always_inline)) {
+                if (more) load(i, !kOneSlice, na, nb);
+                if (kLater && done && i < kStores) store(i);
+            });
+            c = last ? 0 : c + 1;
+            t = last ? t + (int)gridDim.x : t;
+        };
+    static_assert(A_PER + B_PER <= kItems && kStores <= kItems, "a step holds its loads and stores");
+    for (int st = 0; st < nsteps; st += 2) {
+        step(st, sA0, sB0, sA1, sB1);
+        if (st + 1 < nsteps) step(st + 1, sA1, sB1, sA0, sB0);
+    }
+    finish(t - (int)gridDim.x);
+    if (kLater) {
+#pragma unroll
+        for (int k = 0; k < kStores; k++) store(k);
+    }
 }
 
 // Weight gradient of a 3x3 convolution:
@@ -415,30 +652,6 @@ __global__ void flip_transpose_kernel(const uint16_t* __restrict__ w, int cout, 
     const int tap = i / (cout * cin), rem = i % (cout * cin);
     const int co = rem / cin, ci = rem % cin;
     wt[((size_t)(8 - tap) * cin + ci) * cout + co] = w[i];
-}
-
-// Output head: out[px][j] = b[j] + sum_c W[j][c] * d0b[px][c] (fp32).
-// mode 0: log-space prediction; mode 1: irradiance max(exp(out) - 1, 0).
-__global__ void head_kernel(const uint16_t* __restrict__ x, size_t npx, const float* __restrict__ wh,
-                            const float* __restrict__ bh, int mode, float* __restrict__ out)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= npx) return;
-    float v[32];
-    const uint4* src = reinterpret_cast<const uint4*>(x + i * 32);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const uint4 u = src[q];
-        const uint16_t* h = reinterpret_cast<const uint16_t*>(&u);
-#pragma unroll
-        for (int k = 0; k < 8; k++) v[q * 8 + k] = bf2f(h[k]);
-    }
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        float s = bh[j];
-        for (int c = 0; c < 32; c++) s += wh[j * 32 + c] * v[c];
-        out[i * 3 + j] = mode ? fmaxf(expm1f(s), 0.0f) : s;
-    }
 }
 
 // Loss and head gradient, one thread per pixel; 256-thread blocks write
@@ -587,6 +800,7 @@ __device__ inline void texel_values(const vpt_svgf_texel& t, float v[6])
 // Network input: ch 0-2 log1p(1-spp irradiance), 3-5 albedo of the hit
 // block, 6-8 face normal, 9 log1p(hit distance) / 8, 10-31 zero.  Sky
 // pixels: irradiance of their texel, zero albedo / normal / depth.
+template <int kPieces>   // 16-byte pieces stored per pixel: 4, or 2 (channels 0..15)
 __global__ void assemble_kernel(int npx, const float* __restrict__ gb_t, const uint8_t* __restrict__ gb_face,
                                 const uint8_t* __restrict__ gb_block, const vpt_svgf_texel* __restrict__ tex,
                                 const vpt::AlbedoTable albedo, uint16_t* __restrict__ x)
@@ -597,9 +811,9 @@ __global__ void assemble_kernel(int npx, const float* __restrict__ gb_t, const u
     texel_values(tex[i], v);
     const int face = gb_face[i];
     const Decoded d = sh_decode(v, v[4], v[5], face);
-    uint16_t o[32];
+    uint16_t o[8 * kPieces];
 #pragma unroll
-    for (int k = 0; k < 32; k++) o[k] = 0;
+    for (int k = 0; k < 8 * kPieces; k++) o[k] = 0;
     o[0] = f2bf(log1pf(d.r));
     o[1] = f2bf(log1pf(d.g));
     o[2] = f2bf(log1pf(d.b));
@@ -615,9 +829,9 @@ __global__ void assemble_kernel(int npx, const float* __restrict__ gb_t, const u
         o[8] = f2bf(nrm.z);
         o[9] = f2bf(log1pf(t) * 0.125f);
     }
-    uint4* dst = reinterpret_cast<uint4*>(x + (size_t)i * 32);
+    uint4* dst = reinterpret_cast<uint4*>(x + (size_t)i * 8 * kPieces);
 #pragma unroll
-    for (int q = 0; q < 4; q++) dst[q] = *reinterpret_cast<const uint4*>(&o[q * 8]);
+    for (int q = 0; q < kPieces; q++) dst[q] = *reinterpret_cast<const uint4*>(&o[q * 8]);
 }
 
 // acc[i][0..5] (+)= SH-Y, Co, Cg of texel i.
@@ -674,21 +888,44 @@ const Layer kNet[kLayers] = {
     {D1B, E0B, 1, D0A, -1, 96, 32, 0, 0, 0},    {D0A, -1, 0, D0B, -1, 32, 32, 0, 0, 0},
 };
 
-// Persistent workgroups: one per CU and output-channel block (the wide
-// kernel holds one workgroup per CU), never more than the tiles.
+// Persistent workgroups: one per CU and output-channel block (the large
+// tiles' LDS holds one workgroup per CU), never more than the tiles.
 int g_cus = 0;
 
+template <int NT, int R, int WR, int WC, bool kOneSlice, bool kHead = false>
+void conv_go(const ConvArgs& a, int per_cu, hipStream_t s)
+{
+    const int th = WR * R, tw = WC * 16;
+    const int tiles = a.n * ((a.h + th - 1) / th) * ((a.w_ + tw - 1) / tw);
+    const int blocks_y = a.cout / (NT * 16);
+    const int gx = std::min(tiles, std::max(1, per_cu * g_cus / blocks_y));
+    ConvArgs b = a;
+    b.near = (size_t)(th + 2) * a.w_ * std::max(a.ca, a.cb) * sizeof(uint16_t) < ((size_t)1 << 31);
+    hipLaunchKernelGGL((conv3x3_kernel<NT, R, WR, WC, kOneSlice, kHead>), dim3((unsigned)gx, (unsigned)blocks_y),
+                       dim3(64 * WR * WC), 0, s, b);
+}
+
+// 16 x 32 tiles, one workgroup per CU; where those would leave CUs idle (the
+// lower levels of small images), 8 x 16 tiles, 32 channels a workgroup, two
+// workgroups per CU.  The line is one large tile per CU: 120 large tiles
+// (64 -> 64 channels at 320x180) take 15.0 us, in small ones 12.9 us; 460
+// (96 -> 32 at 640x360) take 20.6 us, in small ones 24.5 us.
 int launch_conv(const ConvArgs& a, hipStream_t s)
 {
+    const bool one = a.ca + a.cb == kCi, wide = a.cout % 64 == 0;
     const int tiles = a.n * ((a.h + 15) / 16) * ((a.w_ + 31) / 32);
-    const int cout_t = a.cout % 64 == 0 ? 64 : 32;
-    const int blocks_y = a.cout / cout_t;
-    const int per_block = std::max(1, g_cus / blocks_y);
-    const unsigned gx = (unsigned)std::min(tiles, per_block);
-    if (cout_t == 64) {
-        hipLaunchKernelGGL(conv3x3_wide_kernel<64>, dim3(gx, (unsigned)blocks_y), dim3(512), 0, s, a);
+    if (tiles * (wide ? a.cout / 64 : 1) < g_cus) {
+        if (a.head_w) {
+            conv_go<2, 2, 4, 1, true, true>(a, 2, s);
+        } else {
+            one ? conv_go<2, 2, 4, 1, true>(a, 2, s) : conv_go<2, 2, 4, 1, false>(a, 2, s);
+        }
+    } else if (a.head_w) {
+        conv_go<2, 4, 4, 2, true, true>(a, 1, s);
+    } else if (wide) {
+        one ? conv_go<4, 4, 4, 2, true>(a, 1, s) : conv_go<4, 4, 4, 2, false>(a, 1, s);
     } else {
-        hipLaunchKernelGGL(conv3x3_wide_kernel<32>, dim3(gx, (unsigned)blocks_y), dim3(512), 0, s, a);
+        one ? conv_go<2, 4, 4, 2, true>(a, 1, s) : conv_go<2, 4, 4, 2, false>(a, 1, s);
     }
     HIP_TRY(hipGetLastError());
     return VPT_OK;
@@ -715,11 +952,14 @@ struct vpt_unet {
     uint16_t* d_gcat = nullptr;  // data gradient of a concatenated input
     uint16_t* d_gpool[2] = {};   // gradients of P0, P1
     float* d_pred = nullptr;
+    uint16_t* d_zero = nullptr;  // zeros, read for pixels outside the image
     float* d_part = nullptr;     // weight-gradient partials
     size_t part_floats = 0;
     float* d_head_part = nullptr;
     int slices = 0;
     int adam_t = 0;
+    int* d_x16 = nullptr;        // act[X] holds 16 channels per pixel (vpt_unet_denoise), not 32
+    int last_n = 0, last_h = 0, last_w = 0;   // the last forward pass, while its D0B is not stored (last_n 0: it is)
     float last_loss = 0.0f;
 };
 
@@ -751,6 +991,7 @@ ConvArgs conv_args(vpt_unet* u, const Layer& L, int n, int h, int w)
     a.y = u->act[L.out];
     a.pool = L.pool >= 0 ? u->act[L.pool] : nullptr;
     a.relu = 1;
+    a.zero = u->d_zero;
     a.n = n;
     a.h = h >> L.level;
     a.w_ = w >> L.level;
@@ -758,10 +999,47 @@ ConvArgs conv_args(vpt_unet* u, const Layer& L, int n, int h, int w)
     return a;
 }
 
-int forward(vpt_unet* u, int n, int h, int w, hipStream_t s)
+// The network from act[X] to `out` (exp: irradiance, else log space).  The
+// last layer's activation is stored only when keep_last is set (the backward
+// pass reads it); read_activation makes it again from the layer before.
+int forward(vpt_unet* u, int n, int h, int w, bool x16, bool keep_last, float* out, bool exp, hipStream_t s)
 {
-    for (int l = 0; l < kLayers; l++)
-        if (int rc = launch_conv(conv_args(u, u->net[l], n, h, w), s)) return rc;
+    for (int l = 0; l < kLayers; l++) {
+        ConvArgs a = conv_args(u, u->net[l], n, h, w);
+        if (l == 0) {
+            a.a16 = x16;
+            a.a16_out = u->d_x16;
+        }
+        if (l == kLayers - 1) {
+            a.head_w = u->d_w + u->head_w;
+            a.head_b = u->d_w + u->head_b;
+            a.head_out = out;
+            a.head_exp = exp;
+            if (!keep_last) a.y = nullptr;
+        }
+        if (int rc = launch_conv(a, s)) return rc;
+    }
+    u->last_n = keep_last ? 0 : n;
+    u->last_h = h;
+    u->last_w = w;
+    return VPT_OK;
+}
+
+// Stores the last forward pass's D0B, if it was not, from its D0A: before
+// the weights change, and when it is read.
+int make_last(vpt_unet* u, int n, int h, int w, hipStream_t s)
+{
+    if (!u->last_n) return VPT_OK;
+    u->last_n = 0;
+    return launch_conv(conv_args(u, u->net[kLayers - 1], n, h, w), s);
+}
+
+// A captured pass stores everything, since its replays cannot be known here.
+int is_capturing(hipStream_t s, bool* out)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(s, &cs));
+    *out = cs != hipStreamCaptureStatusNone;
     return VPT_OK;
 }
 
@@ -805,6 +1083,7 @@ int dgrad(vpt_unet* u, const Layer& L, int n, int h, int w, const uint16_t* m, c
     a.w = u->d_wt;
     a.mask = mask;
     a.y = out;
+    a.zero = u->d_zero;
     a.n = n;
     a.h = h >> L.level;
     a.w_ = w >> L.level;
@@ -914,6 +1193,10 @@ struct DeviceGuard {
 
 int unet_upload(vpt_unet* u, const float* host)
 {
+    if (u->last_n) {
+        HIP_TRY(hipDeviceSynchronize());
+        if (int rc = make_last(u, u->last_n, u->last_h, u->last_w, nullptr)) return rc;
+    }
     HIP_TRY(hipMemcpy(u->d_w, host, sizeof(float) * u->n_params, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks_for(u->n_params)), dim3(256), 0, nullptr, u->d_w, u->d_wb,
                        u->n_params);
@@ -945,6 +1228,8 @@ extern "C" VPT_API int vpt_unet_destroy(vpt_unet* u)
     (void)hipFree(u->d_gpool[0]);
     (void)hipFree(u->d_gpool[1]);
     (void)hipFree(u->d_pred);
+    (void)hipFree(u->d_zero);
+    (void)hipFree(u->d_x16);
     (void)hipFree(u->d_part);
     (void)hipFree(u->d_head_part);
     delete u;
@@ -1000,8 +1285,12 @@ extern "C" VPT_API int vpt_unet_create(vpt_ctx* ctx, int max_n, int max_h, int m
     alloc((void**)&u->d_gpool[0], sizeof(uint16_t) * (full >> 2) * 32);
     alloc((void**)&u->d_gpool[1], sizeof(uint16_t) * (full >> 4) * 64);
     alloc((void**)&u->d_pred, sizeof(float) * full * 3);
+    alloc((void**)&u->d_zero, 1024);
+    alloc((void**)&u->d_x16, sizeof(int));
     alloc((void**)&u->d_part, sizeof(float) * u->part_floats);
     alloc((void**)&u->d_head_part, sizeof(float) * 100 * ((full + 255) / 256));
+    if (e == hipSuccess) e = hipMemset(u->d_zero, 0, 1024);
+    if (e == hipSuccess) e = hipMemset(u->d_x16, 0, sizeof(int));
     if (e != hipSuccess) {
         vpt_unet_destroy(u);
         return set_error(VPT_ENOMEM, "vpt_unet_create: allocation failed (%s)", hipGetErrorString(e));
@@ -1071,11 +1360,9 @@ extern "C" VPT_API int vpt_unet_forward(vpt_unet* u, const uint16_t* d_x, int n,
     hipStream_t s = (hipStream_t)stream;
     const size_t npx = (size_t)n * h * w;
     HIP_TRY(hipMemcpyAsync(u->act[X], d_x, sizeof(uint16_t) * npx * 32, hipMemcpyDeviceToDevice, s));
-    if (int rc = forward(u, n, h, w, s)) return rc;
-    hipLaunchKernelGGL(head_kernel, dim3(blocks_for(npx)), dim3(256), 0, s, u->act[D0B], npx, u->d_w + u->head_w,
-                       u->d_w + u->head_b, mode, d_out);
-    HIP_TRY(hipGetLastError());
-    return VPT_OK;
+    bool capturing = false;
+    if (int rc = is_capturing(s, &capturing)) return rc;
+    return forward(u, n, h, w, false, capturing, d_out, mode == 1, s);
 }
 
 extern "C" VPT_API int vpt_unet_backward(vpt_unet* u, const uint16_t* d_x, const float* d_target, int n, int h, int w,
@@ -1087,10 +1374,7 @@ extern "C" VPT_API int vpt_unet_backward(vpt_unet* u, const uint16_t* d_x, const
     hipStream_t s = (hipStream_t)stream;
     const size_t npx = (size_t)n * h * w;
     HIP_TRY(hipMemcpyAsync(u->act[X], d_x, sizeof(uint16_t) * npx * 32, hipMemcpyDeviceToDevice, s));
-    if (int rc = forward(u, n, h, w, s)) return rc;
-    hipLaunchKernelGGL(head_kernel, dim3(blocks_for(npx)), dim3(256), 0, s, u->act[D0B], npx, u->d_w + u->head_w,
-                       u->d_w + u->head_b, 0, u->d_pred);
-    HIP_TRY(hipGetLastError());
+    if (int rc = forward(u, n, h, w, false, true, u->d_pred, false, s)) return rc;
     if (int rc = backward(u, d_target, n, h, w, s)) return rc;
     if (loss) {
         float sum = 0.0f;
@@ -1106,6 +1390,7 @@ extern "C" VPT_API int vpt_unet_adam_step(vpt_unet* u, float lr, void* stream)
     if (!u || !(lr > 0.0f)) return set_error(VPT_EINVAL, "vpt_unet_adam_step: bad arguments");
     DeviceGuard g(u->device);
     const float b1 = 0.9f, b2 = 0.999f;
+    if (int rc = make_last(u, u->last_n, u->last_h, u->last_w, (hipStream_t)stream)) return rc;
     u->adam_t++;
     const float c1 = 1.0f / (1.0f - powf(b1, (float)u->adam_t));
     const float c2 = 1.0f / (1.0f - powf(b2, (float)u->adam_t));
@@ -1115,24 +1400,30 @@ extern "C" VPT_API int vpt_unet_adam_step(vpt_unet* u, float lr, void* stream)
     return VPT_OK;
 }
 
-extern "C" VPT_API int vpt_unet_assemble(vpt_unet* u, const vpt_gbuffer* gb, const vpt_svgf_texel* d_tex,
-                                         uint16_t* d_x, void* stream)
+// The network's input; x16: only channels 0..15, 32 bytes a pixel.
+static int assemble(const char* fn, vpt_unet* u, const vpt_gbuffer* gb, const vpt_svgf_texel* d_tex, uint16_t* d_x,
+                    bool x16, void* stream)
 {
     if (!u || !gb || !d_tex || !d_x || !gb->d_t || !gb->d_face || !gb->d_block)
-        return set_error(VPT_EINVAL, "vpt_unet_assemble: null argument");
+        return set_error(VPT_EINVAL, "%s: null argument", fn);
     vpt::AlbedoTable albedo;
     {
         std::lock_guard<std::mutex> lk(u->ctx->mu);
-        if (!u->ctx->albedo_valid)
-            return set_error(VPT_ESTATE, "vpt_unet_assemble: no albedo table yet (trace GI first)");
+        if (!u->ctx->albedo_valid) return set_error(VPT_ESTATE, "%s: no albedo table yet (trace GI first)", fn);
         memcpy(albedo.v, u->ctx->albedo_host, sizeof(albedo.v));
     }
     DeviceGuard g(u->device);
     const int npx = gb->width * gb->height;
-    hipLaunchKernelGGL(assemble_kernel, dim3(blocks_for((size_t)npx)), dim3(256), 0, (hipStream_t)stream, npx,
-                       gb->d_t, gb->d_face, gb->d_block, d_tex, albedo, d_x);
+    hipLaunchKernelGGL(x16 ? assemble_kernel<2> : assemble_kernel<4>, dim3(blocks_for((size_t)npx)), dim3(256), 0,
+                       (hipStream_t)stream, npx, gb->d_t, gb->d_face, gb->d_block, d_tex, albedo, d_x);
     HIP_TRY(hipGetLastError());
     return VPT_OK;
+}
+
+extern "C" VPT_API int vpt_unet_assemble(vpt_unet* u, const vpt_gbuffer* gb, const vpt_svgf_texel* d_tex,
+                                         uint16_t* d_x, void* stream)
+{
+    return assemble("vpt_unet_assemble", u, gb, d_tex, d_x, false, stream);
 }
 
 extern "C" VPT_API int vpt_unet_denoise(vpt_unet* u, const vpt_gbuffer* gb, const vpt_svgf_texel* d_tex, float* d_rgb,
@@ -1140,15 +1431,11 @@ extern "C" VPT_API int vpt_unet_denoise(vpt_unet* u, const vpt_gbuffer* gb, cons
 {
     if (!u || !gb || !d_rgb) return set_error(VPT_EINVAL, "vpt_unet_denoise: null argument");
     if (int rc = check_dims(u, 1, gb->height, gb->width, "vpt_unet_denoise")) return rc;
-    if (int rc = vpt_unet_assemble(u, gb, d_tex, u->act[X], stream)) return rc;
+    if (int rc = assemble("vpt_unet_denoise", u, gb, d_tex, u->act[X], true, stream)) return rc;
     DeviceGuard g(u->device);
-    hipStream_t s = (hipStream_t)stream;
-    const size_t npx = (size_t)gb->width * gb->height;
-    if (int rc = forward(u, 1, gb->height, gb->width, s)) return rc;
-    hipLaunchKernelGGL(head_kernel, dim3(blocks_for(npx)), dim3(256), 0, s, u->act[D0B], npx, u->d_w + u->head_w,
-                       u->d_w + u->head_b, 1, d_rgb);
-    HIP_TRY(hipGetLastError());
-    return VPT_OK;
+    bool capturing = false;
+    if (int rc = is_capturing((hipStream_t)stream, &capturing)) return rc;
+    return forward(u, 1, gb->height, gb->width, true, capturing, d_rgb, true, (hipStream_t)stream);
 }
 
 extern "C" VPT_API int vpt_texel_accumulate(const vpt_svgf_texel* d_tex, int npx, float* d_acc, int reset, void* stream)
@@ -1180,6 +1467,18 @@ extern "C" VPT_API int vpt_unet_read_activation(vpt_unet* u, int index, int n, i
     DeviceGuard g(u->device);
     const size_t count = ((size_t)n * (h >> kLevel[index]) * (w >> kLevel[index])) * kChannels[index];
     HIP_TRY(hipDeviceSynchronize());
-    HIP_TRY(hipMemcpy(host, u->act[index], sizeof(uint16_t) * count, hipMemcpyDeviceToHost));
+    if (index == D0B) {
+        if (int rc = make_last(u, n, h, w, nullptr)) return rc;
+        HIP_TRY(hipDeviceSynchronize());
+    }
+    int half = 0;   // 16 of the input's 32 channels are stored, the others are zero
+    if (index == X) HIP_TRY(hipMemcpy(&half, u->d_x16, sizeof(int), hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(host, u->act[index], sizeof(uint16_t) * (half ? count / 2 : count), hipMemcpyDeviceToHost));
+    if (half) {
+        for (size_t i = count / 32; i-- > 0;) {
+            memmove(host + i * 32, host + i * 16, 16 * sizeof(uint16_t));
+            memset(host + i * 32 + 16, 0, 16 * sizeof(uint16_t));
+        }
+    }
     return VPT_OK;
 }
