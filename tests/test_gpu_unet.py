@@ -117,6 +117,32 @@ def test_gradients_match_cpu(net):
         assert _rel(a, b) < 0.06 and cos > 0.998, (name, _rel(a, b), cos)
 
 
+@pytest.mark.parametrize("n,h,w", [(1, 4, 4), (2, 12, 36), (3, 20, 100), (1, 60, 68), (5, 64, 64)])
+def test_gradients_at_tile_edges(net, n, h, w):
+    """Weight gradients where the 4 x 32 pixel tiles, their groups over the
+    four waves and the slices have remainders.  The target lies above every
+    prediction, so that no sign of the L1 loss hangs on a rounding; bf16
+    gradients as in test_gradients_match_cpu, same tolerance."""
+    torch = _torch()
+    rng = np.random.default_rng(31)
+    xb, xf = _inputs(rng, n, h, w)
+    target = rng.normal(40.0, 0.5, size=(n, h, w, 3)).astype(np.float32)
+    net.init(22)
+    params = net.get_params()
+    print(f"unet backward {n}x{h}x{w}", flush=True)
+    loss = net.backward(torch.from_numpy(xb.view(np.int16)).cuda(), torch.from_numpy(target).cuda(), n, h, w)
+    g = net.get_grads()
+    ref_loss, ref_g = unet_ref.loss_and_grads(params, xf, target)
+    assert abs(loss - ref_loss) <= 1e-3 * abs(ref_loss)
+    from voxelpathtracer_amd.unet import param_layout
+    for name, off, shape in param_layout()[0]:
+        size = int(np.prod(shape))
+        assert _rel(g[off:off + size], ref_g[off:off + size]) < 0.06, name
+    again = net.backward(torch.from_numpy(xb.view(np.int16)).cuda(), torch.from_numpy(target).cuda(), n, h, w)
+    assert again == loss
+    np.testing.assert_array_equal(net.get_grads(), g)   # a fixed order of sums
+
+
 def _bf16_tensor(a):
     torch = _torch()
     return torch.from_numpy(bf16_to_f32(a.cpu().numpy().view(np.uint16))).cuda()

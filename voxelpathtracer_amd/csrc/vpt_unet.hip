@@ -24,7 +24,7 @@
 // epilogue.  vpt_unet_denoise's input has 16 stored channels (10 are used).
 // The backward pass reuses the forward kernel with flipped, transposed
 // weights (data gradient, ReLU mask in the epilogue) and an MFMA kernel for
-// the weight gradient (K = pixels, LDS-transposed tiles, per-slice partials
+// the weight gradient (K = pixels, transposing LDS reads, per-slice partials
 // reduced in a fixed order, so gradients are deterministic).  Adam updates
 // the fp32 master weights and refreshes the bf16 copies.
 #include <hip/hip_runtime.h>
@@ -84,7 +84,6 @@ __device__ inline uint32_t mask_pair(uint32_t v, uint32_t m)
 }
 
 constexpr int kCi = 32;            // input channels per K slice
-constexpr int kRow = 40;           // LDS row pitch in halves (32 + 8: conflict-free 16-byte reads)
 
 struct ConvArgs {
     const uint16_t* a;   // input A, NHWC with ca channels (half resolution when a_up)
@@ -105,24 +104,6 @@ struct ConvArgs {
     int n, h, w_, cout;
     int near;            // 32-bit byte offsets reach over a tile's halo
 };
-
-// Loads 8 channels (16 bytes) of the conv input at (img, gy, gx), channel
-// c0 of the concatenated input; zero outside the image.
-__device__ inline uint4 load_in8(const ConvArgs& p, int img, int gy, int gx, int c0)
-{
-    if (gy < 0 || gx < 0 || gy >= p.h || gx >= p.w_) return make_uint4(0u, 0u, 0u, 0u);
-    if (c0 < p.ca) {
-        if (p.a_up) {
-            const int hh = p.h >> 1, ww = p.w_ >> 1;
-            const size_t off = (((size_t)img * hh + (gy >> 1)) * ww + (gx >> 1)) * p.ca + c0;
-            return *reinterpret_cast<const uint4*>(p.a + off);
-        }
-        const size_t off = (((size_t)img * p.h + gy) * p.w_ + gx) * p.ca + c0;
-        return *reinterpret_cast<const uint4*>(p.a + off);
-    }
-    const size_t off = (((size_t)img * p.h + gy) * p.w_ + gx) * p.cb + (c0 - p.ca);
-    return *reinterpret_cast<const uint4*>(p.b + off);
-}
 
 typedef __attribute__((address_space(1))) const void GlobalPtr;
 typedef __attribute__((address_space(3))) void LdsPtr;
@@ -536,122 +517,257 @@ __global__ void __launch_bounds__(64 * WR * WC) conv3x3_kernel(ConvArgs p)
     }
 }
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 LdsS16x4;
+
 // Weight gradient of a 3x3 convolution:
 //   dW[tap][co][ci] = sum_px m[px][co] * X[px + off(tap)][ci],  db[co] = sum_px m[px][co]
-// as MFMA products with K = 32 pixels of one output row.  Grid: x = pixel
-// slices, y = COUT_T output-channel blocks, z = 32 input-channel blocks.
-// Each workgroup reduces its slices' row segments and writes a partial
-// [9][COUT_T][32] block (and the bias partial) for the fixed-order reduction.
-template <int COUT_T>
+// as MFMA products with K = 32 pixels of one output row.  A wave owns 32
+// output x 32 input channels of all nine taps (144 accumulators); the four
+// waves of a workgroup are CO x CI of them over the same pixels, times KS =
+// 4 / (CO * CI) over different pixel tiles.  A tile is 4 rows x 32 columns of
+// m with the 6 x 34 pixels of X around it, loaded into LDS as they lie in
+// memory (a row of 64 bytes per pixel and 32 channels); ds_read_b64_tr_b16
+// then gives a lane 4 pixels of its channel, so neither tile is transposed
+// on the way and a dx shift is another first row.  A pixel fragment of X is
+// used for the three output rows around it.  Grid: x = slices of the tiles,
+// y, z = output and input channel blocks.  Each workgroup writes a partial
+// [9][32 CO][32 CI] block (and the bias partial), its KS waves added in a
+// fixed order, for the fixed-order reduction over slices.
+// Measured at 16 x 128 x 128: all ten layers 530 -> 207 us against a kernel
+// that wrote transposed, shifted copies to LDS two bytes at a time.  Bound by
+// latency: a workgroup has about two tiles, one wave per SIMD (held to 256
+// registers for a second workgroup per CU the 64 x 64 blocks spilled and took
+// twice as long).
+constexpr int kWgRows = 4, kWgPitch = 36, kWgXRows = (kWgRows + 2) * kWgPitch;
+constexpr int kWgM = kWgRows * 32 * 64, kWgX = (kWgXRows * 64 + 1023) / 1024 * 1024;   // bytes per 32 channels
+
+// Place of the 16-byte piece q of row `row`: the halves swap every 8 rows,
+// so that the 8-row groups that a transposing read touches lie in different
+// banks.
+__device__ inline int wg_place(int q, int row) { return q ^ ((row >> 2) & 2); }
+
+// 8 pixels (rows row0 + 8 (lane / 16) ...) of channel c0 + lane % 16 of LDS
+// rows of 32 channels.
+__device__ inline bf16x8 wg_frag(const uint8_t* s, int row0, int c0)
+{
+    const int lane = (int)threadIdx.x & 63, i = lane & 15, row = row0 + (lane >> 4) * 8 + (i >> 2);
+    const int piece = (c0 >> 3) + ((i >> 1) & 1);
+    union {
+        s16x4 h[2];
+        bf16x8 v;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (LdsS16x4*)(s + row * 64 + wg_place(piece, row) * 16 + (i & 1) * 8));
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (LdsS16x4*)(s + (row + 4) * 64 + wg_place(piece, row + 4) * 16 + (i & 1) * 8));
+    return u.v;
+}
+
+template <int CO, int CI>
 __global__ void __launch_bounds__(256) wgrad_kernel(ConvArgs p, const uint16_t* __restrict__ m, int cin,
                                                     float* __restrict__ part, float* __restrict__ part_b)
 {
-    constexpr int SUB = (COUT_T / 16) * 2;      // 16x16 subtiles of the COUT_T x 32 block
-    constexpr int PER_WAVE = SUB / 4;
-    __shared__ __attribute__((aligned(16))) uint16_t sM[COUT_T * kRow];
-    __shared__ __attribute__((aligned(16))) uint16_t sX[9 * kCi * kRow];   // [dx][dy][ci][px]
-    __shared__ float sBias[COUT_T];
+    constexpr int KS = 4 / (CO * CI);
+    constexpr int STAGE = CO * kWgM + CI * kWgX;                   // one tile
+    constexpr int ACC = 9 * 32 * 32 * 4;                           // one wave's sums
+    constexpr int BYTES = KS * STAGE > 2 * ACC || KS == 1 ? KS * STAGE : 2 * ACC;
+    constexpr int LOADS = STAGE / 1024, PER = (LOADS + CO * CI - 1) / (CO * CI);
+    __shared__ __attribute__((aligned(16))) uint8_t smem[BYTES];
+    const int lane = (int)threadIdx.x & 63, lm = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int ks = wave / (CO * CI), sub = wave % (CO * CI), wco = sub / CI, wci = sub % CI;
+    const int co0 = ((int)blockIdx.y * CO) * 32, ci0 = ((int)blockIdx.z * CI) * 32;
+    const int tiles_x = (p.w_ + 31) / 32, tiles_y = (p.h + kWgRows - 1) / kWgRows;
+    const int total = p.n * tiles_x * tiles_y, groups = (total + KS - 1) / KS;
+    uint8_t* stage = smem + ks * STAGE;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lm = lane & 15, lk = (lane >> 4) * 8;
-    const int co0 = blockIdx.y * COUT_T, ci0 = blockIdx.z * kCi;
-    const int segs_x = (p.w_ + 31) / 32;
-    const long total = (long)p.n * p.h * segs_x;
+    f32x4 acc[9][2][2], accb[2];   // [tap][ci half][co half]
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[t][i >> 1][i & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    accb[0] = accb[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; i++) ones[i] = (__bf16)1.0f;
 
-    f32x4 acc[PER_WAVE][9];
+    for (int gr = (int)blockIdx.x; gr < groups; gr += (int)gridDim.x) {
+        const int tile = gr * KS + ks;
+        const int img = tile / (tiles_x * tiles_y), rem = tile % (tiles_x * tiles_y);
+        const int y0 = rem / tiles_x * kWgRows, x0 = rem % tiles_x * 32;
+        __syncthreads();   // the tile before has been read
+        if (tile < total) {
 #pragma unroll
-    for (int s = 0; s < PER_WAVE; s++)
-#pragma unroll
-        for (int t = 0; t < 9; t++) acc[s][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float bsum = 0.0f;
-
-    for (long sg = blockIdx.x; sg < total; sg += gridDim.x) {
-        const int img = (int)(sg / ((long)p.h * segs_x));
-        const int rem = (int)(sg % ((long)p.h * segs_x));
-        const int y = rem / segs_x, x0 = (rem % segs_x) * 32;
-        __syncthreads();
-        // m tile, transposed: sM[co][px]
-        for (int e = tid; e < 32 * (COUT_T / 8); e += 256) {
-            const int px = e / (COUT_T / 8), q = e % (COUT_T / 8);
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (x0 + px < p.w_)
-                v = *reinterpret_cast<const uint4*>(m + (((size_t)img * p.h + y) * p.w_ + x0 + px) * p.cout + co0 +
-                                                    q * 8);
-            const uint16_t* h = reinterpret_cast<const uint16_t*>(&v);
-#pragma unroll
-            for (int k = 0; k < 8; k++) sM[(q * 8 + k) * kRow + px] = h[k];
+            for (int k = 0; k < PER; k++) {
+                const int i = sub + k * CO * CI;   // 1 KiB of the stage
+                if (i >= LOADS) continue;
+                const uint16_t* at = nullptr;
+                if (i < CO * (kWgM / 1024)) {
+                    const int piece = i % (kWgM / 1024) * 64 + lane, row = piece >> 2;
+                    const int c = co0 + i / (kWgM / 1024) * 32 + wg_place(piece & 3, row) * 8;
+                    const int y = y0 + (row >> 5), x = x0 + (row & 31);
+                    if (y < p.h && x < p.w_) at = m + (((size_t)img * p.h + y) * p.w_ + x) * p.cout + c;
+                } else {
+                    const int j = i - CO * (kWgM / 1024), piece = j % (kWgX / 1024) * 64 + lane, row = piece >> 2;
+                    int c = ci0 + j / (kWgX / 1024) * 32 + wg_place(piece & 3, row) * 8;
+                    const int y = y0 + row / kWgPitch - 1, x = x0 + row % kWgPitch - 1;
+                    if ((uint32_t)y < (uint32_t)p.h && (uint32_t)x < (uint32_t)p.w_ && row < kWgXRows) {
+                        const bool in_a = c < p.ca;
+                        const int up = in_a ? p.a_up : 0, ch = in_a ? p.ca : p.cb;
+                        if (!in_a) c -= p.ca;
+                        at = (in_a ? p.a : p.b) +
+                             (((size_t)img * (p.h >> up) + (y >> up)) * (p.w_ >> up) + (x >> up)) * ch + c;
+                    }
+                }
+                __builtin_amdgcn_global_load_lds((GlobalPtr*)(at ? at : p.zero), (LdsPtr*)(stage + i * 1024), 16, 0,
+                                                 0);
+            }
         }
-        // input rows y-1..y+1, pixels x0-1..x0+32, channels ci0..ci0+31,
-        // written as three shifted, transposed copies sX[dx][dy][ci][px]
-        for (int e = tid; e < 3 * 34 * 4; e += 256) {
-            const int q = e & 3, pos = e >> 2;
-            const int dy = pos / 34, xx = pos % 34;   // xx = pixel x0 - 1 + xx
-            const uint4 v = load_in8(p, img, y + dy - 1, x0 - 1 + xx, ci0 + q * 8);
-            const uint16_t* h = reinterpret_cast<const uint16_t*>(&v);
+        wait_and_sync();
+        if (tile >= total) continue;
+        const uint8_t* sm = stage + wco * kWgM;
+        const uint8_t* sx = stage + CO * kWgM + wci * kWgX;
+        bf16x8 mf[kWgRows][2];
+#pragma unroll
+        for (int r = 0; r < kWgRows; r++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) mf[r][h] = wg_frag(sm, r * 32, h * 16);
+#pragma unroll
+        for (int hy = 0; hy < kWgRows + 2; hy++) {
 #pragma unroll
             for (int dx = 0; dx < 3; dx++) {
-                const int px = xx - dx;   // X[x0 + px + dx - 1] = loaded pixel
-                if (px < 0 || px >= 32) continue;
+                bf16x8 xf[2];
 #pragma unroll
-                for (int k = 0; k < 8; k++) sX[((dx * 3 + dy) * kCi + q * 8 + k) * kRow + px] = h[k];
+                for (int h = 0; h < 2; h++) xf[h] = wg_frag(sx, hy * kWgPitch + dx, h * 16);
+#pragma unroll
+                for (int dy = 0; dy < 3; dy++) {
+                    const int r = hy - dy;
+                    if (r < 0 || r >= kWgRows) continue;
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        acc[dy * 3 + dx][i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            xf[i >> 1], mf[r][i & 1], acc[dy * 3 + dx][i >> 1][i & 1], 0, 0, 0);
+                }
             }
+            if (hy < kWgRows && wci == 0) {
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    accb[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, mf[hy][h], accb[h], 0, 0, 0);
+            }
+        }
+    }
+    // the KS waves of a channel block: ks + KS / 2 into ks, then 1 into 0
+    float4* const red = reinterpret_cast<float4*>(smem);
+    float* const redb = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int half = KS / 2; half >= 1; half >>= 1) {
+        __syncthreads();
+        const int at = ((ks % half) * CO * CI + sub) * 36 * 64 + lane;
+        static_assert(KS == 1 || (KS / 2) * CO * CI * 36 * 64 * 16 <= BYTES, "the sums fit in the stage's LDS");
+        if (ks >= half && ks < 2 * half) {
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) red[at + (t * 4 + i) * 64] = *reinterpret_cast<float4*>(&acc[t][i >> 1][i & 1]);
         }
         __syncthreads();
-        if (blockIdx.z == 0 && tid < COUT_T) {
-            float s = 0.0f;
-            for (int px = 0; px < 32; px++) s += bf2f(sM[tid * kRow + px]);
-            bsum += s;
+        if (ks < half) {
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float4 v = red[at + (t * 4 + i) * 64];
+                    acc[t][i >> 1][i & 1] += f32x4{v.x, v.y, v.z, v.w};
+                }
         }
+        __syncthreads();
+        if (ks >= half && ks < 2 * half && wci == 0)
 #pragma unroll
-        for (int s = 0; s < PER_WAVE; s++) {
-            const int sub = wave * PER_WAVE + s;
-            const int cs = sub >> 1, ks = sub & 1;
-            const bf16x8 afr = *reinterpret_cast<const bf16x8*>(&sM[(cs * 16 + lm) * kRow + lk]);
+            for (int h = 0; h < 2; h++) redb[(((ks % half) * CO + wco) * 2 + h) * 64 + lane] = accb[h][0];
+        __syncthreads();
+        if (ks < half && wci == 0)
 #pragma unroll
-            for (int t = 0; t < 9; t++) {
-                const int dy = t / 3, dx = t % 3;
-                const bf16x8 bfr = *reinterpret_cast<const bf16x8*>(&sX[((dx * 3 + dy) * kCi + ks * 16 + lm) * kRow + lk]);
-                acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr, bfr, acc[s][t], 0, 0, 0);
-            }
+            for (int h = 0; h < 2; h++) accb[h][0] += redb[(((ks % half) * CO + wco) * 2 + h) * 64 + lane];
+    }
+    if (ks != 0) return;
+    // products give D[ci][co]: a lane holds 4 consecutive input channels
+    float* dst = part + (size_t)blockIdx.x * 9 * p.cout * cin;
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int co = co0 + wco * 32 + (i & 1) * 16 + lm, ci = ci0 + wci * 32 + (i >> 1) * 16 + g * 4;
+            *reinterpret_cast<float4*>(dst + ((size_t)t * p.cout + co) * cin + ci) =
+                *reinterpret_cast<float4*>(&acc[t][i >> 1][i & 1]);
         }
-    }
-    // partial block: part[slice][tap][co][ci] over this block's (co, ci) range
-    const int cout_total = p.cout;
-    float* dst = part + (size_t)blockIdx.x * 9 * cout_total * cin;
+    if (blockIdx.z == 0 && wci == 0 && g == 0)
 #pragma unroll
-    for (int s = 0; s < PER_WAVE; s++) {
-        const int sub = wave * PER_WAVE + s;
-        const int cs = sub >> 1, ks = sub & 1;
-#pragma unroll
-        for (int t = 0; t < 9; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int co = co0 + cs * 16 + (lane >> 4) * 4 + i, ci = ci0 + ks * 16 + lm;
-                dst[((size_t)t * cout_total + co) * cin + ci] = acc[s][t][i];
-            }
-    }
-    if (blockIdx.z == 0 && tid < COUT_T) part_b[(size_t)blockIdx.x * cout_total + co0 + tid] = bsum;
+        for (int h = 0; h < 2; h++)
+            part_b[(size_t)blockIdx.x * p.cout + co0 + wco * 32 + h * 16 + lm] = accb[h][0];
 }
 
-// out[i] = sum_z part[z][i] (z ascending), for n values.
-__global__ void reduce_parts_kernel(const float* __restrict__ part, int slices, size_t n, float* __restrict__ out)
+// out[i] = sum over z of part[z][i], for n values (a multiple of 4), and the
+// same for a second array in the same launch (its blocks come after the
+// first's).  32 groups of a block take every 32nd slice and are added in
+// order, so the sum does not depend on the launch.  Reads of one value's
+// slices in turn (one thread each) had taken 60 us for the 9.4 MB of a 32 ->
+// 32 layer and 235 us for the head's 1,024 partials; now 5 and 7 us.
+__global__ void __launch_bounds__(1024) reduce_parts_kernel(const float* __restrict__ part, int slices, int n,
+                                                            float* __restrict__ out, const float* __restrict__ part2,
+                                                            int n2, float* __restrict__ out2)
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.0f;
-    for (int z = 0; z < slices; z++) s += part[(size_t)z * n + i];
-    out[i] = s;
+    __shared__ float4 red[32][33];
+    const int blocks1 = (n / 4 + 31) / 32;
+    const bool second = (int)blockIdx.x >= blocks1;
+    const float* src = second ? part2 : part;
+    float* dst = second ? out2 : out;
+    const int len = second ? n2 : n;
+    const int x = (int)threadIdx.x & 31, y = (int)threadIdx.x >> 5;
+    const int i = (((int)blockIdx.x - (second ? blocks1 : 0)) * 32 + x) * 4;
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (i < len) {
+#pragma unroll 8
+        for (int z = y; z < slices; z += 32) {
+            const float4 v = *reinterpret_cast<const float4*>(src + (size_t)z * len + i);
+            s.x += v.x;
+            s.y += v.y;
+            s.z += v.z;
+            s.w += v.w;
+        }
+    }
+    red[y][x] = s;
+    __syncthreads();
+    if (y == 0 && i < len) {
+        for (int k = 1; k < 32; k++) {
+            const float4 v = red[k][x];
+            s.x += v.x;
+            s.y += v.y;
+            s.z += v.z;
+            s.w += v.w;
+        }
+        // d_g's layers start at multiples of 4 bytes only
+        dst[i] = s.x;
+        dst[i + 1] = s.y;
+        dst[i + 2] = s.z;
+        dst[i + 3] = s.w;
+    }
 }
 
-// wt[tap][ci][co] = w[8 - tap][co][ci]: the data gradient of a convolution
-// is the convolution of the output gradient with these weights.
-__global__ void flip_transpose_kernel(const uint16_t* __restrict__ w, int cout, int cin, uint16_t* __restrict__ wt)
+// wt[tap][ci][co] = w[8 - tap][co][ci] of every layer (at the layer's own
+// offset): the data gradient of a convolution is the convolution of the
+// output gradient with these weights.
+struct FlipLayers {
+    uint32_t off[10], cout[10], cin[10];
+};
+__global__ void flip_transpose_kernel(const uint16_t* __restrict__ w, const FlipLayers layers,
+                                      uint16_t* __restrict__ wt)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 9 * cout * cin) return;
-    const int tap = i / (cout * cin), rem = i % (cout * cin);
-    const int co = rem / cin, ci = rem % cin;
-    wt[((size_t)(8 - tap) * cin + ci) * cout + co] = w[i];
+    const uint32_t l = blockIdx.y, cout = layers.cout[l], cin = layers.cin[l];
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 9u * cout * cin) return;
+    const uint32_t tap = i / (cout * cin), rem = i % (cout * cin), ci = rem / cout, co = rem % cout;
+    wt[layers.off[l] + i] = w[layers.off[l] + ((8u - tap) * cout + co) * cin + ci];
 }
 
 // Loss and head gradient, one thread per pixel; 256-thread blocks write
@@ -663,9 +779,8 @@ __global__ void __launch_bounds__(256) head_bwd_kernel(const uint16_t* __restric
                                                        const float* __restrict__ target, uint16_t* __restrict__ m,
                                                        float* __restrict__ part)
 {
-    __shared__ float red[100][8];
+    __shared__ float sv[256][33], sg[4][256], red[2][96], red4[4][16];
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float g[3] = {0.0f, 0.0f, 0.0f}, loss = 0.0f;
     float v[32];
     const float inv = 1.0f / (3.0f * (float)npx);
@@ -697,52 +812,95 @@ __global__ void __launch_bounds__(256) head_bwd_kernel(const uint16_t* __restric
 #pragma unroll
         for (int c = 0; c < 32; c++) v[c] = 0.0f;
     }
-    // block reduction of the 100 sums: wave shuffles, then 4 waves in LDS
-    for (int k = 0; k < 100; k++) {
-        float s;
-        if (k < 96) s = g[k / 32] * v[k % 32];
-        else if (k < 99) s = g[k - 96];
-        else s = loss;
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-        if (lane == 0) red[k][wave] = s;
+    // the block's 96 weight sums, two threads each (128 pixels), from LDS;
+    // the other 64 threads take the three bias sums and the loss (16 pixels
+    // each, then in order).  Wave shuffles of all 100 sums took 41 us at 16 x
+    // 128 x 128, this 15.
+#pragma unroll
+    for (int c = 0; c < 32; c++) sv[threadIdx.x][c] = v[c];
+#pragma unroll
+    for (int j = 0; j < 3; j++) sg[j][threadIdx.x] = g[j];
+    sg[3][threadIdx.x] = loss;
+    __syncthreads();
+    const int k = (int)threadIdx.x;
+    if (k < 192) {
+        const int c = k & 31, j = (k >> 5) % 3, h = k / 96;
+        float s = 0.0f;
+#pragma unroll 8
+        for (int q = 0; q < 128; q++) s += sg[j][h * 128 + q] * sv[h * 128 + q][c];
+        red[h][j * 32 + c] = s;
+    } else {
+        const int j = (k - 192) >> 4, q0 = (k & 15) * 16;
+        float s = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 16; q++) s += sg[j][q0 + q];
+        red4[j][k & 15] = s;
     }
     __syncthreads();
-    if (threadIdx.x < 100) {
-        const int k = threadIdx.x;
-        part[(size_t)blockIdx.x * 100 + k] = (red[k][0] + red[k][1]) + (red[k][2] + red[k][3]);
+    if (k < 96) part[(size_t)blockIdx.x * 100 + k] = red[0][k] + red[1][k];
+    if (k >= 96 && k < 100) {
+        float s = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 16; q++) s += red4[k - 96][q];
+        part[(size_t)blockIdx.x * 100 + k] = s;
     }
 }
 
-// Upsample branch of a concatenated-input gradient:
-//   out[n][y][x][c] = (sum of g[n][2y+i][2x+j][c_off + c]) where y_low > 0
-__global__ void sum2x2_mask_kernel(const uint16_t* __restrict__ g, int cg, int c_off, int c, int n, int h, int w,
-                                   const uint16_t* __restrict__ ylow, uint16_t* __restrict__ out)
+// Eight bf16 values as floats, and back (rounded), kept where the matching
+// value of y is > 0.
+__device__ inline void unpack8(const uint4& q, float v[8])
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;   // low-res element
-    const int hh = h >> 1, ww = w >> 1;
-    if (i >= (size_t)n * hh * ww * c) return;
-    const int ch = (int)(i % c);
-    const size_t px = i / c;
-    const int x = (int)(px % ww), y = (int)((px / ww) % hh), img = (int)(px / ((size_t)ww * hh));
-    auto at = [&](int yy, int xx) { return bf2f(g[(((size_t)img * h + yy) * w + xx) * cg + c_off + ch]); };
-    const float s = (at(2 * y, 2 * x) + at(2 * y, 2 * x + 1)) + (at(2 * y + 1, 2 * x) + at(2 * y + 1, 2 * x + 1));
-    out[i] = bf_pos(ylow[i]) ? f2bf(s) : (uint16_t)0;
+    const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = __uint_as_float(i & 1 ? u[i >> 1] & 0xffff0000u : u[i >> 1] << 16);
 }
 
-// Skip branch: out = g[..][c_off + c] (+ 0.25 gpool[n][y/2][x/2][c] when
-// gpool is given), kept where y_skip > 0 (when y_skip is given).
+__device__ inline uint4 pack8_where(const float v[8], const uint4& y)
+{
+    return make_uint4(mask_pair(pack_bf(v[0], v[1]), y.x), mask_pair(pack_bf(v[2], v[3]), y.y),
+                      mask_pair(pack_bf(v[4], v[5]), y.z), mask_pair(pack_bf(v[6], v[7]), y.w));
+}
+
+// Upsample branch of a concatenated-input gradient, 8 channels a thread:
+//   out[n][y][x][c] = (sum of g[n][2y+i][2x+j][c]) where y_low > 0
+// for the first c of g's cg channels.
+__global__ void sum2x2_mask_kernel(const uint16_t* __restrict__ g, int cg, int c, int n, int h, int w,
+                                   const uint16_t* __restrict__ ylow, uint16_t* __restrict__ out)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int hh = h >> 1, ww = w >> 1, c8 = c >> 3;
+    if (i >= (size_t)n * hh * ww * c8) return;
+    const size_t px = i / c8;
+    const int ch = (int)(i % c8) * 8, x = (int)(px % ww);
+    const size_t row = px / ww;   // img * hh + y; the full-resolution row is 2 * row
+    const uint16_t* at = g + ((2 * row * w) + 2 * x) * cg + ch;
+    float v[4][8], s[8];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        unpack8(*reinterpret_cast<const uint4*>(at + ((size_t)(k >> 1) * w + (k & 1)) * cg), v[k]);
+#pragma unroll
+    for (int k = 0; k < 8; k++) s[k] = (v[0][k] + v[1][k]) + (v[2][k] + v[3][k]);
+    *reinterpret_cast<uint4*>(out + i * 8) = pack8_where(s, *reinterpret_cast<const uint4*>(ylow + i * 8));
+}
+
+// Skip branch, 8 channels a thread: out = g[..][c_off + c] + 0.25
+// gpool[n][y/2][x/2][c], kept where y_skip > 0.
 __global__ void skip_mask_kernel(const uint16_t* __restrict__ g, int cg, int c_off, int c, int n, int h, int w,
                                  const uint16_t* __restrict__ gpool, const uint16_t* __restrict__ yskip,
                                  uint16_t* __restrict__ out)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)n * h * w * c) return;
-    const int ch = (int)(i % c);
-    const size_t px = i / c;
-    const int x = (int)(px % w), y = (int)((px / w) % h), img = (int)(px / ((size_t)w * h));
-    float s = bf2f(g[px * cg + c_off + ch]);
-    if (gpool) s += 0.25f * bf2f(gpool[(((size_t)img * (h >> 1) + (y >> 1)) * (w >> 1) + (x >> 1)) * c + ch]);
-    out[i] = (!yskip || bf_pos(yskip[i])) ? f2bf(s) : (uint16_t)0;
+    const int c8 = c >> 3;
+    if (i >= (size_t)n * h * w * c8) return;
+    const size_t px = i / c8;
+    const int ch = (int)(i % c8) * 8, x = (int)(px % w);
+    const size_t row = px / w;   // img * h + y; h is even, so its half is the pooled row
+    float s[8], q[8];
+    unpack8(*reinterpret_cast<const uint4*>(g + px * cg + c_off + ch), s);
+    unpack8(*reinterpret_cast<const uint4*>(gpool + ((row >> 1) * (w >> 1) + (x >> 1)) * c + ch), q);
+#pragma unroll
+    for (int k = 0; k < 8; k++) s[k] += 0.25f * q[k];
+    *reinterpret_cast<uint4*>(out + i * 8) = pack8_where(s, *reinterpret_cast<const uint4*>(yskip + i * 8));
 }
 
 // Adam on the fp32 master parameters; refreshes the bf16 copies.
@@ -946,10 +1104,10 @@ struct vpt_unet {
     float* d_g = nullptr;        // gradients
     float* d_m1 = nullptr;
     float* d_m2 = nullptr;
-    uint16_t* d_wt = nullptr;    // flipped / transposed weights of one layer
+    uint16_t* d_wt = nullptr;    // flipped / transposed weights of every layer
     uint16_t* act[NBUF] = {};    // activations
     uint16_t* grad[NBUF] = {};   // masked gradients (pre-activation) of each buffer
-    uint16_t* d_gcat = nullptr;  // data gradient of a concatenated input
+    uint16_t* d_gcat[2] = {};    // data gradients of the concatenated inputs (of D0A, D1A)
     uint16_t* d_gpool[2] = {};   // gradients of P0, P1
     float* d_pred = nullptr;
     uint16_t* d_zero = nullptr;  // zeros, read for pixels outside the image
@@ -1043,25 +1201,26 @@ int is_capturing(hipStream_t s, bool* out)
     return VPT_OK;
 }
 
+// Weight gradient of a layer.  Channel blocks of 64 x 64, 64 x 32 or 32 x
+// 32; one workgroup per CU in all (more slices would move more partial sums,
+// fewer leave CUs idle), at most one per group of pixel tiles.
 int wgrad(vpt_unet* u, const Layer& L, int n, int h, int w, const uint16_t* m, hipStream_t s)
 {
-    ConvArgs a = conv_args(u, L, n, h, w);
-    const int cin = L.cin;
-    const size_t wsz = (size_t)9 * L.cout * cin;
-    const int slices = u->slices;
-    if (L.cout % 64 == 0) {
-        hipLaunchKernelGGL(wgrad_kernel<64>, dim3((unsigned)slices, (unsigned)(L.cout / 64), (unsigned)(cin / 32)),
-                           dim3(256), 0, s, a, m, cin, u->d_part, u->d_part + (size_t)slices * wsz);
-    } else {
-        hipLaunchKernelGGL(wgrad_kernel<32>, dim3((unsigned)slices, (unsigned)(L.cout / 32), (unsigned)(cin / 32)),
-                           dim3(256), 0, s, a, m, cin, u->d_part, u->d_part + (size_t)slices * wsz);
-    }
+    const ConvArgs a = conv_args(u, L, n, h, w);
+    const int wsz = 9 * L.cout * L.cin;
+    const int co = L.cout % 64 == 0 ? 2 : 1, ci = co == 2 && L.cin % 64 == 0 ? 2 : 1, ks = 4 / (co * ci);
+    const int by = L.cout / (32 * co), bz = L.cin / (32 * ci);
+    const long tiles = (long)a.n * ((a.h + kWgRows - 1) / kWgRows) * ((a.w_ + 31) / 32);
+    const int slices = (int)std::min<long>((tiles + ks - 1) / ks, std::min(u->slices, std::max(1, g_cus / (by * bz))));
+    float* part_b = u->d_part + (size_t)slices * wsz;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)slices, (unsigned)by, (unsigned)bz), dim3(256), 0, s, a, m, L.cin,
+                           u->d_part, part_b);
+    };
+    ci == 2 ? go(wgrad_kernel<2, 2>) : (co == 2 ? go(wgrad_kernel<2, 1>) : go(wgrad_kernel<1, 1>));
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(reduce_parts_kernel, dim3(blocks_for(wsz)), dim3(256), 0, s, u->d_part, slices, wsz,
-                       u->d_g + L.w_off);
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(reduce_parts_kernel, dim3(blocks_for(L.cout)), dim3(256), 0, s,
-                       u->d_part + (size_t)slices * wsz, slices, (size_t)L.cout, u->d_g + L.b_off);
+    hipLaunchKernelGGL(reduce_parts_kernel, dim3((unsigned)((wsz / 4 + 31) / 32 + (L.cout / 4 + 31) / 32)), dim3(1024),
+                       0, s, u->d_part, slices, wsz, u->d_g + L.w_off, part_b, L.cout, u->d_g + L.b_off);
     HIP_TRY(hipGetLastError());
     return VPT_OK;
 }
@@ -1072,15 +1231,11 @@ int wgrad(vpt_unet* u, const Layer& L, int n, int h, int w, const uint16_t* m, h
 int dgrad(vpt_unet* u, const Layer& L, int n, int h, int w, const uint16_t* m, const uint16_t* mask, uint16_t* out,
           hipStream_t s)
 {
-    const size_t wsz = (size_t)9 * L.cout * L.cin;
-    hipLaunchKernelGGL(flip_transpose_kernel, dim3(blocks_for(wsz)), dim3(256), 0, s, u->d_wb + L.w_off, L.cout, L.cin,
-                       u->d_wt);
-    HIP_TRY(hipGetLastError());
     ConvArgs a;
     memset(&a, 0, sizeof(a));
     a.a = m;
     a.ca = L.cout;
-    a.w = u->d_wt;
+    a.w = u->d_wt + L.w_off;
     a.mask = mask;
     a.y = out;
     a.zero = u->d_zero;
@@ -1094,76 +1249,73 @@ int dgrad(vpt_unet* u, const Layer& L, int n, int h, int w, const uint16_t* m, c
 int backward(vpt_unet* u, const float* d_target, int n, int h, int w, hipStream_t s)
 {
     const size_t npx = level_px(u, n, h, w, 0);
-    // head: loss, head gradients, masked gradient of D0B
+    const Layer* N = u->net;
+    {
+        FlipLayers f;
+        int most = 0;
+        for (int l = 0; l < kLayers; l++) {
+            f.off[l] = (uint32_t)N[l].w_off;
+            f.cout[l] = (uint32_t)N[l].cout;
+            f.cin[l] = (uint32_t)N[l].cin;
+            most = std::max(most, 9 * N[l].cout * N[l].cin);
+        }
+        hipLaunchKernelGGL(flip_transpose_kernel, dim3(blocks_for((size_t)most), kLayers), dim3(256), 0, s, u->d_wb, f,
+                           u->d_wt);
+        HIP_TRY(hipGetLastError());
+    }
+    // head: loss, head gradients, masked gradient of D0B; the sums are 96 dW
+    // and 3 db, which end the gradient vector, and the loss behind it
     const unsigned hb = blocks_for(npx);
     hipLaunchKernelGGL(head_bwd_kernel, dim3(hb), dim3(256), 0, s, u->act[D0B], npx, u->d_w + u->head_w, u->d_pred,
                        d_target, u->grad[D0B], u->d_head_part);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(reduce_parts_kernel, dim3(1), dim3(128), 0, s, u->d_head_part, (int)hb, (size_t)100,
-                       u->d_part);
+    hipLaunchKernelGGL(reduce_parts_kernel, dim3(1), dim3(1024), 0, s, u->d_head_part, (int)hb, 100,
+                       u->d_g + u->head_w, (const float*)nullptr, 0, (float*)nullptr);
     HIP_TRY(hipGetLastError());
-    // d_part[0..95] = dW head, [96..98] = db head, [99] = loss sum (lands in d_g[n_params])
-    HIP_TRY(hipMemcpyAsync(u->d_g + u->head_w, u->d_part, sizeof(float) * 100, hipMemcpyDeviceToDevice, s));
 
-    const Layer* N = u->net;
+    auto sum2x2 = [&](const uint16_t* g, int cg, int c, int lh, int lw, const uint16_t* ylow, uint16_t* out) -> int {
+        hipLaunchKernelGGL(sum2x2_mask_kernel, dim3(blocks_for((size_t)n * (lh >> 1) * (lw >> 1) * c / 8)), dim3(256),
+                           0, s, g, cg, c, n, lh, lw, ylow, out);
+        HIP_TRY(hipGetLastError());
+        return VPT_OK;
+    };
+    auto skip = [&](const uint16_t* g, int cg, int off, int c, int lh, int lw, const uint16_t* gpool,
+                    const uint16_t* y, uint16_t* out) -> int {
+        hipLaunchKernelGGL(skip_mask_kernel, dim3(blocks_for((size_t)n * lh * lw * c / 8)), dim3(256), 0, s, g, cg, off,
+                           c, n, lh, lw, gpool, y, out);
+        HIP_TRY(hipGetLastError());
+        return VPT_OK;
+    };
     // layer 9: D0A -> D0B
     if (int rc = wgrad(u, N[9], n, h, w, u->grad[D0B], s)) return rc;
     if (int rc = dgrad(u, N[9], n, h, w, u->grad[D0B], u->act[D0A], u->grad[D0A], s)) return rc;
-    // layer 8: cat(up(D1B), E0B) -> D0A
+    // layer 8: cat(up(D1B), E0B) -> D0A; E0B's part waits in the
+    // concatenated gradient until P0's is known
     if (int rc = wgrad(u, N[8], n, h, w, u->grad[D0A], s)) return rc;
-    if (int rc = dgrad(u, N[8], n, h, w, u->grad[D0A], nullptr, u->d_gcat, s)) return rc;
-    {
-        const size_t lo = level_px(u, n, h, w, 1) * 64;
-        hipLaunchKernelGGL(sum2x2_mask_kernel, dim3(blocks_for(lo)), dim3(256), 0, s, u->d_gcat, 96, 0, 64, n, h, w,
-                           u->act[D1B], u->grad[D1B]);
-        HIP_TRY(hipGetLastError());
-        // the E0B part waits in grad[E0B] (unmasked) until P0's gradient is known
-        const size_t sk = npx * 32;
-        hipLaunchKernelGGL(skip_mask_kernel, dim3(blocks_for(sk)), dim3(256), 0, s, u->d_gcat, 96, 64, 32, n, h, w,
-                           (const uint16_t*)nullptr, (const uint16_t*)nullptr, u->grad[E0A]);
-        HIP_TRY(hipGetLastError());
-    }
+    if (int rc = dgrad(u, N[8], n, h, w, u->grad[D0A], nullptr, u->d_gcat[0], s)) return rc;
+    if (int rc = sum2x2(u->d_gcat[0], 96, 64, h, w, u->act[D1B], u->grad[D1B])) return rc;
     // layer 7: D1A -> D1B
     if (int rc = wgrad(u, N[7], n, h, w, u->grad[D1B], s)) return rc;
     if (int rc = dgrad(u, N[7], n, h, w, u->grad[D1B], u->act[D1A], u->grad[D1A], s)) return rc;
     // layer 6: cat(up(B1), E1B) -> D1A
     if (int rc = wgrad(u, N[6], n, h, w, u->grad[D1A], s)) return rc;
-    if (int rc = dgrad(u, N[6], n, h, w, u->grad[D1A], nullptr, u->d_gcat, s)) return rc;
-    {
-        const size_t lo = level_px(u, n, h, w, 2) * 128;
-        hipLaunchKernelGGL(sum2x2_mask_kernel, dim3(blocks_for(lo)), dim3(256), 0, s, u->d_gcat, 192, 0, 128, n,
-                           h >> 1, w >> 1, u->act[B1], u->grad[B1]);
-        HIP_TRY(hipGetLastError());
-        const size_t sk = level_px(u, n, h, w, 1) * 64;
-        hipLaunchKernelGGL(skip_mask_kernel, dim3(blocks_for(sk)), dim3(256), 0, s, u->d_gcat, 192, 128, 64, n, h >> 1,
-                           w >> 1, (const uint16_t*)nullptr, (const uint16_t*)nullptr, u->grad[E1A]);
-        HIP_TRY(hipGetLastError());
-    }
+    if (int rc = dgrad(u, N[6], n, h, w, u->grad[D1A], nullptr, u->d_gcat[1], s)) return rc;
+    if (int rc = sum2x2(u->d_gcat[1], 192, 128, h >> 1, w >> 1, u->act[B1], u->grad[B1])) return rc;
     // layer 5: B0 -> B1
     if (int rc = wgrad(u, N[5], n, h, w, u->grad[B1], s)) return rc;
     if (int rc = dgrad(u, N[5], n, h, w, u->grad[B1], u->act[B0], u->grad[B0], s)) return rc;
-    // layer 4: P1 -> B0; gradient of P1 (no ReLU on a pooled buffer)
+    // layer 4: P1 -> B0; gradient of P1 (no ReLU on a pooled buffer), then
+    // E1B: skip gradient + pooled gradient, masked by E1B
     if (int rc = wgrad(u, N[4], n, h, w, u->grad[B0], s)) return rc;
     if (int rc = dgrad(u, N[4], n, h, w, u->grad[B0], nullptr, u->d_gpool[1], s)) return rc;
-    {
-        // E1B: skip gradient (held in grad[E1A]) + pooled gradient, masked by E1B
-        const size_t sk = level_px(u, n, h, w, 1) * 64;
-        hipLaunchKernelGGL(skip_mask_kernel, dim3(blocks_for(sk)), dim3(256), 0, s, u->grad[E1A], 64, 0, 64, n, h >> 1,
-                           w >> 1, u->d_gpool[1], u->act[E1B], u->grad[E1B]);
-        HIP_TRY(hipGetLastError());
-    }
+    if (int rc = skip(u->d_gcat[1], 192, 128, 64, h >> 1, w >> 1, u->d_gpool[1], u->act[E1B], u->grad[E1B])) return rc;
     // layer 3: E1A -> E1B
     if (int rc = wgrad(u, N[3], n, h, w, u->grad[E1B], s)) return rc;
     if (int rc = dgrad(u, N[3], n, h, w, u->grad[E1B], u->act[E1A], u->grad[E1A], s)) return rc;
     // layer 2: P0 -> E1A
     if (int rc = wgrad(u, N[2], n, h, w, u->grad[E1A], s)) return rc;
     if (int rc = dgrad(u, N[2], n, h, w, u->grad[E1A], nullptr, u->d_gpool[0], s)) return rc;
-    {
-        const size_t sk = npx * 32;
-        hipLaunchKernelGGL(skip_mask_kernel, dim3(blocks_for(sk)), dim3(256), 0, s, u->grad[E0A], 32, 0, 32, n, h, w,
-                           u->d_gpool[0], u->act[E0B], u->grad[E0B]);
-        HIP_TRY(hipGetLastError());
-    }
+    if (int rc = skip(u->d_gcat[0], 96, 64, 32, h, w, u->d_gpool[0], u->act[E0B], u->grad[E0B])) return rc;
     // layer 1: E0A -> E0B
     if (int rc = wgrad(u, N[1], n, h, w, u->grad[E0B], s)) return rc;
     if (int rc = dgrad(u, N[1], n, h, w, u->grad[E0B], u->act[E0A], u->grad[E0A], s)) return rc;
@@ -1224,7 +1376,8 @@ extern "C" VPT_API int vpt_unet_destroy(vpt_unet* u)
         (void)hipFree(u->act[b]);
         (void)hipFree(u->grad[b]);
     }
-    (void)hipFree(u->d_gcat);
+    (void)hipFree(u->d_gcat[0]);
+    (void)hipFree(u->d_gcat[1]);
     (void)hipFree(u->d_gpool[0]);
     (void)hipFree(u->d_gpool[1]);
     (void)hipFree(u->d_pred);
@@ -1275,13 +1428,14 @@ extern "C" VPT_API int vpt_unet_create(vpt_ctx* ctx, int max_n, int max_h, int m
     alloc((void**)&u->d_g, sizeof(float) * (u->n_params + 1));
     alloc((void**)&u->d_m1, sizeof(float) * u->n_params);
     alloc((void**)&u->d_m2, sizeof(float) * u->n_params);
-    alloc((void**)&u->d_wt, sizeof(uint16_t) * max_w_layer);
+    alloc((void**)&u->d_wt, sizeof(uint16_t) * u->n_params);
     for (int b = 0; b < NBUF; b++) {
         const size_t px = full >> (2 * kLevel[b]);
         alloc((void**)&u->act[b], sizeof(uint16_t) * px * kChannels[b]);
         if (b != X && b != P0 && b != P1) alloc((void**)&u->grad[b], sizeof(uint16_t) * px * kChannels[b]);
     }
-    alloc((void**)&u->d_gcat, sizeof(uint16_t) * full * 96);
+    alloc((void**)&u->d_gcat[0], sizeof(uint16_t) * full * 96);
+    alloc((void**)&u->d_gcat[1], sizeof(uint16_t) * (full >> 2) * 192);
     alloc((void**)&u->d_gpool[0], sizeof(uint16_t) * (full >> 2) * 32);
     alloc((void**)&u->d_gpool[1], sizeof(uint16_t) * (full >> 4) * 64);
     alloc((void**)&u->d_pred, sizeof(float) * full * 3);
