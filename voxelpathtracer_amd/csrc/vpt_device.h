@@ -340,16 +340,102 @@ __device__ __attribute__((always_inline)) inline Hit trav_finish(const WorldView
     return h;
 }
 
+__device__ __attribute__((always_inline)) inline bool trav_inside(const WorldView& w, const Trav& r)
+{
+    return __float_as_uint(r.ox) < trav_bound(w.xmax) && __float_as_uint(r.oy) < trav_bound(w.ymax) &&
+           __float_as_uint(r.oz) < trav_bound(w.zmax);
+}
+
+// The loop's turns of a ray to its end or to r.max_iter, as trav_locate and
+// trav_advance make them, in a form with one exit and selects in place of
+// most branches.  The position must be inside the volume and samples below
+// the cap on entry; returns the last DF byte (0: stopped in a solid cell).
+// Leaving the volume needs no flag: trav_finish finds the position outside.
+// kEager: the one-cell step, which does not need the DF byte, is computed
+// while that byte is on its way.  That shortens the chain from one position
+// to the next, which is what the few long rays that end a launch wait for
+// with most of the chip idle; it costs every turn both kinds of step, which
+// the short rays of a full chip would pay for.
+template <bool kEager>
+__device__ __attribute__((always_inline)) inline int trav_run(const WorldView& w, Trav& r)
+{
+    const int sx = sgn(r.dx), sy = sgn(r.dy), sz = sgn(r.dz);
+    const float hx = (float)((1 + sx) >> 1), hy = (float)((1 + sy) >> 1), hz = (float)((1 + sz) >> 1);
+    const float ex = (float)(sx + 1) - hx, ey = (float)(sy + 1) - hy, ez = (float)(sz + 1) - hz;
+    const float tx = (float)sx * 0.0001f, ty = (float)sy * 0.0001f, tz = (float)sz * 0.0001f;
+    const uint32_t bx = trav_bound(w.xmax), by = trav_bound(w.ymax), bz = trav_bound(w.zmax);
+    int m;
+    bool alive;
+    do {
+        const uint32_t cx = (uint32_t)r.ox, cy = (uint32_t)r.oy, cz = (uint32_t)r.oz;
+        m = plane_byte(w.df, brick_offset_fast(cx, cy, cz, w.row_stride, w.slab_stride));
+        float ax, ay, az;
+        int mi;
+        // the one-cell step of trav_advance
+        auto one_cell = [&]() __attribute__((always_inline)) {
+            const float gx = (float)cx, gy = (float)cy, gz = (float)cz;
+            const float wx = r.ox - gx, wy = r.oy - gy, wz = r.oz - gz;
+            const float fxx = (hx - wx) * r.ix, fyy = (hy - wy) * r.iy, fzz = (hz - wz) * r.iz;
+            const bool x_first = fxx < fyy && sx != 0;
+            const float fxy = x_first ? fxx : fyy;
+            const bool not_z = fxy < fzz || sz == 0;
+            const float fm = not_z ? fxy : fzz;
+            ax = pick(x_first && not_z, (gx + ex) + tx, gx + (wx + r.dx * fm));
+            ay = pick(!x_first && not_z, (gy + ey) + ty, gy + (wy + r.dy * fm));
+            az = pick(not_z, gz + (wz + r.dz * fm), (gz + ez) + tz);
+            mi = not_z ? (x_first ? 0 : 1) : 2;
+        };
+        if (kEager) {
+            one_cell();
+            // all of that before the byte is waited for
+            asm volatile("" : "+v"(ax), "+v"(ay), "+v"(az), "+v"(mi));
+            const bool solid = m == 0, one = m < 4;
+            const float k = df_jump(m);
+            const float nx = one ? ax : r.ox + k * r.dx, ny = one ? ay : r.oy + k * r.dy,
+                        nz = one ? az : r.oz + k * r.dz;
+            r.min_idx = one && !solid ? mi : r.min_idx;
+            r.inter = one && !solid ? 1 : r.inter;
+            r.ox = solid ? r.ox : nx;
+            r.oy = solid ? r.oy : ny;
+            r.oz = solid ? r.oz : nz;
+        } else if (m < 4) {
+            one_cell();
+            const bool solid = m == 0;
+            r.ox = pick(solid, r.ox, ax);
+            r.oy = pick(solid, r.oy, ay);
+            r.oz = pick(solid, r.oz, az);
+            r.min_idx = solid ? r.min_idx : mi;
+            r.inter = solid ? r.inter : 1;
+        } else {
+            const float k = df_jump(m);
+            r.ox = r.ox + k * r.dx;
+            r.oy = r.oy + k * r.dy;
+            r.oz = r.oz + k * r.dz;
+        }
+        r.samples++;
+        alive = m != 0 && r.samples < r.max_iter && __float_as_uint(r.ox) < bx && __float_as_uint(r.oy) < by &&
+                __float_as_uint(r.oz) < bz;
+    } while (alive);
+    return m;
+}
+
+// Steps of a ray after which traverse goes over to the eager turns: at once
+// in a launch that leaves the chip idle lanes anyway.
+constexpr int kLongRay = 24;
+constexpr uint32_t kSmallLaunch = 1024;   // workgroups
+__device__ inline int long_ray_after() { return gridDim.x <= kSmallLaunch ? 0 : kLongRay; }
+
 __device__ inline Hit traverse(const WorldView& w, Vec3 o, Vec3 d, int max_iter)
 {
     Trav r;
-    trav_init(r, o, d, max_iter);
-    uint32_t off;
-    Cell c;
-    // the cap is tested once here and then where trav_advance returns
-    if (max_iter > 0) {
-        while (trav_locate(w, r, off, c)) {
-            if (!trav_advance(r, plane_byte(w.df, off), c)) break;
+    const int after = long_ray_after();
+    trav_init(r, o, d, min(max_iter, after));
+    if (max_iter > 0 && trav_inside(w, r)) {
+        int m = 1;
+        if (after > 0) m = trav_run<false>(w, r);
+        if (m != 0 && max_iter > after && trav_inside(w, r)) {
+            r.max_iter = max_iter;
+            trav_run<true>(w, r);
         }
     }
     return trav_finish(w, r);

@@ -551,18 +551,11 @@ __global__ void __launch_bounds__(256) gi_bounce_kernel(WorldView w, CamView cam
         const Vec3 dir = vpt::mk3(s_ray[3][threadIdx.x], s_ray[4][threadIdx.x], s_ray[5][threadIdx.x]);
         vpt::Trav r;
         vpt::trav_init(r, o, dir, min(g.gi_iter, kGiPhase1));
-        bool capped = false;   // stopped by the phase's step cap, not by a hit or the volume's end
-        if (r.max_iter > 0) {
-            uint32_t off;
-            vpt::Cell c;
-            while (vpt::trav_locate(w, r, off, c)) {
-                const int m = vpt::plane_byte(w.df, off);
-                if (!vpt::trav_advance(r, m, c)) {
-                    capped = m != 0;
-                    break;
-                }
-            }
-        }
+        int m = 0;
+        if (r.max_iter > 0 && vpt::trav_inside(w, r)) m = vpt::trav_run<false>(w, r);
+        // stopped by the phase's step cap, not by a hit (nor, unless with
+        // the last step, by the volume's end)
+        const bool capped = m != 0 && r.samples == r.max_iter;
         rays = 1;
         if (capped && g.gi_iter > kGiPhase1) {
             cont = true;
@@ -607,11 +600,7 @@ __global__ void __launch_bounds__(256) gi_cont_kernel(WorldView w, CamView cam, 
         r.samples = kGiPhase1;   // < gi_iter: only such rays are continued
         r.min_idx = (int)((meta >> 28) & 3u);
         r.inter = (int)((meta >> 30) & 1u);
-        uint32_t off;
-        vpt::Cell c;
-        while (vpt::trav_locate(w, r, off, c)) {
-            if (!vpt::trav_advance(r, vpt::plane_byte(w.df, off), c)) break;
-        }
+        if (vpt::trav_inside(w, r)) vpt::trav_run<true>(w, r);
         const vpt::Hit h = vpt::trav_finish(w, r);
         samples = h.samples - kGiPhase1;   // the first kGiPhase1 were counted by the bounce kernel
         jb = gi_bounce_result(g, albedo.v, o, dir, h, pix, rgb, texels, job);
