@@ -477,6 +477,47 @@ def test_ray_queries_iteration_caps(terrain_world, max_iter):
     assert got["samples"].max() <= max_iter
 
 
+@pytest.mark.parametrize("n", [20_000, 300_000])
+@pytest.mark.parametrize("max_iter", [23, 24, 25, 48, 350])
+def test_ray_queries_long_rays(terrain_world, n, max_iter):
+    """Launches below and above 262,144 rays, where the traversal takes its
+    eager form at once or after 24 steps, with caps around that step: random
+    rays, grazing ones that walk far, axis-aligned directions, -0 and
+    on-boundary origins, and direction components near zero."""
+    g, df, w = terrain_world
+    torch = _torch()
+    rng = np.random.default_rng(57 + max_iter)
+    org = np.stack([rng.uniform(0, 384, n), rng.uniform(0, 128, n), rng.uniform(0, 384, n)], 1)
+    d = rng.normal(size=(n, 3))
+    kind = rng.integers(0, 8, n)
+    low = kind < 3
+    d[low, 1] *= 0.02
+    org[low, 1] = rng.uniform(60, 95, int(low.sum()))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    axis = np.flatnonzero(kind == 3)
+    d[axis] = 0.0
+    d[axis, rng.integers(0, 3, axis.size)] = rng.choice([-1.0, 1.0], axis.size)
+    flat = np.flatnonzero(kind == 4)
+    d[flat, rng.integers(0, 3, flat.size)] = 0.0
+    tiny = np.flatnonzero(kind == 5)
+    d[tiny, rng.integers(0, 3, tiny.size)] = rng.choice([1e-38, -1e-20, 1e-7], tiny.size)
+    edge = np.flatnonzero(kind == 6)
+    org[edge] = np.round(org[edge])
+    rays = np.concatenate([org, d], 1).astype(np.float32)
+    zero = np.flatnonzero(kind == 7)[::2]
+    rays[zero, rng.integers(0, 3, zero.size)] = -0.0
+    dev_rays = torch.from_numpy(rays.view(np.uint8).copy()).cuda()
+    hits = torch.empty(n * C.sizeof(Hit), dtype=torch.uint8, device="cuda")
+    w.trace_rays(dev_rays, hits, n, max_iter)
+    torch.cuda.synchronize()
+    dt = np.dtype([("t", "<f4"), ("voxel", "<u4"), ("face", "u1"), ("block", "u1"), ("samples", "<u2")])
+    got = hits.cpu().numpy().view(dt)
+    ref = oracle.trace_rays(g, df, rays, max_iter)
+    for k in ("t", "face", "block", "samples"):
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+    assert got["samples"].max() == max_iter if max_iter < 100 else got["samples"].max() > 60
+
+
 @pytest.mark.parametrize("dims", [(16, 8, 8), (1024, 16, 8), (16, 1024, 16), (16, 8, 1024)])
 def test_extreme_world_shapes(ctx, dims):
     """Smallest world and worlds at the 1024 limit along each axis: DF and

@@ -13,19 +13,16 @@
 
 namespace vpt {
 
-constexpr int kBrick = 8;
-constexpr int kBrickBytes = 512;
-
-// Spread the three bits of v (0..7) to positions 0, 3, 6.
-__host__ __device__ inline uint32_t spread3(uint32_t v) { return (v & 1u) | ((v & 2u) << 2) | ((v & 4u) << 4); }
+// A brick: 8 x 4 x 4 cells in one 128-byte line, x fastest, then y, then z.
+constexpr int kBrickBytes = 128;
 
 // Read-only view of a world's bricked planes, passed to kernels by value.
 struct WorldView {
     const uint8_t* grid;
     const uint8_t* df;
     int nx, ny, nz;
-    uint32_t row_stride;    // nbx * 512
-    uint32_t slab_stride;   // nbx * nby * 512
+    uint32_t row_stride;    // nbx * 128
+    uint32_t slab_stride;   // nbx * nby * 128
     float xmax, ymax, zmax; // dims - 1 as float (IsInVolume bounds)
 };
 
@@ -39,27 +36,28 @@ __device__ inline uint8_t plane_byte(const uint8_t* p, uint32_t off)
     return ((GlobalByte*)p)[off];   // address-space cast
 }
 
-// Byte offset of cell (x, y, z) in a bricked plane: the three axes
-// contribute independent terms.
+// Byte offset of cell (x, y, z) in a bricked plane, bricks bx-fastest: the
+// three axes contribute independent terms.  (x / 8) * 128 + x % 8 is x + (x /
+// 8) * 120, and the others likewise; bricks and strides fit in 24-bit
+// products.  Eight instructions in the traversal's turns, where the Morton
+// order of 512-byte bricks that this layout replaced took fifteen; a line
+// still covers 8 x 4 x 4 cells.
 __host__ __device__ inline uint32_t brick_offset(uint32_t x, uint32_t y, uint32_t z, uint32_t row_stride,
                                                  uint32_t slab_stride)
 {
-    return ((x >> 3) * kBrickBytes + spread3(x & 7u)) + ((y >> 3) * row_stride + (spread3(y & 7u) << 1)) +
-           ((z >> 3) * slab_stride + (spread3(z & 7u) << 2));
+    return (x + (x >> 3) * (kBrickBytes - 8u)) + ((y << 3) + (y >> 2) * (row_stride - 32u)) +
+           ((z << 5) + (z >> 2) * (slab_stride - 128u));
 }
 
-// brick_offset for the traversal's hot loop, same value: the Morton spread
-// of each axis's low three bits is one v_perm_b32 byte lookup in an 8-entry
-// table held in its two source operands (byte k of {hi, lo} = spread of k),
-// and the brick products are 24-bit multiplies (brick index < 2^7, strides
-// < 2^24).  Full-rate instructions only.
+// The same with 24-bit multiply-adds, for the traversal.
 __device__ inline uint32_t brick_offset_fast(uint32_t x, uint32_t y, uint32_t z, uint32_t row_stride,
                                              uint32_t slab_stride)
 {
-    const uint32_t mx = __builtin_amdgcn_perm(0x49484140u, 0x09080100u, (x & 7u) | 0x0c0c0c00u);
-    const uint32_t my = __builtin_amdgcn_perm(0x92908280u, 0x12100200u, (y & 7u) | 0x0c0c0c00u);
-    const uint32_t mz = __builtin_amdgcn_perm(0x49484140u, 0x09080100u, (z & 7u) | 0x0c0c0c00u);
-    return ((x >> 3) << 9) + mx + __umul24(y >> 3, row_stride) + my + __umul24(z >> 3, slab_stride) + (mz << 2);
+    uint32_t off = __umul24(x >> 3, kBrickBytes - 8u) + x;
+    off = __umul24(y >> 2, row_stride - 32u) + off;
+    off = (y << 3) + off;
+    off = __umul24(z >> 2, slab_stride - 128u) + off;
+    return (z << 5) + off;
 }
 
 struct Vec3 {

@@ -14,9 +14,8 @@ namespace vpt {
 
 int set_error(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 
-// A world in HBM.  Grid and DF live in 8x8x8 bricks (512 B) ordered
-// bx-fastest, with a 9-bit Morton index inside each brick, so that the
-// 128-byte line fetched for one DF sample covers an 8x4x4 block of
+// A world in HBM.  Grid and DF live in 8x4x4 bricks of 128 bytes ordered
+// bx-fastest, so that the line fetched for one DF sample covers a block of
 // neighbouring cells.
 struct World {
     int device = 0;

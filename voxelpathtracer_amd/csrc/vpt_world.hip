@@ -64,7 +64,8 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 
 // ---- layout conversion ----------------------------------------------------
 
-// Linear -> bricked copy: one thread per 16-byte group along x.
+// Linear -> bricked copy: one thread per 16-byte group along x, the rows of
+// two bricks.
 __global__ void brick_kernel(const uint8_t* __restrict__ lin, uint8_t* __restrict__ brk, int nx, int ny, int nz,
                              uint32_t row_stride, uint32_t slab_stride)
 {
@@ -76,11 +77,9 @@ __global__ void brick_kernel(const uint8_t* __restrict__ lin, uint8_t* __restric
     int y = (int)(rest % ny);
     int z = (int)(rest / ny);
     const uint4 v = *reinterpret_cast<const uint4*>(lin + (size_t)z * nx * ny + (size_t)y * nx + (size_t)gx * 16);
-    uint32_t words[4] = {v.x, v.y, v.z, v.w};
-    for (int k = 0; k < 16; k++) {
-        uint8_t b = (uint8_t)(words[k >> 2] >> ((k & 3) * 8));
-        brk[vpt::brick_offset(gx * 16 + k, y, z, row_stride, slab_stride)] = b;
-    }
+    uint8_t* o = brk + vpt::brick_offset(gx * 16, y, z, row_stride, slab_stride);
+    *reinterpret_cast<uint2*>(o) = make_uint2(v.x, v.y);
+    *reinterpret_cast<uint2*>(o + vpt::kBrickBytes) = make_uint2(v.z, v.w);
 }
 
 // Bricked -> linear copy (downloads).
@@ -94,13 +93,10 @@ __global__ void unbrick_kernel(const uint8_t* __restrict__ brk, uint8_t* __restr
     size_t rest = gid / (nx / 16);
     int y = (int)(rest % ny);
     int z = (int)(rest / ny);
-    uint32_t words[4] = {0, 0, 0, 0};
-    for (int k = 0; k < 16; k++) {
-        uint32_t b = brk[vpt::brick_offset(gx * 16 + k, y, z, row_stride, slab_stride)];
-        words[k >> 2] |= b << ((k & 3) * 8);
-    }
+    const uint8_t* o = brk + vpt::brick_offset(gx * 16, y, z, row_stride, slab_stride);
+    const uint2 a = *reinterpret_cast<const uint2*>(o), b = *reinterpret_cast<const uint2*>(o + vpt::kBrickBytes);
     *reinterpret_cast<uint4*>(lin + (size_t)z * nx * ny + (size_t)y * nx + (size_t)gx * 16) =
-        make_uint4(words[0], words[1], words[2], words[3]);
+        make_uint4(a.x, a.y, b.x, b.y);
 }
 
 __global__ void set_blocks_kernel(uint8_t* __restrict__ lin, uint8_t* __restrict__ brk, const uint32_t* __restrict__ edits,
@@ -458,8 +454,8 @@ __global__ void __launch_bounds__(kSlabThreads) __attribute__((amdgpu_waves_per_
 // backward relaxations along z (ManhattanDistanceZ.comp:151-165) of the
 // tile's 8 * TW columns, four adjacent columns per lane (one LDS dword per
 // z) and each column's z range split into 512 / (2 * TW) segments
-// (relax_segments); then the tile -- TW / 8 whole 8x8 bricks wide and one
-// brick high -- is written to the bricked DF with 16-byte stores.
+// (relax_segments); then the tile -- TW / 8 bricks wide and two high -- is
+// written to the bricked DF with 16-byte stores.
 constexpr int kZTileMax = 128 * 1024;
 constexpr int kZThreads = 512;   // threads of a 16-wide tile
 
@@ -506,25 +502,15 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) df
             relax_segments<kSeg>(col, kQ, nz / kSeg, sg, kSeg, -1, true, s_end, q, kQ);
         }
     }
-    // write whole bricks: brick (bx, bz) of this tile, 512 bytes each, one
-    // 16-byte group per lane: bytes m..m+15 of the Morton order
-    const int nbz = nz / 8;
-    for (int i = threadIdx.x; i < (TW / 8) * nbz * 32; i += NT) {
-        const int g = i & 31, brick = i >> 5;       // 32 groups of 16 bytes per brick
-        const int bxl = brick % (TW / 8), bz = brick / (TW / 8);
-        uint32_t words[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const uint32_t m = (uint32_t)(g * 16 + k);   // Morton index in the brick
-            const uint32_t lx = (m & 1u) | ((m >> 2) & 2u) | ((m >> 4) & 4u);
-            const uint32_t ly = ((m >> 1) & 1u) | ((m >> 3) & 2u) | ((m >> 5) & 4u);
-            const uint32_t lz = ((m >> 2) & 1u) | ((m >> 4) & 2u) | ((m >> 6) & 4u);
-            const uint32_t b = tile[(bz * 8 + lz) * kRow + ly * TW + bxl * 8 + lx];
-            words[k >> 2] |= b << (8 * (k & 3));
-        }
-        const size_t dst = (size_t)((x0 >> 3) + bxl) * vpt::kBrickBytes + (size_t)(y0 >> 3) * row_stride +
+    // write whole bricks, one 16-byte group (two rows of 8 cells) per lane:
+    // the TW / 8 bricks side by side in x are consecutive lines
+    for (int i = threadIdx.x; i < (TW / 8) * 2 * (nz / 4) * 8; i += NT) {
+        const int g = i & 7, bx = (i >> 3) % (TW / 8), rest = (i >> 3) / (TW / 8), by = rest & 1, bz = rest >> 1;
+        const uint8_t* src = tile + (bz * 4 + (g >> 1)) * kRow + (by * 4 + (g & 1) * 2) * TW + bx * 8;
+        const uint2 lo = *reinterpret_cast<const uint2*>(src), hi = *reinterpret_cast<const uint2*>(src + TW);
+        const size_t dst = (size_t)((x0 >> 3) + bx) * vpt::kBrickBytes + (size_t)((y0 >> 2) + by) * row_stride +
                            (size_t)bz * slab_stride + (size_t)g * 16;
-        *reinterpret_cast<uint4*>(df_brick + dst) = make_uint4(words[0], words[1], words[2], words[3]);
+        *reinterpret_cast<uint4*>(df_brick + dst) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     }
 }
 
@@ -673,8 +659,8 @@ extern "C" VPT_API int vpt_world_create(vpt_ctx* ctx, int nx, int ny, int nz, vp
     w->ny = ny;
     w->nz = nz;
     w->nbx = nx / 8;
-    w->nby = ny / 8;
-    w->nbz = nz / 8;
+    w->nby = ny / 4;
+    w->nbz = nz / 4;
     size_t v = w->voxels();
     hipError_t e = hipMalloc(&w->d_grid_lin, v);
     if (e == hipSuccess) e = hipMalloc(&w->d_grid, v);
