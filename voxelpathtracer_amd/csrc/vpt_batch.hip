@@ -320,48 +320,98 @@ __global__ void __launch_bounds__(256) persistent_kernel(WorldView w0, const Wor
 }
 
 
-// Served requests, one lane per ray (the launch-wide id selects the
-// segment); a GI bounce that hits a sun-facing block traces its shadow ray
-// in the same lane.  Same traversal code as every other path.
-__global__ void __launch_bounds__(256) serve_direct_kernel(const WorldView* __restrict__ worlds, uint32_t nworlds,
-                                                           Outputs out, uint32_t total)
+__device__ inline void write_hit(vpt_hit* dst, const vpt::Hit& h)
 {
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
-    if (id >= total) return;
-    uint32_t lo = 0, hi = out.nseg;
-    while (hi - lo > 1u) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (out.seg_begin[mid] <= id) lo = mid;
-        else hi = mid;
-    }
-    const vpt::ServeSegment& sg = out.segs[lo];
-    const uint32_t local = sg.first + (id - sg.begin);
-    const vpt_ray q = sg.rays[local];
-    WorldView wv;
-    if (sg.world < nworlds) {
-        wv = worlds[sg.world];
-    } else {
-        memset(&wv, 0, sizeof(wv));
-        wv.xmax = wv.ymax = wv.zmax = -1.0f;
-    }
-    const Vec3 o = vpt::mk3(q.origin[0], q.origin[1], q.origin[2]);
-    const Vec3 d = vpt::mk3(q.dir[0], q.dir[1], q.dir[2]);
-    const vpt::Hit h = vpt::traverse(wv, o, d, sg.max_iter);
     vpt_hit r;
     r.t = h.t;
     r.voxel = h.voxel;
     r.face = (uint8_t)h.face;
     r.block = (uint8_t)h.block;
     r.samples = (uint16_t)min(h.samples, 65535);
-    sg.hits[local] = r;
-    if (sg.kind == VPT_REQ_GI) {
-        const Vec3 L = vpt::mk3(sg.sun[0], sg.sun[1], sg.sun[2]);
-        Vec3 so;
-        float ndotl;
-        uint8_t v = 255;
-        if (h.t > 0.0f && h.block > 0 && vpt::gi_shadow_origin(o, d, h.t, h.face, L, so, ndotl))
-            v = vpt::traverse(wv, so, L, sg.shadow_iter).t > 0.0f ? 1 : 0;
-        sg.vis[local] = v;
+    *dst = r;
+}
+
+__device__ inline WorldView served_world(const WorldView* __restrict__ worlds, uint32_t nworlds, uint32_t world)
+{
+    WorldView wv;
+    if (world < nworlds) {
+        wv = worlds[world];
+    } else {
+        memset(&wv, 0, sizeof(wv));
+        wv.xmax = wv.ymax = wv.zmax = -1.0f;
+    }
+    return wv;
+}
+
+// Served requests, one lane per ray (the launch-wide id selects the
+// segment).  A GI bounce that hits a sun-facing block goes on as its shadow
+// ray: in launches that fill the chip in blocks that hold GI rays, regrouped
+// and compacted within the block, else in the same lane (see RayBlock).
+// Same traversal code as every other path.
+__global__ void __launch_bounds__(256) serve_direct_kernel(const WorldView* __restrict__ worlds, uint32_t nworlds,
+                                                           Outputs out, uint32_t total)
+{
+    __shared__ vpt::RayBlock blk;
+    const uint32_t id0 = blockIdx.x * 256u, id = id0 + threadIdx.x;
+    const bool valid = id < total;
+    uint32_t lo = 0;
+    Vec3 o = vpt::mk3(0.0f, 0.0f, 0.0f), d = o;
+    bool gi = false;
+    if (valid) {
+        uint32_t hi = out.nseg;
+        while (hi - lo > 1u) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (out.seg_begin[mid] <= id) lo = mid;
+            else hi = mid;
+        }
+        const vpt::ServeSegment& sg = out.segs[lo];
+        const vpt_ray q = sg.rays[sg.first + (id - sg.begin)];
+        o = vpt::mk3(q.origin[0], q.origin[1], q.origin[2]);
+        d = vpt::mk3(q.dir[0], q.dir[1], q.dir[2]);
+        gi = sg.kind == VPT_REQ_GI;
+    }
+    const bool grouped = gridDim.x > vpt::kSmallLaunch && __syncthreads_or(gi);
+    if (!grouped) {
+        if (!valid) return;
+        const vpt::ServeSegment& sg = out.segs[lo];
+        const uint32_t local = sg.first + (id - sg.begin);
+        const WorldView wv = served_world(worlds, nworlds, sg.world);
+        const vpt::Hit h = vpt::traverse(wv, o, d, sg.max_iter);
+        write_hit(sg.hits + local, h);
+        if (gi) {
+            const Vec3 L = vpt::mk3(sg.sun[0], sg.sun[1], sg.sun[2]);
+            Vec3 so;
+            float ndotl;
+            uint8_t v = 255;
+            if (h.t > 0.0f && h.block > 0 && vpt::gi_shadow_origin(o, d, h.t, h.face, L, so, ndotl))
+                v = vpt::traverse(wv, so, L, sg.shadow_iter).t > 0.0f ? 1 : 0;
+            sg.vis[local] = v;
+        }
+        return;
+    }
+    // a lane's work: segment << 8 | the ray's lane in the launch's block
+    uint32_t work = valid ? (lo << 8) | threadIdx.x : 0xffffffffu;
+    vpt::regroup(blk, valid ? (gi ? vpt::ray_bin(d.y) : vpt::kRayBins) : vpt::kRayBins + 1, o, d, work);
+    bool job = false;
+    Vec3 so = o;
+    if (work != 0xffffffffu) {
+        const vpt::ServeSegment& sg = out.segs[work >> 8];
+        const uint32_t local = sg.first + (id0 + (work & 255u) - sg.begin);
+        const WorldView wv = served_world(worlds, nworlds, sg.world);
+        const vpt::Hit h = vpt::traverse(wv, o, d, sg.max_iter);
+        write_hit(sg.hits + local, h);
+        if (sg.kind == VPT_REQ_GI) {
+            float ndotl;
+            job = h.t > 0.0f && h.block > 0 &&
+                  vpt::gi_shadow_origin(o, d, h.t, h.face, vpt::mk3(sg.sun[0], sg.sun[1], sg.sun[2]), so, ndotl);
+            if (!job) sg.vis[local] = 255;
+        }
+    }
+    if (vpt::compact(blk, job, so, work)) {
+        const vpt::ServeSegment& sg = out.segs[work >> 8];
+        const WorldView wv = served_world(worlds, nworlds, sg.world);
+        const vpt::Hit h = vpt::traverse(wv, so, vpt::mk3(sg.sun[0], sg.sun[1], sg.sun[2]), sg.shadow_iter);
+        sg.vis[sg.first + (id0 + (work & 255u) - sg.begin)] = h.t > 0.0f ? 1 : 0;
     }
 }
 

@@ -207,4 +207,85 @@ int check_cam(const vpt_camera* cam, const char* fn);
 int check_gbuffer(const vpt_gbuffer* gb, const vpt_camera* cam, const char* fn, bool need_block);
 int check_iter(int max_iter, const char* fn);
 
+// GI ray queries: a workgroup's 256 rays and their shadow rays.
+//
+// Bounce rays' lengths vary widely with their direction's height (rays
+// leaving upward escape in a few steps, grazing ones walk the terrain), and
+// a quarter of them cast a shadow ray at their hit.  In launches that fill
+// the chip the block's rays are regrouped onto lanes by the direction's y
+// (16 bins), so that a wavefront holds rays of similar length, and the
+// shadow rays are compacted onto the first lanes.  In small launches, which
+// wait for their longest ray, each lane goes from its bounce to its shadow
+// ray without waiting for the block.
+constexpr int kRayBins = 16;
+
+struct RayBlock {
+    float r[6][256];
+    uint32_t id[256];
+    int bin[kRayBins + 2];   // counts, then first slots; [kRayBins]: other rays, in place among themselves
+    int jobs;
+};
+
+__device__ inline int ray_bin(float dir_y)
+{
+    return min(kRayBins - 1, max(0, (int)((dir_y + 1.0f) * (0.5f * kRayBins))));
+}
+
+// Every lane's ray to its slot by bin (kRayBins + 1: no ray), then this
+// lane's slot back.  All 256 lanes must call it.
+__device__ inline void regroup(RayBlock& b, int bin, Vec3& o, Vec3& d, uint32_t& id)
+{
+    if (threadIdx.x < kRayBins + 2) b.bin[threadIdx.x] = 0;
+    if (threadIdx.x == 0) b.jobs = 0;
+    __syncthreads();
+    const int rank = atomicAdd(&b.bin[bin], 1);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int acc = 0;
+        for (int k = 0; k < kRayBins + 2; k++) {
+            const int c = b.bin[k];
+            b.bin[k] = acc;
+            acc += c;
+        }
+    }
+    __syncthreads();
+    const int slot = b.bin[bin] + rank;   // < 256: the slots of the block's 256 lanes
+    b.r[0][slot] = o.x;
+    b.r[1][slot] = o.y;
+    b.r[2][slot] = o.z;
+    b.r[3][slot] = d.x;
+    b.r[4][slot] = d.y;
+    b.r[5][slot] = d.z;
+    b.id[slot] = id;
+    __syncthreads();
+    o = mk3(b.r[0][threadIdx.x], b.r[1][threadIdx.x], b.r[2][threadIdx.x]);
+    d = mk3(b.r[3][threadIdx.x], b.r[4][threadIdx.x], b.r[5][threadIdx.x]);
+    id = b.id[threadIdx.x];
+    __syncthreads();   // the slots may be written again (compact)
+}
+
+// The shadow rays (o, id) of the lanes with `job`, packed onto the block's
+// first lanes; whether this lane has one.  All 256 lanes must call it, after
+// regroup.
+__device__ inline bool compact(RayBlock& b, bool job, Vec3& o, uint32_t& id)
+{
+    const uint64_t m = __ballot(job);
+    const int lane = (int)(threadIdx.x & 63);
+    int base = 0;
+    if (lane == 0 && m) base = atomicAdd(&b.jobs, (int)__popcll(m));
+    base = __shfl(base, 0);
+    if (job) {
+        const int slot = base + (int)__popcll(m & ((1ull << lane) - 1ull));
+        b.r[0][slot] = o.x;
+        b.r[1][slot] = o.y;
+        b.r[2][slot] = o.z;
+        b.id[slot] = id;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x >= b.jobs) return false;
+    o = mk3(b.r[0][threadIdx.x], b.r[1][threadIdx.x], b.r[2][threadIdx.x]);
+    id = b.id[threadIdx.x];
+    return true;
+}
+
 }  // namespace vpt

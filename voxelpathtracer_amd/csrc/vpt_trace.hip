@@ -664,31 +664,46 @@ __global__ void __launch_bounds__(256) rays_kernel(WorldView w, const vpt_ray* _
     count_samples(counter, samples, nrays);
 }
 
-// Shadow rays of GI ray queries (second launch of vpt_trace_gi_rays): the
-// bounce hit in hits[i] continues toward the sun when its face sees it.
-__global__ void __launch_bounds__(256) gi_rays_shadow_kernel(WorldView w, const vpt_ray* __restrict__ rays, int n,
-                                                             const vpt_hit* __restrict__ hits, float lx, float ly,
-                                                             float lz, int shadow_iter, uint8_t* __restrict__ vis,
-                                                             unsigned long long* __restrict__ counter)
+// GI ray queries: the bounce, then, when its hit's face sees the sun, the
+// shadow ray from there (see RayBlock).
+__global__ void __launch_bounds__(256) gi_rays_kernel(WorldView w, const vpt_ray* __restrict__ rays, int n, int gi_iter,
+                                                      float lx, float ly, float lz, int shadow_iter,
+                                                      vpt_hit* __restrict__ hits, uint8_t* __restrict__ vis,
+                                                      unsigned long long* __restrict__ counter)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ vpt::RayBlock blk;
+    const Vec3 L = vpt::mk3(lx, ly, lz);
+    uint32_t i = blockIdx.x * 256u + threadIdx.x;
     int samples = 0, nrays = 0;
-    if (i < n) {
+    Vec3 o = vpt::mk3(0.0f, 0.0f, 0.0f), d = o, so = o;
+    if (i < (uint32_t)n) {
         const vpt_ray r = rays[i];
-        const vpt_hit h = hits[i];
-        const Vec3 L = vpt::mk3(lx, ly, lz);
-        Vec3 so;
+        o = vpt::mk3(r.origin[0], r.origin[1], r.origin[2]);
+        d = vpt::mk3(r.dir[0], r.dir[1], r.dir[2]);
+    }
+    const bool grouped = gridDim.x > vpt::kSmallLaunch;
+    if (grouped) vpt::regroup(blk, i < (uint32_t)n ? vpt::ray_bin(d.y) : vpt::kRayBins + 1, o, d, i);
+    bool job = false;
+    if (i < (uint32_t)n) {
+        const vpt::Hit h = vpt::traverse(w, o, d, gi_iter);
+        vpt_hit r;
+        r.t = h.t;
+        r.voxel = h.voxel;
+        r.face = (uint8_t)h.face;
+        r.block = (uint8_t)h.block;
+        r.samples = (uint16_t)min(h.samples, 65535);
+        hits[i] = r;
+        samples = h.samples;
+        nrays = 1;
         float ndotl;
-        uint8_t v = 255;
-        if (h.t > 0.0f && h.block > 0 &&
-            vpt::gi_shadow_origin(vpt::mk3(r.origin[0], r.origin[1], r.origin[2]),
-                                  vpt::mk3(r.dir[0], r.dir[1], r.dir[2]), h.t, h.face, L, so, ndotl)) {
-            vpt::Hit s = vpt::traverse(w, so, L, shadow_iter);
-            v = s.t > 0.0f ? 1 : 0;
-            samples = s.samples;
-            nrays = 1;
-        }
-        vis[i] = v;
+        job = h.t > 0.0f && h.block > 0 && vpt::gi_shadow_origin(o, d, h.t, h.face, L, so, ndotl);
+        if (!job) vis[i] = 255;
+    }
+    if (grouped ? vpt::compact(blk, job, so, i) : job) {
+        const vpt::Hit s = vpt::traverse(w, so, L, shadow_iter);
+        vis[i] = s.t > 0.0f ? 1 : 0;
+        samples += s.samples;
+        nrays++;
     }
     count_samples(counter, samples, nrays);
 }
@@ -1769,11 +1784,8 @@ extern "C" VPT_API int vpt_trace_gi_rays(vpt_world* w, const vpt_ray* d_rays, in
     DeviceGuard g(w->device);
     const WorldView wv = vpt::make_view(w);
     const dim3 grid((unsigned)((n + 255) / 256));
-    hipLaunchKernelGGL(rays_kernel, grid, dim3(256), 0, (hipStream_t)stream, wv, d_rays, n, gi_iter, d_hits,
-                       w->d_counter);
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(gi_rays_shadow_kernel, grid, dim3(256), 0, (hipStream_t)stream, wv, d_rays, n, d_hits,
-                       sun_dir[0], sun_dir[1], sun_dir[2], shadow_iter, d_vis, w->d_counter);
+    hipLaunchKernelGGL(gi_rays_kernel, grid, dim3(256), 0, (hipStream_t)stream, wv, d_rays, n, gi_iter, sun_dir[0],
+                       sun_dir[1], sun_dir[2], shadow_iter, d_hits, d_vis, w->d_counter);
     HIP_TRY(hipGetLastError());
     return VPT_OK;
 }
