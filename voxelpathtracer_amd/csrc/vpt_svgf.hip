@@ -204,28 +204,62 @@ __device__ inline float bil(float t00, float t10, float t01, float t11, float a,
     return top * (1.0f - b) + bot * b;
 }
 
-__device__ inline Tx bil_of(const Tx& q00, const Tx& q10, const Tx& q01, const Tx& q11, const Bil& f)
+// -0 in a register, unknown to the compiler: x * k + (-0) as one fma is the
+// rounded product x * k for every x and k, signs of zero included, and with a
+// binary16 x it is one v_fma_mix_f32, which converts the half on the way
+// (the conversion is exact) where v_cvt_f32_f16 and a multiply take two
+// instructions.  A constant -0 would be folded back into the multiply.  The
+// denoiser passes are bound by VALU issue and bilinear taps of seven
+// binary16 channels are most of it (SVGF frame at 1920x1080: 761 -> 747 us).
+__device__ inline float neg_zero()
+{
+    float z = -0.0f;
+    asm volatile("" : "+v"(z));
+    return z;
+}
+
+// k times the low or high binary16 of w.
+template <bool kHi>
+__device__ inline float mul_h(uint32_t w, float k, float nz)
+{
+    return __builtin_fmaf(h2f(kHi ? w >> 16 : w & 0xffffu), k, nz);
+}
+
+// bil of binary16 values.
+template <bool kHi>
+__device__ inline float bil_h(uint32_t w00, uint32_t w10, uint32_t w01, uint32_t w11, float a, float b, float nz)
+{
+    const float top = mul_h<kHi>(w00, 1.0f - a, nz) + mul_h<kHi>(w10, a, nz);
+    const float bot = mul_h<kHi>(w01, 1.0f - a, nz) + mul_h<kHi>(w11, a, nz);
+    return top * (1.0f - b) + bot * b;
+}
+
+// The bilinear texel of four; ao_sky(word) decodes the two bytes.
+template <class Decode>
+__device__ __attribute__((always_inline)) inline Tx bil_texels(const uint4& q00, const uint4& q10, const uint4& q01,
+                                                               const uint4& q11, float a, float b, float nz,
+                                                               Decode&& ao_sky)
 {
     Tx r;
-    for (int c = 0; c < 4; c++) r.sh[c] = bil(q00.sh[c], q10.sh[c], q01.sh[c], q11.sh[c], f.a, f.b);
-    r.co = bil(q00.co, q10.co, q01.co, q11.co, f.a, f.b);
-    r.cg = bil(q00.cg, q10.cg, q01.cg, q11.cg, f.a, f.b);
-    r.x = bil(q00.x, q10.x, q01.x, q11.x, f.a, f.b);
-    r.ao = bil(q00.ao, q10.ao, q01.ao, q11.ao, f.a, f.b);
-    r.sky = bil(q00.sky, q10.sky, q01.sky, q11.sky, f.a, f.b);
+    r.sh[0] = bil_h<false>(q00.x, q10.x, q01.x, q11.x, a, b, nz);
+    r.sh[1] = bil_h<true>(q00.x, q10.x, q01.x, q11.x, a, b, nz);
+    r.sh[2] = bil_h<false>(q00.y, q10.y, q01.y, q11.y, a, b, nz);
+    r.sh[3] = bil_h<true>(q00.y, q10.y, q01.y, q11.y, a, b, nz);
+    r.co = bil_h<false>(q00.z, q10.z, q01.z, q11.z, a, b, nz);
+    r.cg = bil_h<true>(q00.z, q10.z, q01.z, q11.z, a, b, nz);
+    r.x = bil_h<false>(q00.w, q10.w, q01.w, q11.w, a, b, nz);
+    const float2 b00 = ao_sky(q00.w), b10 = ao_sky(q10.w), b01 = ao_sky(q01.w), b11 = ao_sky(q11.w);
+    r.ao = bil(b00.x, b10.x, b01.x, b11.x, a, b);
+    r.sky = bil(b00.y, b10.y, b01.y, b11.y, a, b);
     return r;
 }
 
-__device__ inline Tx bil_tx(const vpt_svgf_texel* p, const Bil& f)
+// The AO and sky bytes of a texel's last word, through the LDS table.
+__device__ inline float2 ao_sky_lut(uint32_t w, const float* unorm8)
 {
-    return bil_of(load_tx(p, f.i00), load_tx(p, f.i10), load_tx(p, f.i01), load_tx(p, f.i11), f);
-}
-
-__device__ inline Tx bil_tx_lut(const vpt_svgf_texel* p, const Bil& f, const float* unorm8)
-{
-    const uint4* q = reinterpret_cast<const uint4*>(p);
-    return bil_of(load_tx_word_lut(q[f.i00], unorm8), load_tx_word_lut(q[f.i10], unorm8),
-                  load_tx_word_lut(q[f.i01], unorm8), load_tx_word_lut(q[f.i11], unorm8), f);
+    typedef const __attribute__((address_space(3))) float LdsFloat;
+    LdsFloat* t = (LdsFloat*)unorm8;
+    return make_float2(t[(w >> 16) & 0xffu], t[w >> 24]);
 }
 
 // GL NEAREST + REPEAT texel index for coordinates inside (0, 1), where
@@ -310,6 +344,7 @@ __global__ void __launch_bounds__(256) prespatial_kernel(CamView cam, int W, int
     float tco = base.co, tcg = base.cg, tw = 1.0f;
     float tao = base.ao, tsky = base.sky, taow = 1.0f;
     const float phi_color = 4.0f;
+    const float nz = neg_zero();
     for (int x = -1; x <= 1; x++) {
         for (int y = -1; y <= 1; y++) {
             if (x == 0 && y == 0) continue;
@@ -321,9 +356,9 @@ __global__ void __launch_bounds__(256) prespatial_kernel(CamView cam, int W, int
             Vec3 pd = vpt::mk3(fabsf(sp.x - base_pos.x), fabsf(sp.y - base_pos.y), fabsf(sp.z - base_pos.z));
             float dist_sqr = vpt::dot3(pd, pd);
             if (dist_sqr < 1.0f) {
-                Tx s = load_tx_word_lut(in4[j], s_unorm8);
+                const uint4 q = in4[j];
                 Vec3 sn = vpt::face_normal(gb_face[j], 1.0f);
-                float sluma = sh_to_y(s.sh[3]);
+                float sluma = sh_to_y(h2f(q.y >> 16));
                 float nw = vpt_powi(fmaxf(vpt::dot3(base_n, sn), 0.0f), 16);
                 float lw = fabsf(sluma - base_luma) / phi_color;
                 float w = vpt_expf(-lw - nw);
@@ -331,12 +366,16 @@ __global__ void __launch_bounds__(256) prespatial_kernel(CamView cam, int W, int
                 w = (atrous[abs(x)] * atrous[abs(y)]) * w;
                 w = fmaxf(w, 0.01f);
                 w = fclamp(w, 0.0f, 1.0f);
-                for (int k = 0; k < 4; k++) tsh[k] = tsh[k] + s.sh[k] * w;
-                tco = tco + s.co * w;
-                tcg = tcg + s.cg * w;
+                tsh[0] = tsh[0] + mul_h<false>(q.x, w, nz);
+                tsh[1] = tsh[1] + mul_h<true>(q.x, w, nz);
+                tsh[2] = tsh[2] + mul_h<false>(q.y, w, nz);
+                tsh[3] = tsh[3] + mul_h<true>(q.y, w, nz);
+                tco = tco + mul_h<false>(q.z, w, nz);
+                tcg = tcg + mul_h<true>(q.z, w, nz);
                 tw = tw + w;
-                tao = tao + s.ao * w;
-                tsky = tsky + s.sky * w;
+                const float2 as = ao_sky_lut(q.w, s_unorm8);
+                tao = tao + as.x * w;
+                tsky = tsky + as.y * w;
                 taow = taow + w;
             }
         }
@@ -408,6 +447,7 @@ __global__ void __launch_bounds__(256) temporal_kernel(CamView cam, Mat16 prev_v
     float ssh[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     float sco = 0.0f, scg = 0.0f, sao = 0.0f, ssky = 0.0f, slum = 0.0f, sspp = 0.0f, smom = 0.0f;
     int successful = 0;
+    const float nz = neg_zero();
     for (int k = 0; k < 5; k++) {
         float sx = rx + (offx[k] + 0.0f) * tex_w;
         float sy = ry + (offy[k] + 0.0f) * tex_h;
@@ -428,13 +468,13 @@ __global__ void __launch_bounds__(256) temporal_kernel(CamView cam, Mat16 prev_v
         }
         if (valid) {
             float cw = weights[k];
-            Tx h = bil_tx_lut(hist, f, s_unorm8);
+            const uint4* hq = reinterpret_cast<const uint4*>(hist);
+            const Tx h = bil_texels(hq[f.i00], hq[f.i10], hq[f.i01], hq[f.i11], f.a, f.b, nz,
+                                    [&](uint32_t w) { return ao_sky_lut(w, s_unorm8); });
             uint2 u00 = hist_util[f.i00], u10 = hist_util[f.i10], u01 = hist_util[f.i01], u11 = hist_util[f.i11];
-            float spp = bil(h2f(u00.x & 0xffffu), h2f(u10.x & 0xffffu), h2f(u01.x & 0xffffu), h2f(u11.x & 0xffffu),
-                            f.a, f.b);
-            float mom = bil(h2f(u00.x >> 16), h2f(u10.x >> 16), h2f(u01.x >> 16), h2f(u11.x >> 16), f.a, f.b);
-            float lum = bil(h2f(u00.y & 0xffffu), h2f(u10.y & 0xffffu), h2f(u01.y & 0xffffu), h2f(u11.y & 0xffffu),
-                            f.a, f.b);
+            float spp = bil_h<false>(u00.x, u10.x, u01.x, u11.x, f.a, f.b, nz);
+            float mom = bil_h<true>(u00.x, u10.x, u01.x, u11.x, f.a, f.b, nz);
+            float lum = bil_h<false>(u00.y, u10.y, u01.y, u11.y, f.a, f.b, nz);
             for (int c = 0; c < 4; c++) ssh[c] = ssh[c] + h.sh[c] * cw;
             sco = sco + h.co * cw;
             scg = scg + h.cg * cw;
@@ -766,17 +806,19 @@ struct GlobalSrc {
     const uint8_t* face;
     int W, H;
     __device__ uint32_t idx(int vx, int vy) const { return (uint32_t)wrap1(vy, H) * (uint32_t)W + (uint32_t)wrap1(vx, W); }
-    __device__ Tx tex_at(uint32_t j) const
+    __device__ uint4 raw_at(uint32_t j) const
     {
-        return load_tx_word(*reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(in) + j * 16u));
+        return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(in) + j * 16u);
+    }
+    __device__ Tx tex_at(uint32_t j) const { return load_tx_word(raw_at(j)); }
+    __device__ float2 ao_sky(uint32_t w) const
+    {
+        return make_float2(vpt_unorm8_decode((uint8_t)((w >> 16) & 0xffu)), vpt_unorm8_decode((uint8_t)(w >> 24)));
     }
     __device__ float depth_at(uint32_t j) const
     {
         return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(t) + j * 4u);
     }
-    __device__ Tx tex(int vx, int vy) const { return tex_at(idx(vx, vy)); }
-    __device__ float depth(int vx, int vy) const { return depth_at(idx(vx, vy)); }
-    __device__ int fc(int vx, int vy) const { return face[idx(vx, vy)]; }
     __device__ float xch(int vx, int vy) const
     {
         return h2f(*reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(in) + idx(vx, vy) * 16u + 12u) &
@@ -787,10 +829,8 @@ struct GlobalSrc {
 // The same source with the AO / sky bytes decoded through the LDS table.
 struct GlobalSrcLut : GlobalSrc {
     const float* unorm8;   // LDS
-    __device__ Tx tex_at(uint32_t j) const
-    {
-        return load_tx_word_lut(*reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(in) + j * 16u), unorm8);
-    }
+    __device__ Tx tex_at(uint32_t j) const { return load_tx_word_lut(raw_at(j), unorm8); }
+    __device__ float2 ao_sky(uint32_t w) const { return ao_sky_lut(w, unorm8); }
 };
 
 // Normal-weight class of a face byte: the six faces, or 6 for every other
@@ -883,37 +923,48 @@ __device__ __attribute__((always_inline)) inline void atrous_px(const Src& src, 
     const float rphi = 1.0f / phi;
 
     if (!(base_depth < 0.0f)) {
+        const float nz = neg_zero();
         const float jh = (float)jit * 0.5f;
+        // the three columns and rows of the taps: GL LINEAR footprint (as
+        // bil_setup) and NEAREST texel, at virtual coordinates.  Inside the
+        // taps' own branches they were computed eight times each (SVGF frame
+        // at 1920x1080: 747 -> 741 us).
+        struct Line {
+            bool in;
+            float frac;
+            uint32_t i0, i1, near;
+        } col[3], row[3];
+        auto line = [&](float uv, float tex, int k, int n) __attribute__((always_inline)) {
+            const float s = uv + (((float)k * (float)step) * scale + jh) * tex;
+            const float u = s * (float)n - 0.5f;
+            const float fu = floorf(u);
+            const int x0 = (int)fu;
+            return Line{s < 1.0f && s > 0.0f, u - fu, (uint32_t)wrap1(x0, n), (uint32_t)wrap1(x0 + 1, n),
+                        (uint32_t)wrap1((int)floorf(s * (float)n), n)};
+        };
+#pragma unroll
+        for (int k = -1; k <= 1; k++) {
+            col[k + 1] = line(uvx, tex_w, k, W);
+            row[k + 1] = line(uvy, tex_h, k, H);
+            row[k + 1].i0 *= (uint32_t)W;
+            row[k + 1].i1 *= (uint32_t)W;
+            row[k + 1].near *= (uint32_t)W;
+        }
 #pragma unroll
         for (int x = -1; x <= 1; x++) {
 #pragma unroll
             for (int y = -1; y <= 1; y++) {
                 if (x == 0 && y == 0) continue;
-                float ox = ((float)x * (float)step) * scale + jh;
-                float oy = ((float)y * (float)step) * scale + jh;
-                float sx = uvx + ox * tex_w;
-                float sy = uvy + oy * tex_h;
-                if (!in_screen(sx, sy)) continue;
-                // GL LINEAR footprint (as bil_setup), at virtual coordinates
-                const float u = sx * (float)W - 0.5f, v = sy * (float)H - 0.5f;
-                const float fu = floorf(u), fv = floorf(v);
-                const float a = u - fu, b = v - fv;
-                const int x0 = (int)fu, y0 = (int)fv;
-                const uint32_t c0 = (uint32_t)wrap1(x0, W), c1 = (uint32_t)wrap1(x0 + 1, W);
-                const uint32_t r0 = (uint32_t)wrap1(y0, H) * (uint32_t)W, r1 = (uint32_t)wrap1(y0 + 1, H) * (uint32_t)W;
-                const uint32_t j00 = r0 + c0, j10 = r0 + c1, j01 = r1 + c0, j11 = r1 + c1;
+                const Line cx = col[x + 1], ry = row[y + 1];
+                if (!(cx.in && ry.in)) continue;
+                const float a = cx.frac, b = ry.frac;
+                const uint32_t j00 = ry.i0 + cx.i0, j10 = ry.i0 + cx.i1, j01 = ry.i1 + cx.i0, j11 = ry.i1 + cx.i1;
                 float sdepth = bil(src.depth_at(j00), src.depth_at(j10), src.depth_at(j01), src.depth_at(j11), a, b);
                 float ddiff = fabsf(sdepth - base_depth);
                 const float nw = nw32_of(base_class,
-                                         face_class(src.fc((int)floorf(sx * (float)W), (int)floorf(sy * (float)H))));
-                const Tx q00 = src.tex_at(j00), q10 = src.tex_at(j10), q01 = src.tex_at(j01), q11 = src.tex_at(j11);
-                Tx s;
-                for (int c = 0; c < 4; c++) s.sh[c] = bil(q00.sh[c], q10.sh[c], q01.sh[c], q11.sh[c], a, b);
-                s.co = bil(q00.co, q10.co, q01.co, q11.co, a, b);
-                s.cg = bil(q00.cg, q10.cg, q01.cg, q11.cg, a, b);
-                s.x = bil(q00.x, q10.x, q01.x, q11.x, a, b);
-                s.ao = bil(q00.ao, q10.ao, q01.ao, q11.ao, a, b);
-                s.sky = bil(q00.sky, q10.sky, q01.sky, q11.sky, a, b);
+                                         face_class(src.face[ry.near + cx.near]));
+                const Tx s = bil_texels(src.raw_at(j00), src.raw_at(j10), src.raw_at(j01), src.raw_at(j11), a, b, nz,
+                                        [&](uint32_t w) { return src.ao_sky(w); });
                 float slum = sh_to_y(s.sh[3]);
                 float lw = div_rcp(fabsf(slum - base_lum), phi, rphi);
                 // exp(-d)^2 < 1e-4 for every float d >= 4.7, so the depth
