@@ -168,6 +168,27 @@ __device__ inline Bil bil_setup(float s, float t, int W, int H)
     return b;
 }
 
+// vpt_expf for -21 <= x <= 0: the same polynomial; kf has at most five bits
+// and LN2_HI eight, so their product is exact and the subtraction one fma; the
+// scaling by 2^k, k >= -31, is exact in one step.
+__device__ inline float expf_21(float x)
+{
+    const float LOG2E = 1.44269502162933349609375f;
+    const float LN2_HI = 0.693145751953125f;
+    const float LN2_LO = 1.428606765330187045e-06f;
+    const float kf = floorf(x * LOG2E + 0.5f);
+    float r = __builtin_fmaf(-kf, LN2_HI, x);
+    r = r - kf * LN2_LO;
+    float p = 0.0013829420786350965f;
+    p = p * r + 0.008374771103262901f;
+    p = p * r + 0.0416683591902256f;
+    p = p * r + 0.1666642129421234f;
+    p = p * r + 0.49999991059303284f;
+    p = p * r + 1.0f;
+    p = p * r + 1.0f;
+    return __builtin_ldexpf(p, (int)kf);
+}
+
 // vpt_expf for arguments x <= 0, which the sun-shadow weights pass: the
 // same operations, so the same results, without the NaN and overflow tests
 // (they cannot fire) and with the underflow test (x below -87.34 gives 0) as
@@ -262,14 +283,6 @@ __device__ inline float2 ao_sky_lut(uint32_t w, const float* unorm8)
     return make_float2(t[(w >> 16) & 0xffu], t[w >> 24]);
 }
 
-// GL NEAREST + REPEAT texel index for coordinates inside (0, 1), where
-// floor(s * W) lies in [0, W] (W itself when s * W rounds up to W).
-__device__ inline int nearest_idx(float s, float t, int W, int H)
-{
-    int i = wrap1((int)floorf(s * (float)W), W), j = wrap1((int)floorf(t * (float)H), H);
-    return j * W + i;
-}
-
 // The X channel (binary16 in the low half of the texel's last word).
 __device__ inline float load_x(const vpt_svgf_texel* p, size_t i)
 {
@@ -320,6 +333,36 @@ __device__ inline Vec3 position_from(const CamView& c, float sx, float sy, float
     return vpt::mk3(c.iv[12] + dir.x * dist, c.iv[13] + dir.y * dist, c.iv[14] + dir.z * dist);
 }
 
+// Normal class of a face byte: the six faces, or 6 for every other value
+// (GetNormalFromID's (1, 1, 1)).  Two normals are equal exactly where their
+// classes are.
+__device__ inline uint32_t face_class(int f) { return min((uint32_t)f, 6u); }
+
+// clamp(pow(max(dot(n_a, n_b), 0), 32), 0.001, 1) of two face normals is 1
+// where the dot is positive (the same face; (1, 1, 1) against itself or
+// against +x, +y, +z) and 0.001 elsewhere (dots 0 and -1): bit a * 8 + b of
+// this mask.
+constexpr uint64_t kNw32Mask = (1ull << (0 * 8 + 0)) | (1ull << (1 * 8 + 1)) | (1ull << (2 * 8 + 2)) |
+                               (1ull << (3 * 8 + 3)) | (1ull << (4 * 8 + 4)) | (1ull << (5 * 8 + 5)) |
+                               (1ull << (0 * 8 + 6)) | (1ull << (2 * 8 + 6)) | (1ull << (5 * 8 + 6)) |
+                               (1ull << (6 * 8 + 0)) | (1ull << (6 * 8 + 2)) | (1ull << (6 * 8 + 5)) |
+                               (1ull << (6 * 8 + 6));
+
+__device__ inline float nw32_of(uint32_t base_class, uint32_t sample_class)
+{
+    return ((kNw32Mask >> (base_class * 8u + sample_class)) & 1ull) ? 1.0f : 0.001f;
+}
+
+// pow(max(dot(n_a, n_b), 0), 16) of two face normals: 1 where the dot is 1
+// and 0 where it is 0 or -1, except 3^16 (rounded) for (1, 1, 1) against
+// itself.  By class it takes no branch, where the normals' switches took two
+// a tap.
+__device__ inline float nw16_of(uint32_t a, uint32_t b)
+{
+    const float w = ((kNw32Mask >> (a * 8u + b)) & 1ull) ? 1.0f : 0.0f;
+    return (a == 6u && b == 6u) ? 43046720.0f : w;
+}
+
 // ---- Spatial3x3Initial.main (Spatial3x3Initial.glsl:96-176) --------------
 __global__ void __launch_bounds__(256) prespatial_kernel(CamView cam, int W, int H, const float* __restrict__ gb_t,
                                                          const uint8_t* __restrict__ gb_face,
@@ -336,7 +379,7 @@ __global__ void __launch_bounds__(256) prespatial_kernel(CamView cam, int W, int
     const float tex_w = 1.0f / (float)W, tex_h = 1.0f / (float)H;
     float uvx = texc(px, W), uvy = texc(py, H);
     Vec3 base_pos = position_from(cam, uvx, uvy, gb_t[i]);
-    Vec3 base_n = vpt::face_normal(gb_face[i], 1.0f);
+    const uint32_t base_class = face_class(gb_face[i]);
     const uint4* in4 = reinterpret_cast<const uint4*>(in);
     Tx base = load_tx_word_lut(in4[i], s_unorm8);
     float base_luma = sh_to_y(base.sh[3]);
@@ -357,9 +400,8 @@ __global__ void __launch_bounds__(256) prespatial_kernel(CamView cam, int W, int
             float dist_sqr = vpt::dot3(pd, pd);
             if (dist_sqr < 1.0f) {
                 const uint4 q = in4[j];
-                Vec3 sn = vpt::face_normal(gb_face[j], 1.0f);
                 float sluma = sh_to_y(h2f(q.y >> 16));
-                float nw = vpt_powi(fmaxf(vpt::dot3(base_n, sn), 0.0f), 16);
+                float nw = nw16_of(base_class, face_class(gb_face[j]));
                 float lw = fabsf(sluma - base_luma) / phi_color;
                 float w = vpt_expf(-lw - nw);
                 w = fmaxf(w, 0.01f);
@@ -410,14 +452,14 @@ __global__ void __launch_bounds__(256) temporal_kernel(CamView cam, Mat16 prev_v
     if (!pixel_of(W, H, px, py)) return;
     const size_t i = (size_t)py * W + px;
     const float weights[5] = {3.0f / 32.0f, 3.0f / 32.0f, 9.0f / 64.0f, 3.0f / 32.0f, 3.0f / 32.0f};
-    const float offx[5] = {1.0f, 0.0f, 0.0f, -1.0f, 0.0f};
-    const float offy[5] = {0.0f, 1.0f, 0.0f, 0.0f, -1.0f};
+    constexpr int offx[5] = {1, 0, 0, -1, 0};
+    constexpr int offy[5] = {0, 1, 0, 0, -1};
     const float tex_w = 1.0f / (float)W, tex_h = 1.0f / (float)H;
     const float bth = 0.0035f;
     float uvx = texc(px, W), uvy = texc(py, H);
     float base_w = cur_t[i];
     Vec3 base_pos = position_from(cam, uvx, uvy, base_w);
-    Vec3 base_n = vpt::face_normal(cur_face[i], 1.0f);
+    const uint32_t base_class = face_class(cur_face[i]);
     Tx base = load_tx_word_lut(*reinterpret_cast<const uint4*>(cur + i), s_unorm8);
 
     float q0 = vpt::mat_row(prev_vp.m, 0, base_pos.x, base_pos.y, base_pos.z, 1.0f);
@@ -448,22 +490,53 @@ __global__ void __launch_bounds__(256) temporal_kernel(CamView cam, Mat16 prev_v
     float sco = 0.0f, scg = 0.0f, sao = 0.0f, ssky = 0.0f, slum = 0.0f, sspp = 0.0f, smom = 0.0f;
     int successful = 0;
     const float nz = neg_zero();
+    // The taps are the five of a cross: their footprints (as bil_setup, with
+    // 32-bit texel indices) and nearest texels come from three columns and
+    // three rows.
+    struct Line {
+        float s, frac;
+        uint32_t i0, i1, near;
+        bool in;
+    } col[3], row[3];
+    auto line = [&](float at, int n) __attribute__((always_inline)) {
+        const bool in = at < 1.0f - bth && at > bth;
+        const float s = in ? at : 0.5f;   // the reprojection may be infinite or NaN
+        const float u = s * (float)n - 0.5f;
+        const float fu = floorf(u);
+        const int x0 = (int)fu;
+        return Line{s,
+                    u - fu,
+                    (uint32_t)wrap1(x0, n),
+                    (uint32_t)wrap1(x0 + 1, n),
+                    (uint32_t)wrap1((int)floorf(s * (float)n), n),
+                    in};
+    };
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        col[k] = line(rx + (float)(k - 1) * tex_w, W);
+        row[k] = line(ry + (float)(k - 1) * tex_h, H);
+        row[k].i0 *= (uint32_t)W;
+        row[k].i1 *= (uint32_t)W;
+        row[k].near *= (uint32_t)W;
+    }
+#pragma unroll
     for (int k = 0; k < 5; k++) {
-        float sx = rx + (offx[k] + 0.0f) * tex_w;
-        float sy = ry + (offy[k] + 0.0f) * tex_h;
-        if (!(sx < 1.0f - bth && sx > bth && sy < 1.0f - bth && sy > bth)) continue;
-        Bil f = bil_setup(sx, sy, W, H);
+        const Line cx = col[offx[k] + 1], ry3 = row[offy[k] + 1];
+        if (!(cx.in && ry3.in)) continue;
+        struct {
+            uint32_t i00, i10, i01, i11;
+            float a, b;
+        } f = {ry3.i0 + cx.i0, ry3.i0 + cx.i1, ry3.i1 + cx.i0, ry3.i1 + cx.i1, cx.frac, ry3.frac};
         float pw = bil(prev_t[f.i00], prev_t[f.i10], prev_t[f.i01], prev_t[f.i11], f.a, f.b);
-        Vec3 pp = position_from(cam, sx, sy, pw);
-        int ni = nearest_idx(sx, sy, W, H);
-        Vec3 pn = vpt::face_normal(prev_face[ni], 1.0f);
+        Vec3 pp = position_from(cam, cx.s, ry3.s, pw);
+        const uint32_t ni = ry3.near + cx.near;
         Vec3 pd = vpt::mk3(fabsf(base_pos.x - pp.x), fabsf(base_pos.y - pp.y), fabsf(base_pos.z - pp.z));
         float perr = vpt::dot3(pd, pd);
         int sblock = min(max((int)prev_block[ni], 0), 127);
         bool valid = false;
         if (perr < tol && ((pw < 0.0f) == (base_w < 0.0f))) {
             valid = true;
-            if (do_normal && !(pn.x == base_n.x && pn.y == base_n.y && pn.z == base_n.z)) valid = false;
+            if (do_normal && face_class(prev_face[ni]) != base_class) valid = false;
             if (do_block && base_block != sblock) valid = false;
         }
         if (valid) {
@@ -833,25 +906,6 @@ struct GlobalSrcLut : GlobalSrc {
     __device__ float2 ao_sky(uint32_t w) const { return ao_sky_lut(w, unorm8); }
 };
 
-// Normal-weight class of a face byte: the six faces, or 6 for every other
-// value (GetNormalFromID's (1, 1, 1)).
-__device__ inline uint32_t face_class(int f) { return f <= 5 ? (uint32_t)f : 6u; }
-
-// clamp(pow(max(dot(n_a, n_b), 0), 32), 0.001, 1) of two face normals is 1
-// where the dot is positive (the same face; (1, 1, 1) against itself or
-// against +x, +y, +z) and 0.001 elsewhere (dots 0 and -1): bit a * 8 + b of
-// this mask.
-constexpr uint64_t kNw32Mask = (1ull << (0 * 8 + 0)) | (1ull << (1 * 8 + 1)) | (1ull << (2 * 8 + 2)) |
-                               (1ull << (3 * 8 + 3)) | (1ull << (4 * 8 + 4)) | (1ull << (5 * 8 + 5)) |
-                               (1ull << (0 * 8 + 6)) | (1ull << (2 * 8 + 6)) | (1ull << (5 * 8 + 6)) |
-                               (1ull << (6 * 8 + 0)) | (1ull << (6 * 8 + 2)) | (1ull << (6 * 8 + 5)) |
-                               (1ull << (6 * 8 + 6));
-
-__device__ inline float nw32_of(uint32_t base_class, uint32_t sample_class)
-{
-    return ((kNw32Mask >> (base_class * 8u + sample_class)) & 1ull) ? 1.0f : 0.001f;
-}
-
 // One pixel of the pass, reading through `src`.  kMode is the pass's AO /
 // sky filtering as a compile-time value (0: both, step <= 4; 1: sky only,
 // step <= 6; 2: neither), so that the passes that filter neither skip those
@@ -1077,26 +1131,6 @@ __device__ inline int wrapn(int i, int n)
     return r < 0 ? r + n : r;
 }
 
-// GL LINEAR + REPEAT footprint for any coordinate (the shadow filter's taps
-// reach several texels past the image).
-__device__ inline Bil bil_setup_any(float s, float t, int W, int H)
-{
-    float u = s * (float)W - 0.5f;
-    float v = t * (float)H - 0.5f;
-    float fu = floorf(u), fv = floorf(v);
-    Bil b;
-    b.a = u - fu;
-    b.b = v - fv;
-    const int x0 = wrapn((int)fu, W), x1 = wrapn((int)fu + 1, W);
-    const int y0 = wrapn((int)fv, H), y1 = wrapn((int)fv + 1, H);
-    const uint32_t r0 = (uint32_t)y0 * (uint32_t)W, r1 = (uint32_t)y1 * (uint32_t)W;   // W * H < 2^28
-    b.i00 = r0 + (uint32_t)x0;
-    b.i10 = r0 + (uint32_t)x1;
-    b.i01 = r1 + (uint32_t)x0;
-    b.i11 = r1 + (uint32_t)x1;
-    return b;
-}
-
 __device__ inline float dec8(uint8_t c) { return vpt_unorm8_decode(c); }
 
 // x / 3 for 0 <= x <= 2: q0 = x fl(1/3), then one correction with the exact
@@ -1124,25 +1158,14 @@ __device__ inline float log_ratio(float m)
     return fmaf(fmaf(-b, q0, a), y, q0);
 }
 
-// vpt_logf and vpt_powf with log_ratio in place of their one division:
-// the same operations otherwise, so the same results.
-__device__ inline float logf_rcp(float x)
+// vpt_logf for x in [2/3, 1): the same operations with log_ratio in place of
+// the division and without the cases that cannot arise there, so the same
+// results.
+__device__ inline float logf_unit(float x)
 {
-    if (!(x == x)) return x;
-    if (x < 0.0f) return vpt_u2f(0x7fc00000u);
-    if (x == 0.0f) return vpt_u2f(0xff800000u);
-    if (x == vpt_u2f(0x7f800000u)) return x;
-    uint32_t u = vpt_f2u(x);
-    int e = (int)((u >> 23) & 0xffu) - 127;
-    if (e == -127) {
-        u = vpt_f2u(x * 8388608.0f);
-        e = (int)((u >> 23) & 0xffu) - 127 - 23;
-    }
-    float m = vpt_u2f((u & 0x007fffffu) | 0x3f800000u);
-    if (m > 1.41421353816986083984375f) {
-        m = m * 0.5f;
-        e = e + 1;
-    }
+    const bool low = x + x <= 1.41421353816986083984375f;   // x = m 2^-1 with m up to sqrt(2), or m itself
+    const float m = low ? x + x : x;
+    const float fe = low ? -1.0f : 0.0f;
     const float LN2_HI = 0.693145751953125f;
     const float LN2_LO = 1.428606765330187045e-06f;
     float s = log_ratio(m);
@@ -1152,16 +1175,7 @@ __device__ inline float logf_rcp(float x)
     p = p * s2 + 0.2f;
     p = p * s2 + 0.333333333333f;
     float lm = (s + s) + (s + s) * (s2 * p);
-    float fe = (float)e;
     return fe * LN2_HI + (fe * LN2_LO + lm);
-}
-
-__device__ inline float powf_rcp(float x, float y)
-{
-    if (y == 0.0f) return 1.0f;
-    if (x == 0.0f) return y > 0.0f ? 0.0f : vpt_u2f(0x7f800000u);
-    if (x == 1.0f) return 1.0f;
-    return expf_nonpos(y * logf_rcp(x));
 }
 
 // Every float m in [sqrt(2) / 2, sqrt(2)]: log_ratio(m) against the division.
@@ -1171,6 +1185,14 @@ __global__ void log_division_check_kernel(uint32_t u0, uint32_t n, unsigned long
     if (k >= n) return;
     const float m = __uint_as_float(u0 + k);
     if (__float_as_uint(log_ratio(m)) != __float_as_uint((m - 1.0f) / (m + 1.0f))) atomicAdd(bad, 1ull);
+}
+
+// The weight of two mask values (whole numbers) that differ by d: a constant
+// for each of 0, 1, 2 and everything above.
+__device__ inline float mask_weight(float d)
+{
+    const float wa = fclamp(1.0f - fclamp(d / 3.0f, 0.0f, 1.0f), 0.0f, 1.0f);
+    return fclamp(vpt_powi(wa, 7), 0.000001f, 1.0f);
 }
 
 // GetShadowSpatial (ShadowTemporalFilter.glsl:98-150) over the raw mask.
@@ -1186,7 +1208,7 @@ __device__ inline float shadow_spatial_pre(int px, int py, int W, int H, float t
     float total = (float)mask[i];
     const float base = total;
     float weight = 1.0f;
-    const Vec3 bn = vpt::face_normal(cur_face[i], 1.0f);
+    const uint32_t base_class = face_class(cur_face[i]);
     const float b = 0.03f;
     // the eight neighbours are read first (clamped into the image; a tap off
     // the screen margin is skipped below), so the reads are in flight together
@@ -1209,11 +1231,12 @@ __device__ inline float shadow_spatial_pre(int px, int py, int W, int H, float t
             if (!(sx > b && sx < 1.0f - b && sy > b && sy < 1.0f - b)) continue;
             const int k = (x + 1) * 3 + y + 1;
             const float sd = nd[k];
-            const Vec3 sn = vpt::face_normal((uint8_t)nf[k], 1.0f);
-            if (sn.x == bn.x && sn.y == bn.y && sn.z == bn.z && fabsf(sd - base_depth) < 1.0f) {
+            if (face_class((int)nf[k]) == base_class && fabsf(sd - base_depth) < 1.0f) {
                 const float smp = (float)nm[k];
-                float wa = fclamp(1.0f - fclamp(fabsf(smp - base) / 3.0f, 0.0f, 1.0f), 0.0f, 1.0f);
-                wa = fclamp(vpt_powi(wa, 7), 0.000001f, 1.0f);
+                const float dm = fabsf(smp - base);
+                const float wa = dm == 0.0f ? mask_weight(0.0f) : dm == 1.0f ? mask_weight(1.0f)
+                                            : dm == 2.0f             ? mask_weight(2.0f)
+                                                                     : mask_weight(3.0f);
                 total = total + smp * wa;
                 weight = weight + wa;
             }
@@ -1317,11 +1340,20 @@ __global__ void __launch_bounds__(256) shadow_temporal_kernel(CamView cam, Mat16
 // 11-pixel apron, which holds every bilinear footprint and nearest tap of
 // the 7x7 kernel at filter scales up to 1 (offsets up to 3 * 1.2 * 2.6 =
 // 9.36 pixels) -- is staged once in LDS: depth and the decoded colour per
-// cell, and the face's normal class.  A tap whose footprint leaves the
-// staged cells or wraps at the image edge (REPEAT) reads global memory;
-// both paths read the same values.  The normal weight pow(max(dot, 1e-9),
-// 32) of two face normals takes one of three values and comes from a 7x7
-// table built with the same expression.
+// cell, and the face's normal class.  Cells past the image edge hold the
+// texel that REPEAT reads there, so a tap asks only whether it lies in the
+// window.  The normal weight pow(max(dot, 1e-9), 32) of two face normals
+// takes one of three values and comes from a 7x7 table built with the same
+// expression.
+//
+// Bound by VALU issue over up to 49 taps a pixel.  A wavefront whose taps are
+// all in the window (every one at scales up to 1) computes its pixels' seven
+// rows once and keeps them in registers; the others (larger scales) take a
+// loop that works each tap out and reads global memory where it leaves the
+// window.  The choice is the wavefront's, since one that splits runs both
+// loops (320x180 at scale 2.5: 67 us split, 51 us whole).  Temporal pass and
+// filter, 229 -> 149 us at 1920x1080 and 49 -> 27 us at 320x180, of which the
+// cheaper exp and log and the normal classes are a part.
 constexpr int kSfA = 11;
 constexpr int kSfW = 32 + 2 * kSfA, kSfH = 8 + 2 * kSfA, kSfCells = kSfW * kSfH;
 
@@ -1340,9 +1372,7 @@ __global__ void __launch_bounds__(256) shadow_filter_kernel(int W, int H, const 
     const int tx0 = (int)tile.x * 32, ty0 = (int)tile.y * 8;
     const int gx0 = tx0 - kSfA, gy0 = ty0 - kSfA;   // image position of staged cell (0, 0)
     {
-        // the staged cells, seven per thread (256 threads), read together: a
-        // cell off the image reads the nearest one on it and is never read
-        // back from LDS
+        // the staged cells, seven per thread (256 threads), read together
         constexpr int kPer = (kSfCells + 255) / 256;
         const int tid = (int)threadIdx.x;
         __builtin_assume(tid >= 0 && tid < 256);
@@ -1352,7 +1382,7 @@ __global__ void __launch_bounds__(256) shadow_filter_kernel(int W, int H, const 
         for (int k = 0; k < kPer; k++) {
             const int c = tid + 256 * k;
             if (c < kSfCells) {
-                const int gx = min(max(gx0 + c % kSfW, 0), W - 1), gy = min(max(gy0 + c / kSfW, 0), H - 1);
+                const int gx = wrapn(gx0 + c % kSfW, W), gy = wrapn(gy0 + c / kSfW, H);
                 const uint32_t j = (uint32_t)gy * (uint32_t)W + (uint32_t)gx;
                 st[k] = gb_t[j];
                 sc[k] = color[j];
@@ -1406,62 +1436,86 @@ __global__ void __launch_bounds__(256) shadow_filter_kernel(int W, int H, const 
         lm = 0.1f * (1.0f - fn) + 0.5f * fn;
     }
     const float expo = (ve * lm) * 0.9f;
+    // The weight is ((clamp(pow) * dw) * nw) with pow <= 1, so it sits on its
+    // 1e-9 clamp once dw * nw < 1e-9: nw is exactly 0 or 1 for a normal of an
+    // axis, and exp(-d)^3 < 1e-9 for every float d >= 21.  Those taps skip the
+    // exp and the pow.  The pow's base lies in [2/3, 1].
     float tw = 0.0f, ts = 0.0f;
-    for (int x = -size; x <= size; x++) {
-        for (int y = -size; y <= size; y++) {
-            const float sx = uvx + (((float)x * tex_w) * 1.2f * sc) * scale;
-            const float sy = uvy + (((float)y * tex_h) * 1.2f * sc) * scale;
-            // GL LINEAR footprint (as bil_setup_any) and NEAREST texel
-            const float u = sx * (float)W - 0.5f, v = sy * (float)H - 0.5f;
-            const float fu = floorf(u), fv = floorf(v);
-            const float fa = u - fu, fb = v - fv;
-            const int x0 = (int)fu, y0 = (int)fv;
-            const int nxi = (int)floorf(sx * (float)W), nyi = (int)floorf(sy * (float)H);
-            const int lx = x0 - gx0, ly = y0 - gy0, nlx = nxi - gx0, nly = nyi - gy0;
-            const bool staged = x0 >= 0 && x0 + 1 < W && y0 >= 0 && y0 + 1 < H && lx >= 0 && lx + 1 < kSfW &&
-                                ly >= 0 && ly + 1 < kSfH && nxi >= 0 && nxi < W && nyi >= 0 && nyi < H &&
-                                nlx >= 0 && nlx < kSfW && nly >= 0 && nly < kSfH;
-            float d00, d10, d01, d11, c00, c10, c01, c11, nw;
-            if (staged) {
-                const int c = ly * kSfW + lx;
-                const float2 q00 = s_dc[c], q10 = s_dc[c + 1], q01 = s_dc[c + kSfW], q11 = s_dc[c + kSfW + 1];
-                d00 = q00.x; d10 = q10.x; d01 = q01.x; d11 = q11.x;
-                c00 = q00.y; c10 = q10.y; c01 = q01.y; c11 = q11.y;
-                nw = nw_row[s_f[nly * kSfW + nlx]];
-            } else {
-                const uint32_t wx0 = (uint32_t)wrapn(x0, W), wx1 = (uint32_t)wrapn(x0 + 1, W);
-                const uint32_t r0 = (uint32_t)wrapn(y0, H) * (uint32_t)W, r1 = (uint32_t)wrapn(y0 + 1, H) * (uint32_t)W;
-                d00 = gb_t[r0 + wx0]; d10 = gb_t[r0 + wx1]; d01 = gb_t[r1 + wx0]; d11 = gb_t[r1 + wx1];
-                c00 = dec8(color[r0 + wx0]); c10 = dec8(color[r0 + wx1]);
-                c01 = dec8(color[r1 + wx0]); c11 = dec8(color[r1 + wx1]);
-                const uint32_t ni = (uint32_t)wrapn(nyi, H) * (uint32_t)W + (uint32_t)wrapn(nxi, W);
-                nw = nw_row[face_class(gb_face[ni])];
-            }
-            const float sa = bil(c00, c10, c01, c11, fa, fb);
-            // The weight is ((clamp(pow) * dw) * nw) with pow <= 1 (vpt_expf of a
-            // non-positive argument, checked for every float), so it sits on
-            // its 1e-9 clamp once dw * nw < 1e-9: nw is exactly 0 or 1 here
-            // (axis normals, or (1,1,1) against an axis normal), and
-            // exp(-d)^3 < 1e-9 for every float d >= 21.  Those taps skip the
-            // exp and the pow.
-            float w = 0.000000001f;
-            if (nw != 0.0f) {
-                const float sd = bil(d00, d10, d01, d11, fa, fb);
-                const float dd = fabsf(dist - sd);
-                if (dd < 21.0f) {
-                    const float dw = vpt_powi(expf_nonpos(-dd), 3);
-                    if (dw * nw >= 0.000000001f) {
-                        const float le = fclamp(1.0f - fclamp(div3_unit(fabsf(sa - cs)), 0.0f, 1.0f), 0.0f, 1.0f);
-                        w = 1.0f;
-                        w = w * fclamp(powf_rcp(le, expo), 0.0f, 1.0f);
-                        w = w * dw;
-                        w = w * nw;
-                        w = fclamp(w, 0.000000001f, 1.0f);
-                    }
+    auto tap = [&](float2 q00, float2 q10, float2 q01, float2 q11, float nw, float fa,
+                   float fb) __attribute__((always_inline)) {
+        const float sa = bil(q00.y, q10.y, q01.y, q11.y, fa, fb);
+        float w = 0.000000001f;
+        if (nw != 0.0f) {
+            const float sd = bil(q00.x, q10.x, q01.x, q11.x, fa, fb);
+            const float dd = fabsf(dist - sd);
+            if (dd < 21.0f) {
+                const float dw = vpt_powi(expf_21(-dd), 3);
+                if (dw * nw >= 0.000000001f) {
+                    const float le = fclamp(1.0f - fclamp(div3_unit(fabsf(sa - cs)), 0.0f, 1.0f), 0.0f, 1.0f);
+                    w = 1.0f;
+                    if (le < 1.0f) w = fclamp(expf_21(expo * logf_unit(le)), 0.0f, 1.0f);
+                    w = w * dw;
+                    w = w * nw;
+                    w = fclamp(w, 0.000000001f, 1.0f);
                 }
             }
-            ts = ts + sa * w;
-            tw = tw + w;
+        }
+        ts = ts + sa * w;
+        tw = tw + w;
+    };
+    // GL LINEAR footprint and NEAREST texel, before REPEAT, of the tap's
+    // column or row, relative to the window
+    struct Line {
+        float frac;
+        int lo, near;
+    };
+    auto line = [&](float uv, float tex, int k, int n, int g0) __attribute__((always_inline)) {
+        const float s = uv + (((float)k * tex) * 1.2f * sc) * scale;
+        const float u = s * (float)n - 0.5f;
+        const float fu = floorf(u);
+        return Line{u - fu, (int)fu - g0, (int)floorf(s * (float)n) - g0};
+    };
+    auto in_window = [](const Line& l, int n) __attribute__((always_inline)) {
+        return l.lo >= 0 && l.lo + 1 < n && l.near >= 0 && l.near < n;
+    };
+    // a tap's position is monotonic in k, so the outermost ones decide
+    const bool staged = in_window(line(uvx, tex_w, -size, W, gx0), kSfW) && in_window(line(uvx, tex_w, size, W, gx0), kSfW) &&
+                        in_window(line(uvy, tex_h, -size, H, gy0), kSfH) && in_window(line(uvy, tex_h, size, H, gy0), kSfH);
+    if (__all(staged)) {
+        Line row[7];
+#pragma unroll
+        for (int k = 0; k < 7; k++) {
+            row[k] = line(uvy, tex_h, k - 3, H, gy0);
+            row[k].lo = __mul24(row[k].lo, kSfW);
+            row[k].near = __mul24(row[k].near, kSfW);
+        }
+        for (int x = -size; x <= size; x++) {
+            const Line col = line(uvx, tex_w, x, W, gx0);
+#pragma unroll
+            for (int k = 0; k < 7; k++) {
+                if (k - 3 < -size || k - 3 > size) continue;
+                const float2* q = s_dc + row[k].lo + col.lo;
+                tap(q[0], q[1], q[kSfW], q[kSfW + 1], nw_row[s_f[row[k].near + col.near]], col.frac, row[k].frac);
+            }
+        }
+    } else {
+        for (int x = -size; x <= size; x++) {
+            const Line col = line(uvx, tex_w, x, W, gx0);
+            for (int y = -size; y <= size; y++) {
+                const Line row = line(uvy, tex_h, y, H, gy0);
+                if (in_window(col, kSfW) && in_window(row, kSfH)) {
+                    const float2* q = s_dc + row.lo * kSfW + col.lo;
+                    tap(q[0], q[1], q[kSfW], q[kSfW + 1], nw_row[s_f[row.near * kSfW + col.near]], col.frac, row.frac);
+                } else {
+                    const uint32_t c0 = (uint32_t)wrapn(col.lo + gx0, W), c1 = (uint32_t)wrapn(col.lo + gx0 + 1, W);
+                    const uint32_t r0 = (uint32_t)wrapn(row.lo + gy0, H) * (uint32_t)W;
+                    const uint32_t r1 = (uint32_t)wrapn(row.lo + gy0 + 1, H) * (uint32_t)W;
+                    const uint32_t n = (uint32_t)wrapn(row.near + gy0, H) * (uint32_t)W + (uint32_t)wrapn(col.near + gx0, W);
+                    tap(make_float2(gb_t[r0 + c0], dec8(color[r0 + c0])), make_float2(gb_t[r0 + c1], dec8(color[r0 + c1])),
+                        make_float2(gb_t[r1 + c0], dec8(color[r1 + c0])), make_float2(gb_t[r1 + c1], dec8(color[r1 + c1])),
+                        nw_row[face_class(gb_face[n])], col.frac, row.frac);
+                }
+            }
         }
     }
     out[i] = vpt_unorm8_encode(ts / fmaxf(tw, 0.01f));
