@@ -20,3 +20,13 @@ def test_div3_unit_equals_division_on_0_2(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout
     assert r.stdout.strip().endswith("0 mismatches")
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="needs gcc")
+def test_denoiser_exp_and_log_equal_the_full_ones(tmp_path):
+    exe = tmp_path / "exp_log_check"
+    subprocess.run(["gcc", "-O2", "-ffp-contract=off", "-mfma", "-I", str(HERE.parent / "include"),
+                    str(HERE / "native" / "exp_log_check.c"), "-o", str(exe), "-lm"], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout
+    assert r.stdout.strip().endswith("0 mismatches")

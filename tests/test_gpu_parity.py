@@ -421,6 +421,15 @@ def test_svgf_parity_small(ctx, terrain_world):
     _assert_exact(res)
 
 
+@pytest.mark.parametrize("W,H", [(2, 2), (5, 3), (33, 9), (70, 41)])
+def test_svgf_parity_ragged(ctx, terrain_world, W, H):
+    """Images smaller than a tile and its 9x9 apron, and ones a tile does not
+    divide: taps off the image in every pass; bit-exact."""
+    g, df, w = terrain_world
+    res, _, _ = _run_svgf(ctx, w, g, df, W, H, 3)
+    _assert_exact(res)
+
+
 def test_svgf_parity_steady_state(ctx, terrain_world):
     """24 frames of the SVGF camera path at 640x360, every plane bit-exact on
     every frame, with the oracle's state shown to reach the long-history

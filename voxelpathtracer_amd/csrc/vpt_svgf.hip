@@ -168,10 +168,10 @@ __device__ inline Bil bil_setup(float s, float t, int W, int H)
     return b;
 }
 
-// vpt_expf for -21 <= x <= 0: the same polynomial; kf has at most five bits
-// and LN2_HI eight, so their product is exact and the subtraction one fma; the
-// scaling by 2^k, k >= -31, is exact in one step.
-__device__ inline float expf_21(float x)
+// vpt_expf for -32 <= x <= 0: the same polynomial; kf has at most seven bits
+// (for x down to -88) and LN2_HI eight, so their product is exact and the
+// subtraction one fma; the scaling by 2^k, k >= -46, is exact in one step.
+__device__ inline float expf_32(float x)
 {
     const float LOG2E = 1.44269502162933349609375f;
     const float LN2_HI = 0.693145751953125f;
@@ -189,33 +189,12 @@ __device__ inline float expf_21(float x)
     return __builtin_ldexpf(p, (int)kf);
 }
 
-// vpt_expf for arguments x <= 0, which the sun-shadow weights pass: the
-// same operations, so the same results, without the NaN and overflow tests
-// (they cannot fire) and with the underflow test (x below -87.34 gives 0) as
-// a select instead of a branch.  (In the SVGF passes the branch form was as
-// fast or faster.)
-__device__ inline float expf_nonpos(float x)
+// vpt_expf for x <= 0, where it is 0 below -87.34; above, p 2^k is rounded at
+// most once, in either form of the scaling.
+__device__ inline float expf_down(float x)
 {
-    const float LOG2E = 1.44269502162933349609375f;
-    const float LN2_HI = 0.693145751953125f;
-    const float LN2_LO = 1.428606765330187045e-06f;
-    const float kf = floorf(x * LOG2E + 0.5f);
-    float r = x - kf * LN2_HI;
-    r = r - kf * LN2_LO;
-    float p = 0.0013829420786350965f;
-    p = p * r + 0.008374771103262901f;
-    p = p * r + 0.0416683591902256f;
-    p = p * r + 0.1666642129421234f;
-    p = p * r + 0.49999991059303284f;
-    p = p * r + 1.0f;
-    p = p * r + 1.0f;
-    const int k = (int)fmaxf(kf, -300.0f);   // kf >= -126 wherever the result is used
-    const int k1 = k / 2;
-    const int k2 = k - k1;
-    const float s1 = vpt_u2f((uint32_t)(k1 + 127) << 23);
-    const float s2 = vpt_u2f((uint32_t)(k2 + 127) << 23);
-    const float v = (p * s1) * s2;
-    return x < -87.33654022216796875f ? 0.0f : v;
+    const float e = expf_32(fmaxf(x, -88.0f));
+    return x < -87.33654022216796875f ? 0.0f : e;
 }
 
 __device__ inline float bil(float t00, float t10, float t01, float t11, float a, float b)
@@ -624,6 +603,7 @@ __global__ void __launch_bounds__(256) temporal_kernel(CamView cam, Mat16 prev_v
 // the same float additions.  The moment does not enter the weights: when
 // only it differs between cells, the moment sum alone walks the taps.
 constexpr int kVarR = 4;
+constexpr int kVarGroup = 3;   // taps whose weights are worked out together (9: the same time, 63 registers for 46)
 constexpr int kVarSW = 32 + 2 * kVarR, kVarSH = 8 + 2 * kVarR, kVarCells = kVarSW * kVarSH;
 
 __device__ inline int normal_index(uint32_t face) { return face <= 5u ? (int)face : 6; }
@@ -782,46 +762,50 @@ __global__ void __launch_bounds__(256) variance_kernel(int W, int H, const float
             tlum = s_tab[8][k];
         } else
         for (int x = -4; x <= 4; x++) {
-            for (int y = -4; y <= 4; y++) {
-                float sx = uvx + (float)x * tex_w;
-                float sy = uvy + (float)y * tex_h;
-                if (!in_screen(sx, sy)) continue;   // exactly the taps inside the image
-                const int c = (ly + kVarR + y) * kVarSW + (lx + kVarR + x);
-                const float sw = s_t[c];
-                const float nw = nw_row[s_n[c]];
-                const float4 a = s_aux[c];
-                const float4 sh = s_sh[c];
-                const float slum = a.z, smom = a.w;
-                // vpt_expf of a non-positive argument lies in [0, 1] (checked
-                // for every float), so a zero normal weight makes the product
-                // exactly 0.  At a depth gap of 25 or more the product is below
-                // exp(-50) * 3^16 < 1.5e-9 (3^16 is the largest normal weight,
-                // sky against sky), under both clamps below, so it is taken as
-                // 0 without evaluating the exps.  vpt_expf(-0) is exactly 1.
-                float w = 0.0f;
-                const float dd = fabsf(sw - base_w);
-                if (nw != 0.0f && dd < 25.0f) {
-                    float e = 1.0f;
-                    if (dd != 0.0f) e = vpt_expf(-dd);
-                    float dw = e * e;
-                    float lw = fabsf(slum - base_lum) / color_phi;
-                    float el = 1.0f;
-                    if (lw != 0.0f) el = vpt_expf(-lw);
-                    w = (el * nw) * dw;
+            if ((uint32_t)(px + x) >= (uint32_t)W) continue;
+            const int c0 = ly * kVarSW + (lx + kVarR + x);
+#pragma unroll
+            for (int g = 0; g < 9; g += kVarGroup) {
+                // the group's weights first, so that their exps overlap; at
+                // 1920x1080 an SVGF frame 725 -> 708 us, a pipeline frame
+                // 1214 -> 1191 us and at 320x180 276 -> 272 us, the cheaper
+                // exp and division by 5 included
+                float w[kVarGroup];
+#pragma unroll
+                for (int y = 0; y < kVarGroup; y++) {
+                    const int c = c0 + (g + y) * kVarSW;
+                    const float nw = nw_row[s_n[c]];
+                    // vpt_expf of a non-positive argument lies in [0, 1]
+                    // (checked for every float), so at a depth gap of 25 or
+                    // more the product is below exp(-50) * 3^16 < 1.5e-9 (3^16
+                    // is the largest normal weight, sky against sky), under
+                    // both clamps below, and is taken as 0.
+                    const float dd = fabsf(s_t[c] - base_w);
+                    const float e = expf_32(-fminf(dd, 32.0f));
+                    const float lw = div_rcp(fabsf(s_aux[c].z - base_lum), color_phi, 1.0f / color_phi);
+                    const float el = expf_down(-lw);
+                    w[y] = nw != 0.0f && dd < 25.0f ? (el * nw) * (e * e) : 0.0f;
                 }
-                float w2 = w;
-                w = fmaxf(w, 0.000000015f);
-                w2 = fmaxf(w2, 0.0000000015f);
-                tw = tw + w;
-                tmom = tmom + smom * w2;
-                tsh[0] = tsh[0] + sh.x * w;
-                tsh[1] = tsh[1] + sh.y * w;
-                tsh[2] = tsh[2] + sh.z * w;
-                tsh[3] = tsh[3] + sh.w * w;
-                tco = tco + a.x * w;
-                tcg = tcg + a.y * w;
-                tlum = tlum + slum * w2;
-                tw2 = tw2 + w2;
+#pragma unroll
+                for (int y = 0; y < kVarGroup; y++) {
+                    if ((uint32_t)(py + g + y - 4) >= (uint32_t)H) continue;   // exactly the taps inside the image
+                    const int c = c0 + (g + y) * kVarSW;
+                    const float4 a = s_aux[c];
+                    const float4 sh = s_sh[c];
+                    const float slum = a.z, smom = a.w;
+                    const float w1 = fmaxf(w[y], 0.000000015f);
+                    const float w2 = fmaxf(w[y], 0.0000000015f);
+                    tw = tw + w1;
+                    tmom = tmom + smom * w2;
+                    tsh[0] = tsh[0] + sh.x * w1;
+                    tsh[1] = tsh[1] + sh.y * w1;
+                    tsh[2] = tsh[2] + sh.z * w1;
+                    tsh[3] = tsh[3] + sh.w * w1;
+                    tco = tco + a.x * w1;
+                    tcg = tcg + a.y * w1;
+                    tlum = tlum + slum * w2;
+                    tw2 = tw2 + w2;
+                }
             }
         }
         if (tw > 0.0f) {
@@ -1307,11 +1291,11 @@ __global__ void __launch_bounds__(256) shadow_temporal_kernel(CamView cam, Mat16
                                  h2f(hist_frames[f.i11]), f.a, f.b);
             const float fi = fc + inc;
             float bf = fclamp((1.0f - (1.0f / fi)) * 1.2f, 0.01f, 0.97f);
-            const float vr = fclamp(expf_nonpos(-sqrtf(vx * vx + vy * vy)) * 0.8f + 0.6f, 0.00000001f, 1.0f);
+            const float vr = fclamp(expf_down(-sqrtf(vx * vx + vy * vy)) * 0.8f + 0.6f, 0.00000001f, 1.0f);
             bf = bf * vr;
             float dr = 1.0f;
             if (d > 0.4f) {
-                dr = vpt_powi(expf_nonpos(-d), 48);
+                dr = vpt_powi(expf_down(-d), 48);
                 bf = bf * fclamp(dr, 0.0f, 1.0f);
             }
             const float a = fclamp(bf, 0.0f, 0.97f);
@@ -1449,11 +1433,11 @@ __global__ void __launch_bounds__(256) shadow_filter_kernel(int W, int H, const 
             const float sd = bil(q00.x, q10.x, q01.x, q11.x, fa, fb);
             const float dd = fabsf(dist - sd);
             if (dd < 21.0f) {
-                const float dw = vpt_powi(expf_21(-dd), 3);
+                const float dw = vpt_powi(expf_32(-dd), 3);
                 if (dw * nw >= 0.000000001f) {
                     const float le = fclamp(1.0f - fclamp(div3_unit(fabsf(sa - cs)), 0.0f, 1.0f), 0.0f, 1.0f);
                     w = 1.0f;
-                    if (le < 1.0f) w = fclamp(expf_21(expo * logf_unit(le)), 0.0f, 1.0f);
+                    if (le < 1.0f) w = fclamp(expf_32(expo * logf_unit(le)), 0.0f, 1.0f);
                     w = w * dw;
                     w = w * nw;
                     w = fclamp(w, 0.000000001f, 1.0f);
