@@ -432,7 +432,7 @@ VPT_API int vpt_trace_rays(vpt_world* w, const vpt_ray* d_rays, int n, int max_i
  * DiffuseRayTraceFrag.glsl:1202-1222 is used by CalculateDiffuse (:535-664).
  * d_hits[i] = the bounce's hit; d_vis[i] = 1 when the sun is blocked at the
  * hit, 0 when it is visible, 255 when no shadow ray was traced (miss, or
- * N.L < 0.001).  Two one-launch kernels (bounce, then shadow). */
+ * N.L < 0.001).  One launch. */
 VPT_API int vpt_trace_gi_rays(vpt_world* w, const vpt_ray* d_rays, int n, int gi_iter, const float sun_dir[3],
                               int shadow_iter, vpt_hit* d_hits, uint8_t* d_vis, void* stream);
 
