@@ -135,6 +135,9 @@ class Server:
                 vis = torch.empty(n, dtype=torch.uint8, device="cuda")
                 _copy(vis, res.d_vis or 0, n)
                 out["vis"] = vis
+        # a copy within the device returns before it has run, and the results'
+        # memory may be another request's as soon as the caller releases it
+        torch.cuda.default_stream().synchronize()
         return out
 
     def release(self, ticket: int) -> None:
