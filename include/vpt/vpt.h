@@ -528,8 +528,8 @@ VPT_API int vpt_frame_autotune(vpt_frame* f, vpt_world* w, const vpt_camera* cam
  * Results live in server memory until vpt_server_release.  A request's
  * d_rays must hold its rays when it is submitted (the work producing them
  * has completed) and stay valid until the request completes.  The server
- * runs on its own non-blocking stream.  Submit / wait / release may be
- * called from any threads. */
+ * runs on its own non-blocking stream.  Submit / wait / fetch / release may
+ * be called from any threads. */
 typedef struct vpt_server vpt_server;
 
 enum { VPT_SERVE_PLAIN = 0, VPT_SERVE_BATCHED = 1 };
@@ -595,7 +595,14 @@ VPT_API int vpt_server_submit(vpt_server* s, const vpt_request* req, uint64_t* t
 /* Blocks until the request completes (timeout_ms < 0: no limit) and fills
  * *res; VPT_ETIMEOUT if it has not completed in time. */
 VPT_API int vpt_server_wait(vpt_server* s, uint64_t ticket, int timeout_ms, vpt_request_result* res);
-/* Frees a completed request's result memory (the ticket becomes invalid). */
+/* Copies a completed request's results into the non-null arrays of dst (in
+ * device memory, of the sizes vpt_server_wait's result has them) by work on
+ * `stream`, without waiting for it.  A release gives the memory back only
+ * once that work has run.  VPT_ESTATE before the request has completed;
+ * VPT_EINVAL on a stream that is being captured. */
+VPT_API int vpt_server_fetch(vpt_server* s, uint64_t ticket, const vpt_request_result* dst, void* stream);
+/* Frees a completed request's result memory (the ticket becomes invalid).
+ * Copies that the caller made by other means must have run. */
 VPT_API int vpt_server_release(vpt_server* s, uint64_t ticket);
 VPT_API int vpt_server_stats_get(vpt_server* s, vpt_server_stats* st);
 

@@ -212,6 +212,67 @@ def test_admission_waits_for_memory(ctx, scene):
     srv.close()
 
 
+@pytest.mark.parametrize("side", [False, True])
+def test_release_waits_for_the_copies(ctx, scene, side):
+    """Results fetched behind other work of the caller's stream and released
+    at once, with an arena that holds two of the six requests: their memory
+    goes to a waiting request only after the copies, which are right."""
+    torch = _torch()
+    grids, worlds, reqs = scene
+    mix = [reqs[i] for i in (7, 5, 7, 5, 7, 5)]   # 150K GI rays and 200K shadow rays, of different worlds
+    srv = Server(ctx, mode="batched", max_worlds=4, arena_bytes=200_000 * 12 + 150_000 * 13 + 1024)
+    slots = [srv.add_world(w) for w in worlds]
+    stream = torch.cuda.Stream() if side else torch.cuda.default_stream()
+    a = torch.rand((4096, 4096), device="cuda")
+    torch.cuda.synchronize()
+    tickets = [_submit(srv, slots, r) for r in mix]
+    outs, held = [], 0
+    with torch.cuda.stream(stream):
+        for k, t in enumerate(tickets):
+            for _ in range(20):
+                b = a @ a   # milliseconds before the copies can run
+            outs.append(srv.fetch(t))
+            srv.release(t)
+            waiting = srv.stats()["pending"]
+            if not stream.query():   # the copies had not all run when `waiting` was read
+                assert waiting >= len(mix) - 2 - k
+                held += waiting > 0
+        ready = [{n: v.clone() for n, v in o.items() if torch.is_tensor(v)} for o in outs]
+    stream.synchronize()
+    for r, o in zip(mix, ready):
+        _check(r, o)
+    assert held > 0
+    st = srv.stats()
+    assert st["completed"] == len(mix) and st["arena_used"] == 0 and st["arena_peak"] <= st["arena_bytes"]
+    del b
+    srv.close()
+
+
+def test_fetch_arguments(ctx, scene):
+    import ctypes as C
+    from voxelpathtracer_amd import _lib
+    from voxelpathtracer_amd._lib import VPT_EINVAL, RequestResult
+    torch = _torch()
+    grids, worlds, reqs = scene
+    srv = Server(ctx, mode="batched", max_worlds=2)
+    slot = srv.add_world(worlds[0])
+    r = reqs[3]
+    t = srv.submit_rays(slot, r["kind"], r["dev"], r["n"], r["max_iter"], SUN, 128)
+    first, again = srv.fetch(t), srv.fetch(t)   # twice, and into only one of the arrays
+    _check(r, first)
+    _check(r, again)
+    dst = RequestResult()
+    vis = torch.full((r["n"],), 7, dtype=torch.uint8, device="cuda")
+    dst.d_vis = vis.data_ptr()
+    _lib.call("vpt_server_fetch", srv.handle, C.c_uint64(t), C.byref(dst), None)
+    np.testing.assert_array_equal(vis.cpu().numpy(), r["ref_vis"])
+    srv.release(t)
+    with pytest.raises(VptError) as e:
+        srv.fetch(t)
+    assert e.value.code == VPT_EINVAL
+    srv.close()
+
+
 def test_world_slots_and_errors(ctx, scene):
     grids, worlds, reqs = scene
     srv = Server(ctx, mode="batched", max_worlds=2, world_budget=1 << 40)

@@ -202,6 +202,7 @@ _PROTOS = {
     "vpt_server_set_launch_cfg": (_i, [_vp, C.POINTER(LaunchCfg)]),
     "vpt_server_submit": (_i, [_vp, C.POINTER(Request), C.POINTER(C.c_uint64)]),
     "vpt_server_wait": (_i, [_vp, C.c_uint64, _i, C.POINTER(RequestResult)]),
+    "vpt_server_fetch": (_i, [_vp, C.c_uint64, C.POINTER(RequestResult), _vp]),
     "vpt_server_release": (_i, [_vp, C.c_uint64]),
     "vpt_server_stats_get": (_i, [_vp, C.POINTER(ServerStats)]),
     "vpt_unet_create": (_i, [_vp, _i, _i, _i, C.POINTER(_vp)]),

@@ -112,6 +112,9 @@ struct Req {
     State state = State::PENDING;
     int status = VPT_OK;
     vpt_request_result res{};
+    std::vector<hipEvent_t> reads;   // after each fetch's copies, on the caller's streams
+    int fetching = 0;                // fetches that are queueing their copies
+    bool released = false;
 };
 
 struct Part {
@@ -203,6 +206,8 @@ struct vpt_server {
     std::deque<Req*> pending;                 // arrival order
     std::vector<Req*> admitted;               // admission order, not yet completed
     std::unordered_map<uint64_t, Req*> reqs;
+    std::vector<Req*> returning;              // released, their results' copies not known to have run
+    size_t returning_bytes = 0;
     std::deque<Launch> inflight;
     uint64_t next_ticket = 1;
     bool stop = false;
@@ -211,7 +216,42 @@ struct vpt_server {
 
     vpt_server_stats st{};
 
+    // A released request that no fetch is working on: its memory is free at
+    // once, or, where copies of it were queued, when they have run (reclaim).
+    // Waiting for them in fetch costs the caller 8 us a request (a wave of 24
+    // requests of 1K to 2M rays: 975 us, 773 in this form), and an order on
+    // the device would make launches wait for the caller's stream.
+    void give_back(Req* q)
+    {
+        if (!q->reads.empty()) {
+            returning.push_back(q);
+            returning_bytes += q->bytes;
+            return;
+        }
+        if (q->units) arena.release(q->off, q->bytes);
+        delete q;
+    }
+
     // ---- worker ------------------------------------------------------------
+
+    void reclaim()
+    {
+        for (size_t i = 0; i < returning.size();) {
+            Req* q = returning[i];
+            while (!q->reads.empty() && hipEventQuery(q->reads.back()) != hipErrorNotReady) {
+                (void)hipEventDestroy(q->reads.back());
+                q->reads.pop_back();
+            }
+            if (!q->reads.empty()) {
+                i++;
+                continue;
+            }
+            returning_bytes -= q->bytes;
+            returning[i] = returning.back();
+            returning.pop_back();
+            give_back(q);
+        }
+    }
 
     void admit()
     {
@@ -475,6 +515,7 @@ struct vpt_server {
                 if (e == hipErrorNotReady) break;
                 retire_front(e == hipSuccess ? VPT_OK : VPT_EDEVICE);
             }
+            reclaim();
             admit();
             if (cfg.mode == VPT_SERVE_PLAIN) {
                 Req* q = nullptr;
@@ -515,7 +556,9 @@ struct vpt_server {
                     continue;
                 }
             }
-            if (stop && admitted.empty() && inflight.empty()) {
+            // requests that wait for memory which is about to come back
+            const bool awaiting = !pending.empty() && !returning.empty();
+            if (stop && admitted.empty() && inflight.empty() && !awaiting) {
                 // shutting down: what cannot be admitted any more fails
                 while (!pending.empty()) {
                     Req* q = pending.front();
@@ -536,6 +579,9 @@ struct vpt_server {
                     woken = false;
                     cv_work.wait_for(lk, std::chrono::microseconds(20), [this] { return woken; });
                 }
+            } else if (awaiting) {
+                woken = false;
+                cv_work.wait_for(lk, std::chrono::microseconds(20), [this] { return woken; });
             } else {
                 woken = false;
                 cv_work.wait(lk, [this] { return woken || stop; });
@@ -564,7 +610,14 @@ extern "C" VPT_API int vpt_server_destroy(vpt_server* s)
         s->worker.join();
     }
     DeviceGuard g(s->device);
-    for (auto& kv : s->reqs) delete kv.second;
+    for (auto& kv : s->reqs) s->returning.push_back(kv.second);
+    for (Req* q : s->returning) {
+        for (hipEvent_t e : q->reads) {
+            (void)hipEventSynchronize(e);   // the copies read the arena
+            (void)hipEventDestroy(e);
+        }
+        delete q;
+    }
     for (auto& kv : s->frames) vpt_frame_destroy(kv.second);
     for (Slot& sl : s->slots) {
         (void)hipFree(sl.d_segs);
@@ -790,6 +843,67 @@ extern "C" VPT_API int vpt_server_wait(vpt_server* s, uint64_t ticket, int timeo
     return VPT_OK;
 }
 
+extern "C" VPT_API int vpt_server_fetch(vpt_server* s, uint64_t ticket, const vpt_request_result* dst, void* stream)
+{
+    if (!s || !dst) return set_error(VPT_EINVAL, "vpt_server_fetch: null argument");
+    const hipStream_t st = (hipStream_t)stream;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
+        return set_error(VPT_EINVAL, "vpt_server_fetch: the stream is being captured");
+    Req* q = nullptr;
+    {
+        std::lock_guard<std::mutex> lk(s->mu);
+        auto it = s->reqs.find(ticket);
+        if (it == s->reqs.end())
+            return set_error(VPT_EINVAL, "vpt_server_fetch: unknown ticket %llu", (unsigned long long)ticket);
+        q = it->second;
+        if (q->state != State::DONE)
+            return set_error(VPT_ESTATE, "vpt_server_fetch: request %llu has not completed", (unsigned long long)ticket);
+        if (q->status)
+            return set_error(q->status, "vpt_server_fetch: request %llu failed", (unsigned long long)ticket);
+        q->fetching++;   // a release meanwhile leaves the request to us
+    }
+    const vpt_request_result& r = q->res;
+    const size_t n = q->units;
+    const struct {
+        void* to;
+        const void* from;
+        size_t bytes;
+    } parts[] = {{dst->d_hits, r.d_hits, n * sizeof(vpt_hit)},
+                 {dst->d_vis, r.d_vis, n},
+                 {dst->gbuffer.d_t, r.gbuffer.d_t, n * 4},
+                 {dst->gbuffer.d_face, r.gbuffer.d_face, n},
+                 {dst->gbuffer.d_block, r.gbuffer.d_block, n},
+                 {dst->gbuffer.d_voxel, r.gbuffer.d_voxel, n * 4},
+                 {dst->d_mask, r.d_mask, n},
+                 {dst->d_rgb, r.d_rgb, n * 12}};
+    hipEvent_t ev = nullptr;
+    hipError_t e = hipSuccess;
+    if (n) {
+        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        for (const auto& p : parts)
+            if (e == hipSuccess && p.to && p.from)
+                e = hipMemcpyAsync(p.to, p.from, p.bytes, hipMemcpyDeviceToDevice, st);
+        if (e == hipSuccess) e = hipEventRecord(ev, st);
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(st);   // the copies that were queued
+            if (ev) (void)hipEventDestroy(ev);
+            ev = nullptr;
+        }
+    }
+    {
+        std::lock_guard<std::mutex> lk(s->mu);
+        q->fetching--;
+        if (ev) q->reads.push_back(ev);
+        if (q->released && !q->fetching) {
+            s->give_back(q);
+            s->wake();
+        }
+    }
+    if (e != hipSuccess) return set_error(VPT_EDEVICE, "vpt_server_fetch: copy failed (%s)", hipGetErrorString(e));
+    return VPT_OK;
+}
+
 extern "C" VPT_API int vpt_server_release(vpt_server* s, uint64_t ticket)
 {
     if (!s) return set_error(VPT_EINVAL, "vpt_server_release: null server");
@@ -800,10 +914,10 @@ extern "C" VPT_API int vpt_server_release(vpt_server* s, uint64_t ticket)
     Req* q = it->second;
     if (q->state != State::DONE)
         return set_error(VPT_ESTATE, "vpt_server_release: request %llu has not completed", (unsigned long long)ticket);
-    if (q->units) s->arena.release(q->off, q->bytes);
     s->world_refs[q->r.world]--;
     s->reqs.erase(it);
-    delete q;
+    q->released = true;
+    if (!q->fetching) s->give_back(q);
     s->wake();   // freed memory may admit a waiting request
     return VPT_OK;
 }
@@ -813,7 +927,7 @@ extern "C" VPT_API int vpt_server_stats_get(vpt_server* s, vpt_server_stats* st)
     if (!s || !st) return set_error(VPT_EINVAL, "vpt_server_stats_get: null argument");
     std::lock_guard<std::mutex> lk(s->mu);
     *st = s->st;
-    st->arena_used = s->arena.used;
+    st->arena_used = s->arena.used - s->returning_bytes;
     st->arena_peak = s->arena.peak;
     st->pending = (uint32_t)s->pending.size();
     st->active = (uint32_t)s->admitted.size();

@@ -20,24 +20,6 @@ from .world import Context, World, _ptr
 
 KINDS = {"primary": _lib.VPT_REQ_PRIMARY, "shadow": _lib.VPT_REQ_SHADOW, "gi": _lib.VPT_REQ_GI,
          "frame": _lib.VPT_REQ_FRAME}
-_HIP_MEMCPY_DEFAULT = 4
-_hip = None
-
-
-def _copy(dst_tensor, src_ptr: int, nbytes: int) -> None:
-    """Device-to-device copy of nbytes from a raw device pointer (the
-    caller has synchronised with the producing work)."""
-    global _hip
-    if _hip is None:
-        _hip = C.CDLL("libamdhip64.so")
-        _hip.hipMemcpy.restype = C.c_int
-        _hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
-    if nbytes == 0:
-        return
-    rc = _hip.hipMemcpy(C.c_void_p(dst_tensor.data_ptr()), C.c_void_p(src_ptr), C.c_size_t(nbytes),
-                        _HIP_MEMCPY_DEFAULT)
-    if rc != 0:
-        raise RuntimeError(f"hipMemcpy failed with {rc}")
 
 
 def now_ns() -> int:
@@ -111,7 +93,10 @@ class Server:
         return res
 
     def fetch(self, ticket: int) -> dict:
-        """Waits for the request and copies its results into new cuda tensors."""
+        """Waits for the request and copies its results into new cuda tensors,
+        on the current stream: like other tensors made there, they are ready
+        for later work of that stream.  The request may be released at once;
+        its memory is given to another only when the copies have run."""
         import torch
         res = self.wait(ticket)
         if res.status != 0:
@@ -119,25 +104,26 @@ class Server:
         out = {"t_arrival_ns": res.t_arrival_ns, "t_admit_ns": res.t_admit_ns, "t_start_ns": res.t_start_ns,
                "t_done_ns": res.t_done_ns}
         n = res.n
+        dst = RequestResult()
+
+        def new(name: str, dtype, count: int) -> int:
+            out[name] = torch.empty(count, dtype=dtype, device="cuda")
+            return out[name].data_ptr()
+
         if res.kind == _lib.VPT_REQ_FRAME:
-            for name, ptr, dt, per in (("t", res.gbuffer.d_t, torch.float32, 1), ("face", res.gbuffer.d_face,
-                                       torch.uint8, 1), ("block", res.gbuffer.d_block, torch.uint8, 1),
-                                       ("voxel", res.gbuffer.d_voxel, torch.int32, 1),
-                                       ("mask", res.d_mask, torch.uint8, 1), ("rgb", res.d_rgb, torch.float32, 3)):
-                t = torch.empty(n * per, dtype=dt, device="cuda")
-                _copy(t, ptr, t.numel() * t.element_size())
-                out[name] = t
+            gb = dst.gbuffer
+            gb.d_t = new("t", torch.float32, n)
+            gb.d_face = new("face", torch.uint8, n)
+            gb.d_block = new("block", torch.uint8, n)
+            gb.d_voxel = new("voxel", torch.int32, n)
+            dst.d_mask = new("mask", torch.uint8, n)
+            dst.d_rgb = new("rgb", torch.float32, 3 * n)
         else:
-            hits = torch.empty(n * 12, dtype=torch.uint8, device="cuda")
-            _copy(hits, res.d_hits or 0, n * 12)
-            out["hits"] = hits
+            dst.d_hits = new("hits", torch.uint8, 12 * n)
             if res.kind == _lib.VPT_REQ_GI:
-                vis = torch.empty(n, dtype=torch.uint8, device="cuda")
-                _copy(vis, res.d_vis or 0, n)
-                out["vis"] = vis
-        # a copy within the device returns before it has run, and the results'
-        # memory may be another request's as soon as the caller releases it
-        torch.cuda.default_stream().synchronize()
+                dst.d_vis = new("vis", torch.uint8, n)
+        call("vpt_server_fetch", self.handle, C.c_uint64(ticket), C.byref(dst),
+             C.c_void_p(torch.cuda.current_stream().cuda_stream))
         return out
 
     def release(self, ticket: int) -> None:
