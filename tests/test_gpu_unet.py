@@ -211,6 +211,60 @@ def test_denoise_activations(ctx, h, w):
     world.close()
 
 
+def test_last_activation(ctx):
+    """The last activation, which an inference pass does not store, read in
+    parts and again, after the weights changed, and after replays of a
+    captured pass of another size: always the values that a pass which stores
+    it (the backward pass) has with the same weights, bit for bit."""
+    torch = _torch()
+    rng = np.random.default_rng(71)
+    n, h, w = 3, 16, 20
+    x = {k: torch.from_numpy(_inputs(rng, *k)[0].view(np.int16)).cuda() for k in ((n, h, w), (2, 12, 36))}
+    tgt = {k: torch.zeros(k + (3,), device="cuda") for k in x}
+    out = {k: torch.empty(k + (3,), device="cuda") for k in x}
+    small = (2, 12, 36)
+    u = UNet(ctx, n, h, 64)
+    u.init(3)
+    want = {}
+    for k in x:
+        u.backward(x[k], tgt[k], *k)
+        want[k] = u.activation(12, *k)
+    u.backward(x[n, h, w], tgt[n, h, w], n, h, w)   # gradients for the steps below
+
+    u.forward(x[n, h, w], n, h, w, out[n, h, w])
+    one = u.activation(12, 1, h, w)
+    np.testing.assert_array_equal(one, want[n, h, w][:1])
+    np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])
+    tall = u.activation(12, 1, n * h, w)            # the same values under another shape
+    np.testing.assert_array_equal(tall.ravel(), want[n, h, w].ravel())
+    np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])
+
+    u.forward(x[n, h, w], n, h, w, out[n, h, w])
+    params = u.get_params()
+    u.adam_step(0.05)
+    np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])
+    u.set_params(params)
+
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        u.forward(x[small], *small, out[small])
+    u.forward(x[n, h, w], n, h, w, out[n, h, w])
+    np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])   # recorded, not run
+    for _ in range(3):
+        graph.replay()
+        np.testing.assert_array_equal(u.activation(12, *small), want[small])
+        u.forward(x[n, h, w], n, h, w, out[n, h, w])
+        np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])
+        graph.replay()
+        u.adam_step(0.05)
+        np.testing.assert_array_equal(u.activation(12, *small), want[small])
+        u.set_params(params)
+    del graph
+    u.close()
+
+
 def test_training_beats_input(ctx, net):
     """Tracer-rendered pairs (1 spp -> 64 spp at 64x64), 150 Adam steps: the
     loss falls and the network beats its own 1-spp input on held-out pairs."""

@@ -85,6 +85,15 @@ __device__ inline uint32_t mask_pair(uint32_t v, uint32_t m)
 
 constexpr int kCi = 32;            // input channels per K slice
 
+// What the last forward pass left in the activation buffers, written by its
+// kernels, so that it also holds for replays of a captured pass.
+struct LastPass {
+    int x16;             // act[X] holds 16 channels per pixel (vpt_unet_denoise), not 32
+    int n, h, w;         // the pass's sizes where its D0B was not stored (n = 0: it was)
+    float bias[32];      // then also the last layer's parameters as the pass read them
+    uint16_t w_[9 * 32 * 32];
+};
+
 struct ConvArgs {
     const uint16_t* a;   // input A, NHWC with ca channels (half resolution when a_up)
     const uint16_t* b;   // concatenated input B, NHWC with cb channels (full resolution)
@@ -100,7 +109,7 @@ struct ConvArgs {
     int head_exp;        // head_out = max(exp(.) - 1, 0)
     int ca, cb, a_up, relu;
     int a16;             // input A holds only its first 16 channels (the others are zero)
-    int* a16_out;        // a16 is noted here, or null
+    LastPass* pass;      // the first layer notes a16 here, the last one the rest; or null
     int n, h, w_, cout;
     int near;            // 32-bit byte offsets reach over a tile's halo
 };
@@ -468,7 +477,23 @@ __global__ void __launch_bounds__(64 * WR * WC) conv3x3_kernel(ConvArgs p)
             }
         }
     };
-    if (p.a16_out && blockIdx.x == 0 && threadIdx.x == 0) *p.a16_out = p.a16;
+    if (p.pass && blockIdx.x == 0) {
+        if (!kHead) {
+            if (threadIdx.x == 0) p.pass->x16 = p.a16;
+        } else {
+            if (threadIdx.x == 0) {
+                p.pass->n = p.y ? 0 : p.n;
+                p.pass->h = p.h;
+                p.pass->w = p.w_;
+            }
+            if (!p.y) {
+                if (threadIdx.x < COUT) p.pass->bias[threadIdx.x] = p.bias[threadIdx.x];
+                const uint32_t* from = reinterpret_cast<const uint32_t*>(p.w);
+                uint32_t* to = reinterpret_cast<uint32_t*>(p.pass->w_);
+                for (int i = (int)threadIdx.x; i < 9 * COUT * kCi / 2; i += 64 * NW) to[i] = from[i];
+            }
+        }
+    }
     {
         aim((int)blockIdx.x, 0);
 #pragma unroll
@@ -1116,8 +1141,7 @@ struct vpt_unet {
     float* d_head_part = nullptr;
     int slices = 0;
     int adam_t = 0;
-    int* d_x16 = nullptr;        // act[X] holds 16 channels per pixel (vpt_unet_denoise), not 32
-    int last_n = 0, last_h = 0, last_w = 0;   // the last forward pass, while its D0B is not stored (last_n 0: it is)
+    LastPass* d_pass = nullptr;
     float last_loss = 0.0f;
 };
 
@@ -1159,16 +1183,18 @@ ConvArgs conv_args(vpt_unet* u, const Layer& L, int n, int h, int w)
 
 // The network from act[X] to `out` (exp: irradiance, else log space).  The
 // last layer's activation is stored only when keep_last is set (the backward
-// pass reads it); read_activation makes it again from the layer before.
+// pass reads it): vpt_unet_read_activation makes it from the layer before
+// and the parameters in LastPass.
 int forward(vpt_unet* u, int n, int h, int w, bool x16, bool keep_last, float* out, bool exp, hipStream_t s)
 {
     for (int l = 0; l < kLayers; l++) {
         ConvArgs a = conv_args(u, u->net[l], n, h, w);
         if (l == 0) {
             a.a16 = x16;
-            a.a16_out = u->d_x16;
+            a.pass = u->d_pass;
         }
         if (l == kLayers - 1) {
+            a.pass = u->d_pass;
             a.head_w = u->d_w + u->head_w;
             a.head_b = u->d_w + u->head_b;
             a.head_out = out;
@@ -1177,27 +1203,6 @@ int forward(vpt_unet* u, int n, int h, int w, bool x16, bool keep_last, float* o
         }
         if (int rc = launch_conv(a, s)) return rc;
     }
-    u->last_n = keep_last ? 0 : n;
-    u->last_h = h;
-    u->last_w = w;
-    return VPT_OK;
-}
-
-// Stores the last forward pass's D0B, if it was not, from its D0A: before
-// the weights change, and when it is read.
-int make_last(vpt_unet* u, int n, int h, int w, hipStream_t s)
-{
-    if (!u->last_n) return VPT_OK;
-    u->last_n = 0;
-    return launch_conv(conv_args(u, u->net[kLayers - 1], n, h, w), s);
-}
-
-// A captured pass stores everything, since its replays cannot be known here.
-int is_capturing(hipStream_t s, bool* out)
-{
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    HIP_TRY(hipStreamIsCapturing(s, &cs));
-    *out = cs != hipStreamCaptureStatusNone;
     return VPT_OK;
 }
 
@@ -1345,10 +1350,6 @@ struct DeviceGuard {
 
 int unet_upload(vpt_unet* u, const float* host)
 {
-    if (u->last_n) {
-        HIP_TRY(hipDeviceSynchronize());
-        if (int rc = make_last(u, u->last_n, u->last_h, u->last_w, nullptr)) return rc;
-    }
     HIP_TRY(hipMemcpy(u->d_w, host, sizeof(float) * u->n_params, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks_for(u->n_params)), dim3(256), 0, nullptr, u->d_w, u->d_wb,
                        u->n_params);
@@ -1382,7 +1383,7 @@ extern "C" VPT_API int vpt_unet_destroy(vpt_unet* u)
     (void)hipFree(u->d_gpool[1]);
     (void)hipFree(u->d_pred);
     (void)hipFree(u->d_zero);
-    (void)hipFree(u->d_x16);
+    (void)hipFree(u->d_pass);
     (void)hipFree(u->d_part);
     (void)hipFree(u->d_head_part);
     delete u;
@@ -1440,11 +1441,11 @@ extern "C" VPT_API int vpt_unet_create(vpt_ctx* ctx, int max_n, int max_h, int m
     alloc((void**)&u->d_gpool[1], sizeof(uint16_t) * (full >> 4) * 64);
     alloc((void**)&u->d_pred, sizeof(float) * full * 3);
     alloc((void**)&u->d_zero, 1024);
-    alloc((void**)&u->d_x16, sizeof(int));
+    alloc((void**)&u->d_pass, sizeof(LastPass));
     alloc((void**)&u->d_part, sizeof(float) * u->part_floats);
     alloc((void**)&u->d_head_part, sizeof(float) * 100 * ((full + 255) / 256));
     if (e == hipSuccess) e = hipMemset(u->d_zero, 0, 1024);
-    if (e == hipSuccess) e = hipMemset(u->d_x16, 0, sizeof(int));
+    if (e == hipSuccess) e = hipMemset(u->d_pass, 0, sizeof(LastPass));
     if (e != hipSuccess) {
         vpt_unet_destroy(u);
         return set_error(VPT_ENOMEM, "vpt_unet_create: allocation failed (%s)", hipGetErrorString(e));
@@ -1514,9 +1515,7 @@ extern "C" VPT_API int vpt_unet_forward(vpt_unet* u, const uint16_t* d_x, int n,
     hipStream_t s = (hipStream_t)stream;
     const size_t npx = (size_t)n * h * w;
     HIP_TRY(hipMemcpyAsync(u->act[X], d_x, sizeof(uint16_t) * npx * 32, hipMemcpyDeviceToDevice, s));
-    bool capturing = false;
-    if (int rc = is_capturing(s, &capturing)) return rc;
-    return forward(u, n, h, w, false, capturing, d_out, mode == 1, s);
+    return forward(u, n, h, w, false, false, d_out, mode == 1, s);
 }
 
 extern "C" VPT_API int vpt_unet_backward(vpt_unet* u, const uint16_t* d_x, const float* d_target, int n, int h, int w,
@@ -1544,7 +1543,6 @@ extern "C" VPT_API int vpt_unet_adam_step(vpt_unet* u, float lr, void* stream)
     if (!u || !(lr > 0.0f)) return set_error(VPT_EINVAL, "vpt_unet_adam_step: bad arguments");
     DeviceGuard g(u->device);
     const float b1 = 0.9f, b2 = 0.999f;
-    if (int rc = make_last(u, u->last_n, u->last_h, u->last_w, (hipStream_t)stream)) return rc;
     u->adam_t++;
     const float c1 = 1.0f / (1.0f - powf(b1, (float)u->adam_t));
     const float c2 = 1.0f / (1.0f - powf(b2, (float)u->adam_t));
@@ -1587,9 +1585,7 @@ extern "C" VPT_API int vpt_unet_denoise(vpt_unet* u, const vpt_gbuffer* gb, cons
     if (int rc = check_dims(u, 1, gb->height, gb->width, "vpt_unet_denoise")) return rc;
     if (int rc = assemble("vpt_unet_denoise", u, gb, d_tex, u->act[X], true, stream)) return rc;
     DeviceGuard g(u->device);
-    bool capturing = false;
-    if (int rc = is_capturing((hipStream_t)stream, &capturing)) return rc;
-    return forward(u, 1, gb->height, gb->width, true, capturing, d_rgb, true, (hipStream_t)stream);
+    return forward(u, 1, gb->height, gb->width, true, false, d_rgb, true, (hipStream_t)stream);
 }
 
 extern "C" VPT_API int vpt_texel_accumulate(const vpt_svgf_texel* d_tex, int npx, float* d_acc, int reset, void* stream)
@@ -1621,12 +1617,17 @@ extern "C" VPT_API int vpt_unet_read_activation(vpt_unet* u, int index, int n, i
     DeviceGuard g(u->device);
     const size_t count = ((size_t)n * (h >> kLevel[index]) * (w >> kLevel[index])) * kChannels[index];
     HIP_TRY(hipDeviceSynchronize());
-    if (index == D0B) {
-        if (int rc = make_last(u, n, h, w, nullptr)) return rc;
+    int last[4] = {0, 0, 0, 0};   // x16, n, h, w
+    if (index == X || index == D0B) HIP_TRY(hipMemcpy(last, u->d_pass, sizeof(last), hipMemcpyDeviceToHost));
+    if (index == D0B && last[1]) {
+        // made from the pass's own D0A, parameters and sizes, whatever part is read
+        ConvArgs a = conv_args(u, u->net[kLayers - 1], last[1], last[2], last[3]);
+        a.w = u->d_pass->w_;
+        a.bias = u->d_pass->bias;
+        if (int rc = launch_conv(a, nullptr)) return rc;
         HIP_TRY(hipDeviceSynchronize());
     }
-    int half = 0;   // 16 of the input's 32 channels are stored, the others are zero
-    if (index == X) HIP_TRY(hipMemcpy(&half, u->d_x16, sizeof(int), hipMemcpyDeviceToHost));
+    const bool half = index == X && last[0];   // 16 of the input's 32 channels are stored, the others are zero
     HIP_TRY(hipMemcpy(host, u->act[index], sizeof(uint16_t) * (half ? count / 2 : count), hipMemcpyDeviceToHost));
     if (half) {
         for (size_t i = count / 32; i-- > 0;) {
