@@ -229,8 +229,12 @@ def test_last_activation(ctx):
     for k in x:
         u.backward(x[k], tgt[k], *k)
         want[k] = u.activation(12, *k)
-    u.backward(x[n, h, w], tgt[n, h, w], n, h, w)   # gradients for the steps below
+    other = torch.from_numpy(_inputs(rng, n, h, w)[0].view(np.int16)).cuda()
 
+    def soil():   # another pass's values in every buffer
+        u.backward(other, tgt[n, h, w], n, h, w)
+
+    soil()
     u.forward(x[n, h, w], n, h, w, out[n, h, w])
     one = u.activation(12, 1, h, w)
     np.testing.assert_array_equal(one, want[n, h, w][:1])
@@ -239,6 +243,7 @@ def test_last_activation(ctx):
     np.testing.assert_array_equal(tall.ravel(), want[n, h, w].ravel())
     np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])
 
+    soil()
     u.forward(x[n, h, w], n, h, w, out[n, h, w])
     params = u.get_params()
     u.adam_step(0.05)
@@ -253,10 +258,12 @@ def test_last_activation(ctx):
     u.forward(x[n, h, w], n, h, w, out[n, h, w])
     np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])   # recorded, not run
     for _ in range(3):
+        soil()
         graph.replay()
         np.testing.assert_array_equal(u.activation(12, *small), want[small])
         u.forward(x[n, h, w], n, h, w, out[n, h, w])
         np.testing.assert_array_equal(u.activation(12, n, h, w), want[n, h, w])
+        u.forward(x[n, h, w], n, h, w, out[n, h, w])
         graph.replay()
         u.adam_step(0.05)
         np.testing.assert_array_equal(u.activation(12, *small), want[small])
