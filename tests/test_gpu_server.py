@@ -119,6 +119,62 @@ def test_gi_rays_match_oracle(ctx, scene):
     np.testing.assert_array_equal(r["ref_vis"], expect)
 
 
+def _gi_oracle(g, rays, max_iter, shadow_iter):
+    """Hits and visibility of GI ray queries: the oracle's bounce, its
+    continuation origin and shadow trace."""
+    df = oracle.df_build(g)
+    b = oracle.trace_rays(g, df, rays, max_iter)
+    L = np.asarray(SUN, np.float32)
+    normals = np.array([[0, 0, 1], [0, 0, -1], [0, 1, 0], [0, -1, 0], [-1, 0, 0], [1, 0, 0]], np.float32)
+    hit = (b["t"] > 0) & (b["block"] > 0)
+    hn = normals[np.where(hit, b["face"], 0).astype(np.int64)]
+    cont = hit & (np.maximum((hn * L).sum(1, dtype=np.float32), np.float32(0)) >= np.float32(0.001))
+    vis = np.full(len(rays), 255, np.uint8)
+    with np.errstate(invalid="ignore", over="ignore"):   # the misses of infinite directions
+        so = ((rays[:, :3] + rays[:, 3:] * b["t"][:, None]) + hn * np.float32(0.045)).astype(np.float32)
+    s = oracle.trace_rays(g, df, np.concatenate([so[cont], np.broadcast_to(L, (cont.sum(), 3))], 1), shadow_iter)
+    vis[cont] = (s["t"] > 0).astype(np.uint8)
+    return b, vis
+
+
+@pytest.mark.parametrize("served", [False, True])
+@pytest.mark.parametrize("n", [262_144, 262_145, 300_001])
+def test_large_gi_launches_match_oracle(ctx, scene, n, served):
+    """GI ray queries around 1,024 blocks, above which a block regroups its
+    rays and compacts their shadow rays, with a ragged last block, hits and
+    visibility against the oracle; among the rays directions that are long,
+    infinite or NaN, which belong to no bin of heights."""
+    torch = _torch()
+    grids, worlds, _ = scene
+    g, w = grids[0], worlds[0]
+    rng = np.random.default_rng(n)
+    rays = _rays(rng, n, g.shape[::-1])
+    rays[:, 1] = rng.uniform(20, 110, n)
+    odd = rng.choice(n, 4000, replace=False)
+    rays[odd, 3 + rng.integers(0, 3, odd.size)] = rng.choice(
+        np.array([np.nan, np.inf, -np.inf, 1e30, -1e30, 3e38, -7.5, 900.0], np.float32), odd.size)
+    dev = _dev(rays)
+    print(f"gi rays n={n} served={served}", flush=True)
+    if served:
+        srv = Server(ctx, mode="batched", max_worlds=1, max_launch_rays=1 << 20)
+        t = srv.submit_rays(srv.add_world(w), "gi", dev, n, 48, SUN, 128)
+        out = srv.fetch(t)
+        hits, vis = out["hits"], out["vis"]
+    else:
+        hits = torch.empty(n * 12, dtype=torch.uint8, device="cuda")
+        vis = torch.empty(n, dtype=torch.uint8, device="cuda")
+        w.trace_gi_rays(dev, hits, vis, n, 48, SUN, 128)
+    got, vis = hits.cpu().numpy().view(HIT_DTYPE), vis.cpu().numpy()
+    if served:
+        srv.release(t)
+        srv.close()
+    ref, ref_vis = _gi_oracle(g, rays, 48, 128)
+    for k in ("t", "face", "block", "samples"):
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+    assert (ref_vis == 0).sum() > 1000 and (ref_vis == 1).sum() > 1000 and (ref_vis == 255).sum() > 1000
+    np.testing.assert_array_equal(vis, ref_vis)
+
+
 @pytest.mark.parametrize("mode", ["batched", "plain"])
 def test_alone_equals_mix(ctx, scene, mode):
     torch = _torch()

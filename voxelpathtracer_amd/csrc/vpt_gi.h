@@ -226,9 +226,11 @@ struct RayBlock {
     int jobs;
 };
 
+// Clamped as a float: a caller's direction may be of any length, infinite or
+// NaN (bin 0), which a conversion to int leaves undefined.
 __device__ inline int ray_bin(float dir_y)
 {
-    return min(kRayBins - 1, max(0, (int)((dir_y + 1.0f) * (0.5f * kRayBins))));
+    return (int)fminf(fmaxf((dir_y + 1.0f) * (0.5f * kRayBins), 0.0f), (float)(kRayBins - 1));
 }
 
 // Every lane's ray to its slot by bin (kRayBins + 1: no ray), then this
