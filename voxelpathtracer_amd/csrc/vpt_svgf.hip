@@ -766,26 +766,40 @@ __global__ void __launch_bounds__(256) variance_kernel(int W, int H, const float
             const int c0 = ly * kVarSW + (lx + kVarR + x);
 #pragma unroll
             for (int g = 0; g < 9; g += kVarGroup) {
-                // the group's weights first, so that their exps overlap; at
-                // 1920x1080 an SVGF frame 725 -> 708 us, a pipeline frame
-                // 1214 -> 1191 us and at 320x180 276 -> 272 us, the cheaper
-                // exp and division by 5 included
-                float w[kVarGroup];
+                // the group's weights first, so that their exps overlap
+                // (1920x1080: an SVGF frame 725 -> 708 us, a pipeline frame
+                // 1214 -> 1191 us, the cheaper exp and division by 5
+                // included); where no lane's weights need an exp, as between
+                // the pixels of a sky, they are left out: small images wait
+                // for the block that holds both sky and ground (259x100: a
+                // frame 112 us without this, 105 with it)
+                float w[kVarGroup], dd[kVarGroup], dl[kVarGroup];
+                bool live[kVarGroup], exps = false;
 #pragma unroll
                 for (int y = 0; y < kVarGroup; y++) {
                     const int c = c0 + (g + y) * kVarSW;
-                    const float nw = nw_row[s_n[c]];
                     // vpt_expf of a non-positive argument lies in [0, 1]
                     // (checked for every float), so at a depth gap of 25 or
                     // more the product is below exp(-50) * 3^16 < 1.5e-9 (3^16
                     // is the largest normal weight, sky against sky), under
-                    // both clamps below, and is taken as 0.
-                    const float dd = fabsf(s_t[c] - base_w);
-                    const float e = expf_32(-fminf(dd, 32.0f));
-                    const float lw = div_rcp(fabsf(s_aux[c].z - base_lum), color_phi, 1.0f / color_phi);
-                    const float el = expf_down(-lw);
-                    w[y] = nw != 0.0f && dd < 25.0f ? (el * nw) * (e * e) : 0.0f;
+                    // both clamps below, and is taken as 0.  vpt_expf(-0) is 1.
+                    w[y] = nw_row[s_n[c]];
+                    dd[y] = fabsf(s_t[c] - base_w);
+                    dl[y] = fabsf(s_aux[c].z - base_lum);
+                    live[y] = w[y] != 0.0f && dd[y] < 25.0f;
+                    exps = exps || (live[y] && dd[y] + dl[y] != 0.0f);
                 }
+                if (exps) {
+#pragma unroll
+                    for (int y = 0; y < kVarGroup; y++) {
+                        const float e = expf_32(-fminf(dd[y], 32.0f));
+                        const float lw = div_rcp(dl[y], color_phi, 1.0f / color_phi);
+                        const float el = expf_down(-lw);
+                        w[y] = (el * w[y]) * (e * e);
+                    }
+                }
+#pragma unroll
+                for (int y = 0; y < kVarGroup; y++) w[y] = live[y] ? w[y] : 0.0f;
 #pragma unroll
                 for (int y = 0; y < kVarGroup; y++) {
                     if ((uint32_t)(py + g + y - 4) >= (uint32_t)H) continue;   // exactly the taps inside the image
