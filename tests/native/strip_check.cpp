@@ -1,5 +1,5 @@
-// Every tile of an image comes once in strip order, and strip_pixels is the
-// running sum of the tiles' on-screen pixels.  Prints the mismatches.
+// Every tile of an image comes once in strip order and in the denoisers', and
+// strip_pixels is the running sum of the tiles' on-screen pixels.  Prints the mismatches.
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -25,6 +25,14 @@ int main(int argc, char** argv)
             sum += (size_t)((x1 < W ? x1 : W) - (int)p.x * 16) * (size_t)((y1 < H ? y1 : H) - (int)p.y * 16);
         }
         bad += vpt::strip_pixels(tx * ty, W, H) != sum || sum != (size_t)W * H;
+
+        // the denoisers' order of their 32x8 tiles
+        const uint32_t dx = (uint32_t)(W + 31) / 32u, dy = (uint32_t)(H + 7) / 8u;
+        std::vector<int> once(dx * dy, 0);
+        for (uint32_t t = 0; t < dx * dy; t++) {
+            const vpt::TileXY p = vpt::pass_tile_at(t, dx, dy);
+            bad += p.x >= dx || p.y >= dy || once[p.y * dx + p.x]++;
+        }
     }
     printf("%d mismatches\n", bad);
     return bad != 0;

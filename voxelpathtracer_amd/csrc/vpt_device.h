@@ -471,4 +471,10 @@ __device__ inline TileXY screen_tile(uint32_t tx, uint32_t ty)
     return strip_tile(xcd_remap(blockIdx.x, tx * ty), tx, ty);
 }
 
+// The same for the denoisers' passes, in their order.
+__device__ inline TileXY pass_tile(uint32_t tx, uint32_t ty)
+{
+    return pass_tile_at(xcd_remap(blockIdx.x, tx * ty), tx, ty);
+}
+
 }  // namespace vpt

@@ -39,6 +39,21 @@ VPT_HD TileXY strip_tile(uint32_t t, uint32_t tx, uint32_t ty)
     return TileXY{s * sw + r % width, r / width};
 }
 
+// The denoisers' order: bands, row by row from the top, where every tile has
+// a CU to itself (256 of them), so that no XCD's load is left to level and
+// the strips only cost: the blocks of a last column a few pixels wide lie on
+// one XCD, take their branches alike and wait for the same instructions (482
+// x 91: pre-spatial pass 13.2 us, in bands 6.8; SVGF frame 114 / 97).  Above,
+// strips: SVGF frame of 712 x 104 (299 tiles of 32 x 8) in strips / bands 112
+// / 106 us, 900 x 91 (348) 104 / 112, 482 x 180 (368) 109 / 114, 482 x 360
+// 124 / 138; below, 640 x 91 (240) 99 / 102, 200 x 91 (84) 113 / 103.
+constexpr uint32_t kBandTiles = 256u;
+
+VPT_HD TileXY pass_tile_at(uint32_t t, uint32_t tx, uint32_t ty)
+{
+    return tx * ty <= kBandTiles ? TileXY{t % tx, t / tx} : strip_tile(t, tx, ty);
+}
+
 // Pixels of the first t 16x16 tiles of a W x H image in strip order.
 inline size_t strip_pixels(uint32_t t, int W, int H)
 {
