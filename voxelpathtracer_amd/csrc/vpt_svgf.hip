@@ -1348,9 +1348,12 @@ __global__ void __launch_bounds__(256) shadow_temporal_kernel(CamView cam, Mat16
 // all in the window (every one at scales up to 1) computes its pixels' seven
 // rows once and keeps them in registers; the others (larger scales) take a
 // loop that works each tap out and reads global memory where it leaves the
-// window.  The choice is the wavefront's, since one that splits runs both
-// loops (320x180 at scale 2.5: 67 us split, 51 us whole).  Temporal pass and
-// filter, 229 -> 149 us at 1920x1080 and 49 -> 27 us at 320x180, of which the
+// window; only the reads differ there, so that a wavefront with both kinds
+// of tap works each out once (608x207 at scale 2.5: 54 us with a tap of its
+// own on either side, 45 with one).  The choice of the loop is the
+// wavefront's, since one that splits runs both (320x180 at scale 2.5: 67 us
+// split, 51 whole, 41 with the one tap).  Temporal pass and filter, 229 ->
+// 143 us at 1920x1080 and 49 -> 27 us at 320x180 at scale 1, of which the
 // cheaper exp and log and the normal classes are a part.
 constexpr int kSfA = 11;
 constexpr int kSfW = 32 + 2 * kSfA, kSfH = 8 + 2 * kSfA, kSfCells = kSfW * kSfH;
@@ -1501,18 +1504,29 @@ __global__ void __launch_bounds__(256) shadow_filter_kernel(int W, int H, const 
             const Line col = line(uvx, tex_w, x, W, gx0);
             for (int y = -size; y <= size; y++) {
                 const Line row = line(uvy, tex_h, y, H, gy0);
+                // the texels by either way, then one tap for both: lanes of one
+                // wavefront differ
+                float2 q00, q10, q01, q11;
+                float nw;
                 if (in_window(col, kSfW) && in_window(row, kSfH)) {
                     const float2* q = s_dc + row.lo * kSfW + col.lo;
-                    tap(q[0], q[1], q[kSfW], q[kSfW + 1], nw_row[s_f[row.near * kSfW + col.near]], col.frac, row.frac);
+                    q00 = q[0];
+                    q10 = q[1];
+                    q01 = q[kSfW];
+                    q11 = q[kSfW + 1];
+                    nw = nw_row[s_f[row.near * kSfW + col.near]];
                 } else {
                     const uint32_t c0 = (uint32_t)wrapn(col.lo + gx0, W), c1 = (uint32_t)wrapn(col.lo + gx0 + 1, W);
                     const uint32_t r0 = (uint32_t)wrapn(row.lo + gy0, H) * (uint32_t)W;
                     const uint32_t r1 = (uint32_t)wrapn(row.lo + gy0 + 1, H) * (uint32_t)W;
                     const uint32_t n = (uint32_t)wrapn(row.near + gy0, H) * (uint32_t)W + (uint32_t)wrapn(col.near + gx0, W);
-                    tap(make_float2(gb_t[r0 + c0], dec8(color[r0 + c0])), make_float2(gb_t[r0 + c1], dec8(color[r0 + c1])),
-                        make_float2(gb_t[r1 + c0], dec8(color[r1 + c0])), make_float2(gb_t[r1 + c1], dec8(color[r1 + c1])),
-                        nw_row[face_class(gb_face[n])], col.frac, row.frac);
+                    q00 = make_float2(gb_t[r0 + c0], dec8(color[r0 + c0]));
+                    q10 = make_float2(gb_t[r0 + c1], dec8(color[r0 + c1]));
+                    q01 = make_float2(gb_t[r1 + c0], dec8(color[r1 + c0]));
+                    q11 = make_float2(gb_t[r1 + c1], dec8(color[r1 + c1]));
+                    nw = nw_row[face_class(gb_face[n])];
                 }
+                tap(q00, q10, q01, q11, nw, col.frac, row.frac);
             }
         }
     }
