@@ -15,9 +15,14 @@
 
 #include "vpt_device.h"
 #include "vpt_internal.h"
+#include "vpt_short_math.h"
 
 using vpt::set_error;
 using vpt::Vec3;
+using vpt::div3_unit;
+using vpt::div_rcp;
+using vpt::expf_32;
+using vpt::expf_down;
 
 #define HIP_TRY(expr)                                                                          \
     do {                                                                                       \
@@ -168,35 +173,6 @@ __device__ inline Bil bil_setup(float s, float t, int W, int H)
     return b;
 }
 
-// vpt_expf for -32 <= x <= 0: the same polynomial; kf has at most seven bits
-// (for x down to -88) and LN2_HI eight, so their product is exact and the
-// subtraction one fma; the scaling by 2^k, k >= -46, is exact in one step.
-__device__ inline float expf_32(float x)
-{
-    const float LOG2E = 1.44269502162933349609375f;
-    const float LN2_HI = 0.693145751953125f;
-    const float LN2_LO = 1.428606765330187045e-06f;
-    const float kf = floorf(x * LOG2E + 0.5f);
-    float r = __builtin_fmaf(-kf, LN2_HI, x);
-    r = r - kf * LN2_LO;
-    float p = 0.0013829420786350965f;
-    p = p * r + 0.008374771103262901f;
-    p = p * r + 0.0416683591902256f;
-    p = p * r + 0.1666642129421234f;
-    p = p * r + 0.49999991059303284f;
-    p = p * r + 1.0f;
-    p = p * r + 1.0f;
-    return __builtin_ldexpf(p, (int)kf);
-}
-
-// vpt_expf for x <= 0, where it is 0 below -87.34; above, p 2^k is rounded at
-// most once, in either form of the scaling.
-__device__ inline float expf_down(float x)
-{
-    const float e = expf_32(fmaxf(x, -88.0f));
-    return x < -87.33654022216796875f ? 0.0f : e;
-}
-
 __device__ inline float bil(float t00, float t10, float t01, float t11, float a, float b)
 {
     float top = t00 * (1.0f - a) + t10 * a;
@@ -283,22 +259,6 @@ __device__ inline bool pixel_of(int W, int H, int& px, int& py)
 dim3 pass_grid(int W, int H) { return dim3((unsigned)(((W + 31) / 32) * ((H + 7) / 8))); }
 
 __device__ inline float texc(int p, int n) { return ((float)p + 0.5f) / (float)n; }
-
-// a / b given y = 1 / b (the correctly rounded reciprocal), for quotients
-// that are zero or normal with an exactly representable remainder, which is
-// the case for every weighted mean and weight ratio below: q0 = a y lies
-// within an ulp of a / b, the remainder a - b q0 is exact in an fma, and
-// q0 + (a - b q0) y rounded once is the correctly rounded quotient
-// (Markstein, IBM J. Res. Dev. 34(1), 1990).  A zero q0 is returned as is,
-// keeping the sign that the correction's addition would drop.  Three VALU
-// operations and a select per quotient, against about ten for a division,
-// where several quotients share a divisor.
-__device__ inline float div_rcp(float a, float b, float y)
-{
-    const float q0 = a * y;
-    const float q = fmaf(fmaf(-b, q0, a), y, q0);
-    return q0 == 0.0f ? q0 : q;
-}
 
 // vpt::normalize3 of the camera ray through (sx, sy), its three components
 // divided by the length through one reciprocal (div_rcp), then the point at
@@ -1131,17 +1091,6 @@ __device__ inline int wrapn(int i, int n)
 
 __device__ inline float dec8(uint8_t c) { return vpt_unorm8_decode(c); }
 
-// x / 3 for 0 <= x <= 2: q0 = x fl(1/3), then one correction with the exact
-// remainder x - 3 q0 (an fma).  Equal to the IEEE division for every float
-// in [0, 2], subnormals included (tests/test_exact_division_cpu.py checks
-// all of them); three VALU operations in place of the division's ten.
-__device__ inline float div3_unit(float x)
-{
-    const float y = 1.0f / 3.0f;
-    const float q0 = x * y;
-    return fmaf(fmaf(-3.0f, q0, x), y, q0);
-}
-
 // (m - 1) / (m + 1) for the m that vpt_logf's reduction leaves, [sqrt(2) / 2,
 // sqrt(2)]: v_rcp_f32, one Newton step for the reciprocal, then one
 // correction with the exact remainder.  Equal to the IEEE division for
@@ -1156,24 +1105,11 @@ __device__ inline float log_ratio(float m)
     return fmaf(fmaf(-b, q0, a), y, q0);
 }
 
-// vpt_logf for x in [2/3, 1): the same operations with log_ratio in place of
-// the division and without the cases that cannot arise there, so the same
-// results.
+// vpt_logf for x in [2/3, 1).
 __device__ inline float logf_unit(float x)
 {
-    const bool low = x + x <= 1.41421353816986083984375f;   // x = m 2^-1 with m up to sqrt(2), or m itself
-    const float m = low ? x + x : x;
-    const float fe = low ? -1.0f : 0.0f;
-    const float LN2_HI = 0.693145751953125f;
-    const float LN2_LO = 1.428606765330187045e-06f;
-    float s = log_ratio(m);
-    float s2 = s * s;
-    float p = 0.111111111111f;
-    p = p * s2 + 0.142857142857f;
-    p = p * s2 + 0.2f;
-    p = p * s2 + 0.333333333333f;
-    float lm = (s + s) + (s + s) * (s2 * p);
-    return fe * LN2_HI + (fe * LN2_LO + lm);
+    const vpt::UnitLog r = vpt::log_unit_reduce(x);
+    return vpt::log_unit_sum(log_ratio(r.m), r.e);
 }
 
 // Every float m in [sqrt(2) / 2, sqrt(2)]: log_ratio(m) against the division.
