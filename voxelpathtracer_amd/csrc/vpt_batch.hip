@@ -4,10 +4,11 @@
 // Every lane holds one ray.  Each loop turn the wavefront refills its idle
 // lanes from a wave-private chunk of the queue (one atomicAdd per `chunk`
 // rays) and advances every active ray by one iteration of the reference's
-// loop (trav_prepare / trav_advance, the same code as the one-launch
-// kernels, so hits are bit-identical).  A
-// finished ray writes its result by kind; a diffuse-GI ray that hits a
-// sun-facing block continues in the same slot as the hit's shadow ray.
+// loop (trav_prepare / trav_advance; the one-launch kernels make the same
+// turns in trav_run, around the same one-cell step, and hits are
+// bit-identical: tests/test_gpu_batch.py).  A finished ray writes its result
+// by kind; a diffuse-GI ray that hits a sun-facing block continues in the
+// same slot as the hit's shadow ray.
 //
 // The frame path runs: persistent primary rays (pixel index -> ray) ->
 // secondary-ray generation with wave-level compaction (ballot + popcount +

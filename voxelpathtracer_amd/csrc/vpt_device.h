@@ -239,17 +239,21 @@ __device__ __attribute__((always_inline)) inline void trav_init(Trav& r, Vec3 o,
 // Bit pattern of (float)dim, dim = max + 1 (0 for the empty view, max = -1).
 __device__ inline uint32_t trav_bound(float max) { return __float_as_uint(max + 1.0f); }
 
-// trav_prepare without the iteration cap, for loops that test the cap
-// where trav_advance returns.
-__device__ __attribute__((always_inline)) inline bool trav_locate(const WorldView& w, Trav& r, uint32_t& off,
-                                                                  Cell& c)
+// IsInVolume(floor(o)), one unsigned compare per axis: floor(o) lies in
+// [0, dim - 1] exactly when o lies in [+0, dim); non-negative floats order as
+// their bit patterns, and negative values and NaN have patterns above every
+// bound.
+__device__ __attribute__((always_inline)) inline bool trav_inside(const WorldView& w, const Trav& r)
 {
-    // IsInVolume(floor(o)), one unsigned compare per axis: floor(o) lies in
-    // [0, dim - 1] exactly when o lies in [+0, dim); non-negative floats
-    // order as their bit patterns, and negative values and NaN have patterns
-    // above every bound.
-    if (!(__float_as_uint(r.ox) < trav_bound(w.xmax) && __float_as_uint(r.oy) < trav_bound(w.ymax) &&
-          __float_as_uint(r.oz) < trav_bound(w.zmax))) {
+    return __float_as_uint(r.ox) < trav_bound(w.xmax) && __float_as_uint(r.oy) < trav_bound(w.ymax) &&
+           __float_as_uint(r.oz) < trav_bound(w.zmax);
+}
+
+__device__ __attribute__((always_inline)) inline bool trav_prepare(const WorldView& w, Trav& r, uint32_t& off,
+                                                                   Cell& c)
+{
+    if (r.samples >= r.max_iter) return false;
+    if (!trav_inside(w, r)) {
         r.inter = 0;
         return false;
     }
@@ -261,10 +265,51 @@ __device__ __attribute__((always_inline)) inline bool trav_locate(const WorldVie
     return true;
 }
 
-__device__ __attribute__((always_inline)) inline bool trav_prepare(const WorldView& w, Trav& r, uint32_t& off,
-                                                                   Cell& c)
+// What the one-cell step needs of a ray's direction: the signs, h = (1 + s)
+// / 2, e = s + 1 - h and s * 0.0001.
+struct StepDir {
+    int sx, sz;
+    float hx, hy, hz, ex, ey, ez, tx, ty, tz;
+};
+
+__device__ __attribute__((always_inline)) inline StepDir step_dir(const Trav& r)
 {
-    return r.samples < r.max_iter && trav_locate(w, r, off, c);
+    const int sx = sgn(r.dx), sy = sgn(r.dy), sz = sgn(r.dz);
+    const float hx = (float)((1 + sx) >> 1), hy = (float)((1 + sy) >> 1), hz = (float)((1 + sz) >> 1);
+    return StepDir{sx,
+                   sz,
+                   hx,
+                   hy,
+                   hz,
+                   (float)(sx + 1) - hx,
+                   (float)(sy + 1) - hy,
+                   (float)(sz + 1) - hz,
+                   (float)sx * 0.0001f,
+                   (float)sy * 0.0001f,
+                   (float)sz * 0.0001f};
+}
+
+// E == 1: the one-cell step from cell c to (ax, ay, az) across axis mi, with
+// selects on the step axis (no divergent branches: fewer exec-mask moves in
+// the loop).  The reference forms float(int(o) + s) + w, then adds s * 0.0001
+// on the step axis.  On that axis w is 1 - h, and the integers add exactly:
+// (g + s) + (1 - h) = g + (s + 1 - h), also for the s = 0 that the y axis can
+// be picked with.  On the others s is 0 and w moves by d * fm.
+__device__ __attribute__((always_inline)) inline void one_cell(const Trav& r, const StepDir& s, const Cell& c,
+                                                               float& ax, float& ay, float& az, int& mi)
+{
+    // float(int(o)) of the reference is the cell's corner
+    const float gx = (float)c.x, gy = (float)c.y, gz = (float)c.z;
+    const float wx = r.ox - gx, wy = r.oy - gy, wz = r.oz - gz;
+    const float fxx = (s.hx - wx) * r.ix, fyy = (s.hy - wy) * r.iy, fzz = (s.hz - wz) * r.iz;
+    const bool x_first = fxx < fyy && s.sx != 0;
+    const float fxy = x_first ? fxx : fyy;
+    const bool not_z = fxy < fzz || s.sz == 0;
+    const float fm = not_z ? fxy : fzz;
+    ax = pick(x_first && not_z, (gx + s.ex) + s.tx, gx + (wx + r.dx * fm));
+    ay = pick(!x_first && not_z, (gy + s.ey) + s.ty, gy + (wy + r.dy * fm));
+    az = pick(not_z, gz + (wz + r.dz * fm), (gz + s.ez) + s.tz);
+    mi = not_z ? (x_first ? 0 : 1) : 2;
 }
 
 __device__ __attribute__((always_inline)) inline bool trav_advance(Trav& r, int m, const Cell& c)
@@ -272,27 +317,9 @@ __device__ __attribute__((always_inline)) inline bool trav_advance(Trav& r, int 
     r.samples++;
     if (m == 0) return false;   // E == 0
     if (m < 4) {
-        // E == 1: the one-cell step, with selects on the step axis (no
-        // divergent branches: fewer exec-mask moves in the loop)
-        const int sx = sgn(r.dx), sy = sgn(r.dy), sz = sgn(r.dz);
-        const int hx = (1 + sx) >> 1, hy = (1 + sy) >> 1, hz = (1 + sz) >> 1;
-        // float(int(o)) of the reference is the cell's corner
-        const float gx = (float)c.x, gy = (float)c.y, gz = (float)c.z;
-        const float wx = r.ox - gx, wy = r.oy - gy, wz = r.oz - gz;
-        const float fxx = ((float)hx - wx) * r.ix;
-        const float fyy = ((float)hy - wy) * r.iy;
-        const float fzz = ((float)hz - wz) * r.iz;
-        const int mi = (fxx < fyy && sx != 0) ? ((fxx < fzz || sz == 0) ? 0 : 2) : ((fyy < fzz || sz == 0) ? 1 : 2);
-        const bool m0 = mi == 0, m1 = mi == 1, m2 = mi == 2;
-        const float fm = m0 ? fxx : (m1 ? fyy : fzz);
-        // The reference forms float(int(o) + s) + w, then adds s * 0.0001 on
-        // the step axis.  On that axis w is 1 - h, and the integers add
-        // exactly: (g + s) + (1 - h) = g + (s + 1 - h), also for the s = 0
-        // that the y axis can be picked with.  On the others s is 0 and w
-        // moves by d * fm.
-        const float ax = pick(m0, (gx + (float)(sx + 1 - hx)) + (float)sx * 0.0001f, gx + (wx + r.dx * fm));
-        const float ay = pick(m1, (gy + (float)(sy + 1 - hy)) + (float)sy * 0.0001f, gy + (wy + r.dy * fm));
-        const float az = pick(m2, (gz + (float)(sz + 1 - hz)) + (float)sz * 0.0001f, gz + (wz + r.dz * fm));
+        float ax, ay, az;
+        int mi;
+        one_cell(r, step_dir(r), c, ax, ay, az, mi);
         r.ox = ax;
         r.oy = ay;
         r.oz = az;
@@ -338,13 +365,7 @@ __device__ __attribute__((always_inline)) inline Hit trav_finish(const WorldView
     return h;
 }
 
-__device__ __attribute__((always_inline)) inline bool trav_inside(const WorldView& w, const Trav& r)
-{
-    return __float_as_uint(r.ox) < trav_bound(w.xmax) && __float_as_uint(r.oy) < trav_bound(w.ymax) &&
-           __float_as_uint(r.oz) < trav_bound(w.zmax);
-}
-
-// The loop's turns of a ray to its end or to r.max_iter, as trav_locate and
+// The loop's turns of a ray to its end or to r.max_iter, as trav_prepare and
 // trav_advance make them, in a form with one exit and selects in place of
 // most branches.  The position must be inside the volume and samples below
 // the cap on entry; returns the last DF byte (0: stopped in a solid cell).
@@ -357,34 +378,17 @@ __device__ __attribute__((always_inline)) inline bool trav_inside(const WorldVie
 template <bool kEager>
 __device__ __attribute__((always_inline)) inline int trav_run(const WorldView& w, Trav& r)
 {
-    const int sx = sgn(r.dx), sy = sgn(r.dy), sz = sgn(r.dz);
-    const float hx = (float)((1 + sx) >> 1), hy = (float)((1 + sy) >> 1), hz = (float)((1 + sz) >> 1);
-    const float ex = (float)(sx + 1) - hx, ey = (float)(sy + 1) - hy, ez = (float)(sz + 1) - hz;
-    const float tx = (float)sx * 0.0001f, ty = (float)sy * 0.0001f, tz = (float)sz * 0.0001f;
+    const StepDir s = step_dir(r);
     const uint32_t bx = trav_bound(w.xmax), by = trav_bound(w.ymax), bz = trav_bound(w.zmax);
     int m;
     bool alive;
     do {
-        const uint32_t cx = (uint32_t)r.ox, cy = (uint32_t)r.oy, cz = (uint32_t)r.oz;
-        m = plane_byte(w.df, brick_offset_fast(cx, cy, cz, w.row_stride, w.slab_stride));
+        const Cell c{(uint32_t)r.ox, (uint32_t)r.oy, (uint32_t)r.oz};
+        m = plane_byte(w.df, brick_offset_fast(c.x, c.y, c.z, w.row_stride, w.slab_stride));
         float ax, ay, az;
         int mi;
-        // the one-cell step of trav_advance
-        auto one_cell = [&]() __attribute__((always_inline)) {
-            const float gx = (float)cx, gy = (float)cy, gz = (float)cz;
-            const float wx = r.ox - gx, wy = r.oy - gy, wz = r.oz - gz;
-            const float fxx = (hx - wx) * r.ix, fyy = (hy - wy) * r.iy, fzz = (hz - wz) * r.iz;
-            const bool x_first = fxx < fyy && sx != 0;
-            const float fxy = x_first ? fxx : fyy;
-            const bool not_z = fxy < fzz || sz == 0;
-            const float fm = not_z ? fxy : fzz;
-            ax = pick(x_first && not_z, (gx + ex) + tx, gx + (wx + r.dx * fm));
-            ay = pick(!x_first && not_z, (gy + ey) + ty, gy + (wy + r.dy * fm));
-            az = pick(not_z, gz + (wz + r.dz * fm), (gz + ez) + tz);
-            mi = not_z ? (x_first ? 0 : 1) : 2;
-        };
         if (kEager) {
-            one_cell();
+            one_cell(r, s, c, ax, ay, az, mi);
             // all of that before the byte is waited for
             asm volatile("" : "+v"(ax), "+v"(ay), "+v"(az), "+v"(mi));
             const bool solid = m == 0, one = m < 4;
@@ -397,7 +401,7 @@ __device__ __attribute__((always_inline)) inline int trav_run(const WorldView& w
             r.oy = solid ? r.oy : ny;
             r.oz = solid ? r.oz : nz;
         } else if (m < 4) {
-            one_cell();
+            one_cell(r, s, c, ax, ay, az, mi);
             const bool solid = m == 0;
             r.ox = pick(solid, r.ox, ax);
             r.oy = pick(solid, r.oy, ay);
