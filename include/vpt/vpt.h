@@ -521,8 +521,9 @@ VPT_API int vpt_frame_autotune(vpt_frame* f, vpt_world* w, const vpt_camera* cam
  * requests together in one kernel (a request larger than a launch is split
  * over several) — one lane per ray by default, or the persistent refill
  * kernel when the launch shape's bit 1 is clear (vpt_server_set_launch_cfg)
- * — GI bounces continue as their shadow rays in the same lane, up to max_inflight launches are queued on the device at once,
- * and requests that arrive meanwhile join the next launch.  Results are
+ * — GI bounces continue as their shadow rays within the launch, up to
+ * max_inflight launches are queued on the device at once, and requests that
+ * arrive meanwhile join the next launch.  Results are
  * bit-identical in both modes and do not depend on what else is in flight.
  *
  * Results live in server memory until vpt_server_release.  A request's

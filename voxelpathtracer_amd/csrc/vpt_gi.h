@@ -222,7 +222,7 @@ constexpr int kRayBins = 16;
 struct RayBlock {
     float r[6][256];
     uint32_t id[256];
-    int bin[kRayBins + 2];   // counts, then first slots; [kRayBins]: other rays, in place among themselves
+    int bin[kRayBins + 2];   // counts, then first slots; [kRayBins]: other rays
     int jobs;
 };
 
@@ -233,8 +233,9 @@ __device__ inline int ray_bin(float dir_y)
     return (int)fminf(fmaxf((dir_y + 1.0f) * (0.5f * kRayBins), 0.0f), (float)(kRayBins - 1));
 }
 
-// Every lane's ray to its slot by bin (kRayBins + 1: no ray), then this
-// lane's slot back.  All 256 lanes must call it.
+// Every lane's ray to its slot by bin (kRayBins: rays that have none, kRayBins
+// + 1: no ray; the order within a bin is not fixed), then this lane's slot
+// back.  All 256 lanes must call it.
 __device__ inline void regroup(RayBlock& b, int bin, Vec3& o, Vec3& d, uint32_t& id)
 {
     if (threadIdx.x < kRayBins + 2) b.bin[threadIdx.x] = 0;

@@ -602,8 +602,8 @@ __global__ void __launch_bounds__(256) variance_kernel(int W, int H, const float
     bool uniform = false, uniform_m = false;
     if (__syncthreads_or(spatial)) {
         // the block's cells, three per thread (256 threads), read together:
-        // an off-screen cell reads the nearest on-screen one and is never
-        // read back from LDS
+        // an off-screen cell reads the nearest on-screen one (weights are
+        // worked out from it with its group's, and dropped)
         constexpr int kPer = (kVarCells + 255) / 256;
         const int tid = (int)threadIdx.x;
         __builtin_assume(tid >= 0 && tid < 256);

@@ -173,18 +173,22 @@ __device__ inline int place_piece(int place, int row) { return (place - (row >> 
 // it, so a step reads 3 * (R + 2) pixel fragments for 9 * R * NT products.
 // The weight rows are ordered so that a lane ends with 8 consecutive
 // channels of its pixel for each 32 channels: bias, ReLU, mask, 2x2 pooling
-// and the 1x1 head run in registers, and 16 lanes store 1 KiB of
-// consecutive pixels (COUT = 32) with one 16-byte store each.
+// and the 1x1 head run in registers, and a wave stores 1 KiB of consecutive
+// pixels (COUT = 32), 16 bytes a lane.
 // kOneSlice (32 input channels): the weights are loaded once per launch.
 // kHead: the network's last convolution, with the 1x1 output head over its
 // stored values in registers (p.y null: the values themselves are not
 // stored).
-// What bounds it at 1920x1080: the 32-channel layers at full resolution move
-// 266 to 300 MB (55 to 75 us, 4 to 5 TB/s), the 64-channel ones are held by
-// the products' issue and what a step does between them (d1a 105 us, 1.1
-// PFLOP/s of the 2.0 that random data sustains; its two waves per SIMD leave
-// the barrier together).  Measured, whole denoise call: 1920x1080 894 -> 632
-// us, 640x360 204 -> 134 us, against a kernel that staged through registers
+// What bounds it at 1920x1080 (profiled): of the 32-channel layers at full
+// resolution, memory where they store their activation (e0a 199 MB in 49 us,
+// e0b 299 MB in 67 us, 4 to 4.5 TB/s), the epilogue in the last one, which
+// with the head moves 158 MB in 76 us (2.1 TB/s); the 64-channel ones are
+// held by the products' issue and what a step does between them (d1a 100 us,
+// 1.15 PFLOP/s of the 2.0 that random data sustains; its two waves per SIMD
+// leave the barrier together), those of two and three slices also by their
+// weights, loaded again each step (d0a 136 us, 0.84 PFLOP/s).  Measured,
+// whole denoise call: 1920x1080 894 -> 608
+// us, 640x360 204 -> 135 us, against a kernel that staged through registers
 // behind two barriers a step, read each pixel fragment for each of the three
 // rows and stored through LDS, with the head and a 32-channel input apart.
 // A second workgroup per CU on 16x16 tiles was slower for these layers.
