@@ -28,10 +28,12 @@ int main(int argc, char** argv)
 
         // the denoisers' order of their 32x8 tiles
         const uint32_t dx = (uint32_t)(W + 31) / 32u, dy = (uint32_t)(H + 7) / 8u;
-        std::vector<int> once(dx * dy, 0);
-        for (uint32_t t = 0; t < dx * dy; t++) {
-            const vpt::TileXY p = vpt::pass_tile_at(t, dx, dy);
-            bad += p.x >= dx || p.y >= dy || once[p.y * dx + p.x]++;
+        for (int narrow = 0; narrow < 2; narrow++) {
+            std::vector<int> once(dx * dy, 0);
+            for (uint32_t t = 0; t < dx * dy; t++) {
+                const vpt::TileXY p = vpt::pass_tile_at(t, dx, dy, narrow != 0);
+                bad += p.x >= dx || p.y >= dy || once[p.y * dx + p.x]++;
+            }
         }
     }
     printf("%d mismatches\n", bad);

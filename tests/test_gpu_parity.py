@@ -421,10 +421,11 @@ def test_svgf_parity_small(ctx, terrain_world):
     _assert_exact(res)
 
 
-@pytest.mark.parametrize("W,H", [(2, 2), (5, 3), (33, 9), (70, 41)])
+@pytest.mark.parametrize("W,H", [(2, 2), (5, 3), (33, 9), (70, 41), (260, 241)])
 def test_svgf_parity_ragged(ctx, terrain_world, W, H):
     """Images smaller than a tile and its 9x9 apron, and ones a tile does not
-    divide: taps off the image in every pass; bit-exact."""
+    divide: taps off the image in every pass; and one of more than 256 tiles
+    whose last column is narrow; bit-exact."""
     g, df, w = terrain_world
     res, _, _ = _run_svgf(ctx, w, g, df, W, H, 3)
     _assert_exact(res)

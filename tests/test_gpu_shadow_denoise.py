@@ -115,7 +115,7 @@ def test_shadow_denoise_filter_scale(ctx, terrain_world):
 
 
 @pytest.mark.parametrize("W,H,scale", [(2, 2, 1.0), (5, 3, 1.0), (11, 9, 1.0), (33, 17, 1.0), (70, 41, 0.3),
-                                       (70, 41, 1.2), (70, 41, 6.0)])
+                                       (70, 41, 1.2), (70, 41, 6.0), (260, 241, 2.5)])
 def test_shadow_denoise_window_edges(ctx, terrain_world, W, H, scale):
     """Images narrower than the filter's staged window (its cells repeat the
     image several times) and a scale at which some of a tile's pixels reach

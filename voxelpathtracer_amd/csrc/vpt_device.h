@@ -475,10 +475,11 @@ __device__ inline TileXY screen_tile(uint32_t tx, uint32_t ty)
     return strip_tile(xcd_remap(blockIdx.x, tx * ty), tx, ty);
 }
 
-// The same for the denoisers' passes, in their order.
-__device__ inline TileXY pass_tile(uint32_t tx, uint32_t ty)
+// The same for the denoisers' passes over 32x8 tiles, in their order.
+__device__ inline TileXY pass_tile(int W, int H)
 {
-    return pass_tile_at(xcd_remap(blockIdx.x, tx * ty), tx, ty);
+    const uint32_t tx = (uint32_t)(W + 31) / 32u, ty = (uint32_t)(H + 7) / 8u;
+    return pass_tile_at(xcd_remap(blockIdx.x, tx * ty), tx, ty, (uint32_t)(W - 1) % 32u < 7u);
 }
 
 }  // namespace vpt

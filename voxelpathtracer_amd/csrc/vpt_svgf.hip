@@ -248,9 +248,7 @@ __device__ inline float load_x(const vpt_svgf_texel* p, size_t i)
 // 512-byte texel rows), dealt to XCDs in the denoisers' order.
 __device__ inline bool pixel_of(int W, int H, int& px, int& py)
 {
-    const uint32_t tiles_x = (uint32_t)(W + 31) / 32u;
-    const uint32_t tiles_y = (uint32_t)(H + 7) / 8u;
-    const vpt::TileXY tile = vpt::pass_tile(tiles_x, tiles_y);
+    const vpt::TileXY tile = vpt::pass_tile(W, H);
     px = (int)tile.x * 32 + (int)(threadIdx.x & 31);
     py = (int)tile.y * 8 + (int)(threadIdx.x >> 5);
     return px < W && py < H;
@@ -584,8 +582,7 @@ __global__ void __launch_bounds__(256) variance_kernel(int W, int H, const float
     // reads no SH cell afterwards), so that six blocks fit in a CU's LDS
     static_assert(sizeof(float) * 9 * 82 <= sizeof(float4) * kVarCells, "s_tab fits in s_sh");
     float (*const s_tab)[82] = reinterpret_cast<float (*)[82]>(s_sh);
-    const uint32_t tiles_x = (uint32_t)(W + 31) / 32u;
-    const vpt::TileXY tile = vpt::pass_tile(tiles_x, (uint32_t)(H + 7) / 8u);
+    const vpt::TileXY tile = vpt::pass_tile(W, H);
     const int x0 = (int)tile.x * 32, y0 = (int)tile.y * 8;
     const int lx = (int)(threadIdx.x & 31), ly = (int)(threadIdx.x >> 5);
     const int px = x0 + lx, py = y0 + ly;
@@ -1304,8 +1301,7 @@ __global__ void __launch_bounds__(256) shadow_filter_kernel(int W, int H, const 
     __shared__ float2 s_dc[kSfCells];   // depth, decoded colour
     __shared__ uint8_t s_f[kSfCells];   // normal class (face, or 6)
     __shared__ float s_nw[7 * 8];
-    const uint32_t tiles_x = (uint32_t)(W + 31) / 32u;
-    const vpt::TileXY tile = vpt::pass_tile(tiles_x, (uint32_t)(H + 7) / 8u);
+    const vpt::TileXY tile = vpt::pass_tile(W, H);
     const int tx0 = (int)tile.x * 32, ty0 = (int)tile.y * 8;
     const int gx0 = tx0 - kSfA, gy0 = ty0 - kSfA;   // image position of staged cell (0, 0)
     {

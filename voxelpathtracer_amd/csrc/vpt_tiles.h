@@ -39,19 +39,27 @@ VPT_HD TileXY strip_tile(uint32_t t, uint32_t tx, uint32_t ty)
     return TileXY{s * sw + r % width, r / width};
 }
 
-// The denoisers' order: bands, row by row from the top, where every tile has
-// a CU to itself (256 of them), so that no XCD's load is left to level and
-// the strips only cost: the blocks of a last column a few pixels wide lie on
-// one XCD, take their branches alike and wait for the same instructions (482
-// x 91: pre-spatial pass 13.2 us, in bands 6.8; SVGF frame 114 / 97).  Above,
-// strips: SVGF frame of 712 x 104 (299 tiles of 32 x 8) in strips / bands 112
-// / 106 us, 900 x 91 (348) 104 / 112, 482 x 180 (368) 109 / 114, 482 x 360
-// 124 / 138; below, 640 x 91 (240) 99 / 102, 200 x 91 (84) 113 / 103.
+// The denoisers' order.  Bands, row by row from the top, where every tile has
+// a CU to itself (256 of them): no XCD's load is left to level there.  SVGF
+// frame of 200 x 91 (84 tiles of 32 x 8) in strips / bands 113 / 103 us, 482
+// x 110 (224) 121 / 96, 640 x 91 (240) 99 / 102; above, 900 x 91 (348) 104 /
+// 112, 482 x 180 (368) 109 / 114, 482 x 360 124 / 138.
+// A last column a few pixels wide (`narrow`) is not part of the strips; its
+// tiles come one after each row's worth of the others.  As a strip of its own
+// its blocks lay on one XCD, took their branches alike and waited for the same
+// instructions (pre-spatial pass of 482 x 91: 13.2 us, 6.8 where they were
+// spread): SVGF frame of 260 x 241 136 -> 112 us, 1924 x 1080 752 -> 732.
 constexpr uint32_t kBandTiles = 256u;
 
-VPT_HD TileXY pass_tile_at(uint32_t t, uint32_t tx, uint32_t ty)
+VPT_HD TileXY pass_tile_at(uint32_t t, uint32_t tx, uint32_t ty, bool narrow)
 {
-    return tx * ty <= kBandTiles ? TileXY{t % tx, t / tx} : strip_tile(t, tx, ty);
+    if (tx * ty <= kBandTiles) return TileXY{t % tx, t / tx};
+    if (narrow && tx > 1u) {
+        const uint32_t row = t / tx;
+        if (t % tx == tx - 1u) return TileXY{tx - 1u, row};
+        return strip_tile(t - row, tx - 1u, ty);
+    }
+    return strip_tile(t, tx, ty);
 }
 
 // Pixels of the first t 16x16 tiles of a W x H image in strip order.
