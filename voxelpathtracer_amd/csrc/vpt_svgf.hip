@@ -566,6 +566,16 @@ constexpr int kVarSW = 32 + 2 * kVarR, kVarSH = 8 + 2 * kVarR, kVarCells = kVarS
 
 __device__ inline int normal_index(uint32_t face) { return face <= 5u ? (int)face : 6; }
 
+// Launches of at most three blocks a CU wait for the block that holds both
+// sky and ground; there (kSkipExps) the exps of a group whose live taps all
+// have the pixel's own depth and luminance, as between the pixels of a sky,
+// are left out.  SVGF frame of 259x100 (117 tiles), with every exp / without
+// those 101 / 96 us, 482x91 (192) 109 / 97, 600x240 (570) 125 / 117, 640x360
+// (900) 143 / 144; at 1920x1080 the test costs more than it saves (this
+// kernel 174 / 188 us in a frame without a history).
+constexpr int kSkipExpsTiles = 768;
+
+template <bool kSkipExps>
 __global__ void __launch_bounds__(256) variance_kernel(int W, int H, const float* __restrict__ gb_t,
                                                        const uint8_t* __restrict__ gb_face,
                                                        const vpt_svgf_texel* __restrict__ in,
@@ -723,23 +733,20 @@ __global__ void __launch_bounds__(256) variance_kernel(int W, int H, const float
             const int c0 = ly * kVarSW + (lx + kVarR + x);
 #pragma unroll
             for (int g = 0; g < 9; g += kVarGroup) {
-                // the group's weights first, so that their exps overlap
-                // (1920x1080: an SVGF frame 725 -> 708 us, a pipeline frame
-                // 1214 -> 1191 us, the cheaper exp and division by 5
-                // included); where no lane's weights need an exp, as between
-                // the pixels of a sky, they are left out: small images wait
-                // for the block that holds both sky and ground (259x100: a
-                // frame 112 us without this, 105 with it)
+                // the group's weights first, so that their exps overlap (an
+                // SVGF frame at 1920x1080 725 -> 708 us, a pipeline frame 1214
+                // -> 1191 us, the cheaper exp and division by 5 included)
                 float w[kVarGroup], dd[kVarGroup], dl[kVarGroup];
-                bool live[kVarGroup], exps = false;
+                bool live[kVarGroup], exps = !kSkipExps;
 #pragma unroll
                 for (int y = 0; y < kVarGroup; y++) {
                     const int c = c0 + (g + y) * kVarSW;
                     // vpt_expf of a non-positive argument lies in [0, 1]
-                    // (checked for every float), so at a depth gap of 25 or
-                    // more the product is below exp(-50) * 3^16 < 1.5e-9 (3^16
-                    // is the largest normal weight, sky against sky), under
-                    // both clamps below, and is taken as 0.  vpt_expf(-0) is 1.
+                    // (tests/native/exp_log_check.cpp), so at a depth gap of 25
+                    // or more the product is below exp(-50) * 3^16 < 1.5e-9
+                    // (3^16 is the largest normal weight, sky against sky),
+                    // under both clamps below, and is taken as 0.  vpt_expf(-0)
+                    // is 1.
                     w[y] = nw_row[s_n[c]];
                     dd[y] = fabsf(s_t[c] - base_w);
                     dl[y] = fabsf(s_aux[c].z - base_lum);
@@ -1579,8 +1586,8 @@ extern "C" VPT_API int vpt_svgf_frame(vpt_svgf* s, const vpt_camera* cam, const 
                        prev->d_t, prev->d_face, prev->d_block, temporal_in, s->d_temporal[hist], s->d_util[hist],
                        s->d_temporal[next], s->d_util[next]);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(variance_kernel, grid, block, 0, st, W, H, cur->d_t, cur->d_face, s->d_temporal[next],
-                       s->d_util[next], s->d_var);
+    hipLaunchKernelGGL(grid.x <= (unsigned)kSkipExpsTiles ? variance_kernel<true> : variance_kernel<false>, grid, block,
+                       0, st, W, H, cur->d_t, cur->d_face, s->d_temporal[next], s->d_util[next], s->d_var);
     HIP_TRY(hipGetLastError());
     const float scale = 1.0f + (2.4f - 1.0f) * s->prm.resolution_scale;   // mix(1, 2.4, u_ResolutionScale)
     const vpt_svgf_texel* src = s->d_var;
