@@ -238,7 +238,11 @@ struct vpt_server {
     {
         for (size_t i = 0; i < returning.size();) {
             Req* q = returning[i];
-            while (!q->reads.empty() && hipEventQuery(q->reads.back()) != hipErrorNotReady) {
+            while (!q->reads.empty()) {
+                // another error says nothing of the copies: asked again
+                // later, except when the server shuts down
+                const hipError_t e = hipEventQuery(q->reads.back());
+                if (e == hipErrorNotReady || (e != hipSuccess && !stop)) break;
                 (void)hipEventDestroy(q->reads.back());
                 q->reads.pop_back();
             }
@@ -862,6 +866,7 @@ extern "C" VPT_API int vpt_server_fetch(vpt_server* s, uint64_t ticket, const vp
         if (q->status)
             return set_error(q->status, "vpt_server_fetch: request %llu failed", (unsigned long long)ticket);
         q->fetching++;   // a release meanwhile leaves the request to us
+        q->reads.reserve(q->reads.size() + (size_t)q->fetching);
     }
     const vpt_request_result& r = q->res;
     const size_t n = q->units;
