@@ -39,7 +39,7 @@ VPT_HD TileXY strip_tile(uint32_t t, uint32_t tx, uint32_t ty)
     return TileXY{s * sw + r % width, r / width};
 }
 
-// The denoisers' order.  Bands, row by row from the top, where every tile has
+// The denoisers' order.  Bands, row by row from the bottom, where every tile has
 // a CU to itself (256 of them): no XCD's load is left to level there.  SVGF
 // frame of 200 x 91 (84 tiles of 32 x 8) in strips / bands 113 / 103 us, 482
 // x 110 (224) 121 / 96, 640 x 91 (240) 99 / 102; above, 900 x 91 (348) 104 /
