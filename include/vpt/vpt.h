@@ -598,8 +598,10 @@ VPT_API int vpt_server_submit(vpt_server* s, const vpt_request* req, uint64_t* t
 VPT_API int vpt_server_wait(vpt_server* s, uint64_t ticket, int timeout_ms, vpt_request_result* res);
 /* Copies a completed request's results into the non-null arrays of dst (in
  * device memory, of the sizes vpt_server_wait's result has them) by work on
- * `stream`, without waiting for it.  A release gives the memory back only
- * once that work has run.  VPT_ESTATE before the request has completed;
+ * `stream`, without waiting for it.  Arrays that lie in dst as vpt_server_wait's
+ * result has them (each 256-byte aligned behind the one before) go in one copy,
+ * with the bytes between them.  A release gives the memory back only once that
+ * work has run.  VPT_ESTATE before the request has completed;
  * VPT_EINVAL on a stream that is being captured. */
 VPT_API int vpt_server_fetch(vpt_server* s, uint64_t ticket, const vpt_request_result* dst, void* stream);
 /* Frees a completed request's result memory (the ticket becomes invalid).

@@ -322,6 +322,14 @@ def test_fetch_arguments(ctx, scene):
     dst.d_vis = vis.data_ptr()
     _lib.call("vpt_server_fetch", srv.handle, C.c_uint64(t), C.byref(dst), None)
     np.testing.assert_array_equal(vis.cpu().numpy(), r["ref_vis"])
+    # arrays apart from each other, at odd addresses, with guards behind them
+    one = torch.full((r["n"] * 13 + 64,), 9, dtype=torch.uint8, device="cuda")
+    dst.d_hits, dst.d_vis = one.data_ptr() + 1, one.data_ptr() + 1 + r["n"] * 12 + 4
+    _lib.call("vpt_server_fetch", srv.handle, C.c_uint64(t), C.byref(dst), None)
+    got = one.cpu().numpy()
+    np.testing.assert_array_equal(got[1:1 + r["n"] * 12], first["hits"].cpu().numpy())
+    np.testing.assert_array_equal(got[5 + r["n"] * 12:5 + r["n"] * 13], r["ref_vis"])
+    assert got[0] == 9 and (got[1 + r["n"] * 12:5 + r["n"] * 12] == 9).all() and (got[5 + r["n"] * 13:] == 9).all()
     srv.release(t)
     with pytest.raises(VptError) as e:
         srv.fetch(t)

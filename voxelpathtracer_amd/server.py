@@ -105,23 +105,22 @@ class Server:
                "t_done_ns": res.t_done_ns}
         n = res.n
         dst = RequestResult()
-
-        def new(name: str, dtype, count: int) -> int:
-            out[name] = torch.empty(count, dtype=dtype, device="cuda")
-            return out[name].data_ptr()
-
         if res.kind == _lib.VPT_REQ_FRAME:
-            gb = dst.gbuffer
-            gb.d_t = new("t", torch.float32, n)
-            gb.d_face = new("face", torch.uint8, n)
-            gb.d_block = new("block", torch.uint8, n)
-            gb.d_voxel = new("voxel", torch.int32, n)
-            dst.d_mask = new("mask", torch.uint8, n)
-            dst.d_rgb = new("rgb", torch.float32, 3 * n)
+            parts = (("t", torch.float32, 4), ("face", torch.uint8, 1), ("block", torch.uint8, 1),
+                     ("voxel", torch.int32, 4), ("mask", torch.uint8, 1), ("rgb", torch.float32, 12))
+        elif res.kind == _lib.VPT_REQ_GI:
+            parts = (("hits", torch.uint8, 12), ("vis", torch.uint8, 1))
         else:
-            dst.d_hits = new("hits", torch.uint8, 12 * n)
-            if res.kind == _lib.VPT_REQ_GI:
-                dst.d_vis = new("vis", torch.uint8, n)
+            parts = (("hits", torch.uint8, 12),)
+        # one block, laid out as the server's, so that one copy fills it
+        sizes = [(n * per + 255) // 256 * 256 for _, _, per in parts]
+        block = torch.empty(sum(sizes), dtype=torch.uint8, device="cuda")
+        at, base = 0, block.data_ptr()
+        for (name, dtype, per), size in zip(parts, sizes):
+            piece = block[at:at + n * per]
+            out[name] = piece if dtype is torch.uint8 else piece.view(dtype)
+            setattr(dst.gbuffer if name in ("t", "face", "block", "voxel") else dst, "d_" + name, base + at)
+            at += size
         call("vpt_server_fetch", self.handle, C.c_uint64(ticket), C.byref(dst),
              C.c_void_p(torch.cuda.current_stream().cuda_stream))
         return out
